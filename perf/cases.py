@@ -55,6 +55,14 @@ def listed():
 
 
 def draw(rng):
+    known = [{k: v for k, v in c.items() if k != "name"} for c in listed()]
+    while True:
+        c = _draw(rng)
+        if c not in known:
+            return c
+
+
+def _draw(rng):
     kind = rng.choice(["poisson", "poisson", "poisson", "poisson", "fields", "fields", "hydro", "convection",
                        "viscous", "sequence", "train"])
     domain, mesh = rng.choice([("PPN", "UUD"), ("PPN", "UUD"), ("NNN", "DDD"), ("NPN", "DUD"), ("PNN", "UDD")])
@@ -80,7 +88,7 @@ def draw(rng):
     if kind == "viscous":
         c["loc"] = rng.randint(0, 3)
     if kind in ("sequence", "train"):
-        c["domain"], c["mesh"] = "PPN", "UUD"
+        del c["domain"], c["mesh"]   # periodic in x and y, walls and stretching in z
     return c
 
 
