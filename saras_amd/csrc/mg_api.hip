@@ -297,6 +297,7 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
         for (int q = 0; q < 2; q++) launch_fill<float>(m->zdir[q], sz, 0.0f, m->stream);
     }
     if (d->coarseDirect) RETCHK(build_coarse_direct(m));
+    if (rb_pass_attr()) return set_err(SR_ERR_HIP, "LDS size of the sweep kernels refused");
     // coarse end of the cycle in LDS
     {
         int dev = 0, lds_max = 65536;
@@ -475,6 +476,23 @@ void sr::mark(sr_mg *m, hipEvent_t e) {
         m->marks_off = true;
     }
 }
+// Whether a smoothing of `count` red-black sweeps runs as one-launch sweeps (launch_rb_pass) that need
+// no ghosts beforehand.  They hand colour 1 back and forth between u and a second buffer and have to
+// end in u: any count from zero, even counts otherwise.
+static bool passes_ok(const Lay &L, const Bc &bc, int count, bool zero_start) {
+    return count > 0 && (zero_start || count % 2 == 0) && rb_pass_ok(L, bc);
+}
+
+template <typename T>
+static void smooth_passes(const Lay &L, T *u, T *t, const T *f, T *const *c, const Bc &bc, int count, bool zero_start,
+                          hipStream_t s) {
+    for (int n = 0; n < count; n++) {
+        // sweep n writes to u when an even number of sweeps follows, and reads the other buffer
+        T *bo = (count - 1 - n) % 2 == 0 ? u : t;
+        launch_rb_pass<T>(L, bo == u ? t : u, u, bo, f, c[0], c[1], c[2], bc, zero_start && n == 0, n + 1 == count, s);
+    }
+}
+
 // smooth(): ghosts, then `count` red-black sweeps (each updated node refreshes its face ghosts);
 // exact = 1 adds the closing imposeBC of poisson_d3.cc:181 (edge and corner ghosts included).
 void sr::smooth_level(sr_mg *m, int l, int count, int zeroBC, bool zero_start, bool exact, hipEvent_t ea,
@@ -482,7 +500,12 @@ void sr::smooth_level(sr_mg *m, int l, int count, int zeroBC, bool zero_start, b
     Level &V = m->lv[l];
     Bc bc = pressure_bc(m, l, zeroBC);
     hipStream_t s = m->stream;
-    if (m->d.gsSmooth) {
+    if (m->d.gsSmooth && !exact && !first_done && passes_ok(V.L, bc, count, zero_start)) {
+        // colour 1 of tmp is free: the residual after pre-smoothing is formed on colour 0
+        if (ea) mark(m, ea);
+        smooth_passes<double>(V.L, V.u, V.t, V.f, V.c64, bc, count, zero_start, s);
+        if (eb) mark(m, eb);
+    } else if (m->d.gsSmooth) {
         // the red-black sweeps read face ghosts only: a level whose face-ghost images are current
         // (faces_ready) needs no fill
         if (!zero_start && !faces_ready) launch_fill_ghosts<double>(V.L, V.u, bc, s);
@@ -555,8 +578,9 @@ void sr::vcycle_fp64(sr_mg *m) {
         residual_level(m, l, red0 ? 0 : -1, l > 0);
         // a level smoothed from zero by Gauss-Seidel starts with a colour-0 half sweep that reads no
         // u: the restriction that makes its right-hand side does it (ZeroStart)
-        const bool fuse = d.gsSmooth && d.preSmooth > 0 && l + 1 != Lc && l + 1 != D;
         Level &Nx = m->lv[l + 1];
+        const bool fuse = d.gsSmooth && d.preSmooth > 0 && l + 1 != Lc && l + 1 != D &&
+                          !passes_ok(Nx.L, pressure_bc(m, l + 1, 1), d.preSmooth, true);
         const ZeroStart<double> zs{Nx.u, Nx.c64[0], Nx.c64[1], Nx.c64[2], pressure_bc(m, l + 1, 1)};
         launch_restrict<double>(m->lv[l].L, Nx.L, m->lv[l].t, Nx.f, m->stream, red0, fuse ? &zs : nullptr);
         if (l + 1 == Lc) {
@@ -579,8 +603,8 @@ void sr::vcycle_fp64(sr_mg *m) {
     // rule there is an image rule), so the post-smoothing starts without a ghost fill; level 0 keeps
     // the separate fill (measured faster there)
     for (int l = bottom - 1; l >= 0; l--) {
-        const bool img = l > 0 && d.gsSmooth;
         const Bc bc = pressure_bc(m, l, 1);
+        const bool img = l > 0 && d.gsSmooth && !passes_ok(m->lv[l].L, bc, d.postSmooth, false);
         launch_prolong<double, double>(m->lv[l].L, m->lv[l + 1].L, m->lv[l + 1].u, m->lv[l].u, 1, m->stream, pcol,
                                        img ? &bc : nullptr);
         smooth_level(m, l, d.postSmooth, l == 0 ? 0 : 1, false, false, nullptr, nullptr, img);
@@ -604,6 +628,12 @@ static void smooth32(sr_mg *m, int l, int count, int zeroBC, bool zero_start, hi
     bool wall = bc.rule[0] == G_WALL || bc.rule[1] == G_WALL || bc.rule[2] == G_WALL;
     bool zs = zero_start && !wall;
     hipStream_t s = m->stream;
+    if (!first_done && passes_ok(V.L, bc, count, zs)) {
+        if (ea) mark(m, ea);
+        smooth_passes<float>(V.L, V.u32, V.t32, V.f32, V.c32, bc, count, zs, s);
+        if (eb) mark(m, eb);
+        return;
+    }
     if (!zs && !(faces_ready && !zero_start)) {
         if (zero_start) launch_fill<float>(V.u32, lay_size(V.L), 0.0f, s);
         launch_fill_ghosts<float>(V.L, V.u32, bc, s);
@@ -641,7 +671,8 @@ void sr::vcycle_fp32(sr_mg *m) {
         Level &Nx = m->lv[l + 1];
         const Bc nb = error_bc(m, l + 1, 1);
         const bool nwall = nb.rule[0] == G_WALL || nb.rule[1] == G_WALL || nb.rule[2] == G_WALL;
-        const bool fuse = m->pre32 > 0 && !nwall && l + 1 != Lc && l + 1 != D;
+        const bool fuse = m->pre32 > 0 && !nwall && l + 1 != Lc && l + 1 != D &&
+                          !passes_ok(Nx.L, nb, m->pre32, true);
         const ZeroStart<float> zs{Nx.u32, Nx.c32[0], Nx.c32[1], Nx.c32[2], nb};
         launch_restrict<float>(V.L, Nx.L, V.t32, Nx.f32, s, red0, fuse ? &zs : nullptr);
         if (l + 1 == Lc) {
@@ -667,9 +698,10 @@ void sr::vcycle_fp32(sr_mg *m) {
     // post-smoothing starts without a ghost fill (as in the FP64 cycle)
     for (int l = bottom - 1; l >= 0; l--) {
         const Bc bc = error_bc(m, l, 1);
+        const bool img = l > 0 && !passes_ok(m->lv[l].L, bc, m->post32, false);
         launch_prolong<float, float>(m->lv[l].L, m->lv[l + 1].L, m->lv[l + 1].u32, m->lv[l].u32, 1, s, pcol,
-                                     l > 0 ? &bc : nullptr);
-        smooth32(m, l, m->post32, l == 0 ? 0 : 1, false, nullptr, nullptr, l > 0);
+                                     img ? &bc : nullptr);
+        smooth32(m, l, m->post32, l == 0 ? 0 : 1, false, nullptr, nullptr, img);
     }
 }
 

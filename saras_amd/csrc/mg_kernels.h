@@ -12,6 +12,15 @@ template <typename T> void launch_fill_ghosts(const Lay &L, T *a, const Bc &bc, 
 template <typename T>
 void launch_rb_sweep(const Lay &L, T *u, const T *f, const T *cx, const T *cy, const T *cz, int color,
                      const Bc &bc, bool zero_start, hipStream_t s);
+// One full red-black sweep (colour 0, then colour 1) in a single launch (mg_pass.hip): colour 1 is
+// read from ub and written to bo (another buffer, see there), colour 0 and the face-ghost images are
+// stored, in u and bo, by the last sweep of a smoothing only.  zero: u is known to be zero (ub unused).
+// rb_pass_ok: the levels and ghost rules it takes.
+bool rb_pass_ok(const Lay &L, const Bc &bc);
+int rb_pass_attr();   // once per device, before the first launch
+template <typename T>
+void launch_rb_pass(const Lay &L, const T *ub, T *u, T *bo, const T *f, const T *cx, const T *cy, const T *cz,
+                    const Bc &bc, bool zero, bool last, hipStream_t s);
 template <typename T, typename TO>
 // img: each computed node also writes its face and edge ghost images by *img (image rules only;
 // corner ghosts are not written)

@@ -16,6 +16,7 @@
 // and the Gauss-Seidel update u = (sum_d lp_d u(+1) + lm_d u(-1) - f) / sum_d lc_d, which equals the
 // reference quotient of poisson_d3.cc:140-147 after dividing numerator and denominator by 2 hx^2hy^2hz^2.
 #include "mg_kernels.h"
+#include "mg_device.h"
 #include "mg_state.h"
 #include "xcd.h"
 
@@ -31,13 +32,6 @@ struct Geo {
     unsigned d1;
     float inv1;
 };
-
-__device__ inline unsigned fdivu(unsigned r, unsigned d, float inv) {
-    unsigned q = (unsigned)((float)r * inv);
-    int rem = (int)r - (int)(q * d);
-    q += (unsigned)(rem >= (int)d) - (unsigned)(rem < 0);
-    return q;
-}
 
 // Grid-stride order for reductions over a whole level: the blocks of XCD x (blockIdx % 8) walk the
 // x-th contiguous eighth of the logical blocks, so the neighbour planes a block reads stay in that
