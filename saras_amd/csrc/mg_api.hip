@@ -97,7 +97,7 @@ static void plan_coarse(sr_mg *m, int &first, CoarseDesc &D, size_t &lds, size_t
         t.last = depth;
         if (depth - f + 1 > 8) continue;
         for (int q = 0; q <= depth - f; q++) t.L[q] = m->lv[f + q].L;
-        size_t bytes = coarse_cycle_plan<T>(t, limit);
+        size_t bytes = coarse_cycle_plan<T>(t);
         if (bytes <= limit) {
             first = f;
             D = t;
@@ -191,10 +191,20 @@ static int build_coarse_direct(sr_mg *m) {
     return SR_OK;
 }
 
-static void finish_coarse(sr_mg *m, CoarseDesc &D, bool fp32) {
+template <typename T>
+static int upload_coarse_coef(sr_mg *m, CoarseDesc &D, T *&dev) {
+    std::vector<T> c((size_t)D.ncoef, T(0));
     for (int q = 0; q <= D.last - D.first; q++)
-        for (int a = 0; a < 3; a++)
-            D.cg[q][a] = fp32 ? (const void *)m->lv[D.first + q].c32[a] : (const void *)m->lv[D.first + q].c64[a];
+        for (int a = 0; a < 3; a++) {
+            const std::vector<double> &h = m->lv[D.first + q].coef_h[a];
+            std::copy(h.begin(), h.end(), c.begin() + (D.off_c[q][a] - D.off_c[0][0]));
+        }
+    RETCHK(upload_vec(&dev, c));
+    D.coef = dev;
+    return SR_OK;
+}
+
+static void finish_coarse(sr_mg *m, CoarseDesc &D, bool fp32) {
     D.pre = fp32 ? m->pre32 : m->d.preSmooth;
     D.post = fp32 ? m->post32 : m->d.postSmooth;
     D.bc = pressure_bc(m, D.first, 1);
@@ -309,11 +319,13 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
             plan_coarse<double>(m, m->coarse_first64, m->cdesc64, m->clds64, limit);
             if (m->coarse_first64 <= depth) {
                 finish_coarse(m, m->cdesc64, false);
+                RETCHK(upload_coarse_coef<double>(m, m->cdesc64, m->ccoef64));
                 if (coarse_cycle_attr<double>(m->clds64)) m->coarse_first64 = 1 << 20;
             }
             plan_coarse<float>(m, m->coarse_first32, m->cdesc32, m->clds32, limit);
             if (m->coarse_first32 <= depth) {
                 finish_coarse(m, m->cdesc32, true);
+                RETCHK(upload_coarse_coef<float>(m, m->cdesc32, m->ccoef32));
                 if (coarse_cycle_attr<float>(m->clds32)) m->coarse_first32 = 1 << 20;
             }
         }
@@ -395,6 +407,7 @@ extern "C" int sr_mg_destroy(sr_mg *m) {
         (void)hipFree(m->zdir[q]);
     }
     (void)hipFree(m->pinv64); (void)hipFree(m->pinv32);
+    (void)hipFree(m->ccoef64); (void)hipFree(m->ccoef32);
     (void)hipFree(m->gpart); (void)hipFree(m->gcoef);
     for (Level &V : m->lv) {
         (void)hipFree(V.u); (void)hipFree(V.f); (void)hipFree(V.t);

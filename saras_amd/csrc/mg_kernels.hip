@@ -44,23 +44,6 @@ __device__ inline void xcd_range(unsigned total, unsigned &first, unsigned &stri
     end = min(total, (x + 1u) * chunk);
 }
 
-// t = (a * n1 + b) * n2 + c for t < 2^24, split with float-reciprocal divisions (fdivu) instead of
-// integer divisions: the single-workgroup kernels are bound by their VALU issue rate
-struct Div3 {
-    unsigned n1, n2;
-    float i1, i2;
-};
-__device__ inline Div3 div3(int n1, int n2) {
-    return Div3{(unsigned)n1, (unsigned)n2, 1.0f / (float)n1, 1.0f / (float)n2};
-}
-__device__ inline void split3(const Div3 &D, int t, int &a, int &b, int &c) {
-    unsigned r = fdivu((unsigned)t, D.n2, D.i2);
-    c = t - (int)(r * D.n2);
-    unsigned q = fdivu(r, D.n1, D.i1);
-    b = (int)(r - q * D.n1);
-    a = (int)q;
-}
-
 __device__ inline bool geo_slot(const Geo &g, unsigned b, unsigned &ip, unsigned &r) {
     unsigned p = b / g.bpp;
     r = (b - p * g.bpp) * 256u + threadIdx.x;
@@ -153,42 +136,6 @@ __global__ void __launch_bounds__(256) k_fill_ghosts(Lay L, T *__restrict__ a, B
 // ------------------------------------------------------------------------------------------------
 // red-black Gauss-Seidel half sweep
 // ------------------------------------------------------------------------------------------------
-// Face-ghost images of an updated node: a node whose padded index is the source of a ghost of a
-// periodic / mirror / anti direction writes that ghost (same colour, so no other thread of this
-// half sweep reads it).  Edge and corner ghosts are not read by the 7-point stencil.
-// Diagonal of the 7-point operator at a node from the three directions' coefficient quadruples
-// (c+, c-, c0, pad).  The FP64 quadruples store c0 = c+ + c- (rounded once, at set-up), so the sum
-// is formed from c+ and c-, which the stencil loads anyway, with the same value as from c0; the FP32
-// quadruples hold each value rounded separately and use c0.
-template <typename T>
-__device__ __forceinline__ T diag3(const T *X, const T *Y, const T *Z) {
-    if constexpr (sizeof(T) == 8) return (X[0] + X[1]) + (Y[0] + Y[1]) + (Z[0] + Z[1]);
-    else return X[2] + Y[2] + Z[2];
-}
-
-template <typename T>
-__device__ inline void write_images(const Lay &L, T *u, int ip, int jp, int kp, T v, const Bc &bc) {
-    int n[3] = {L.nx, L.ny, L.nz};
-    int p[3] = {ip, jp, kp};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        int r = bc.rule[d];
-        if (r > G_ANTI) continue;
-        T w = (r == G_ANTI) ? -v : v;
-        int g0 = ghost_src(r, 0, n[d]), g1 = ghost_src(r, n[d] + 1, n[d]);
-        if (p[d] == g0) {
-            int q[3] = {p[0], p[1], p[2]};
-            q[d] = 0;
-            u[lay_idx(L, q[0], q[1], q[2])] = w;
-        }
-        if (p[d] == g1) {
-            int q[3] = {p[0], p[1], p[2]};
-            q[d] = n[d] + 1;
-            u[lay_idx(L, q[0], q[1], q[2])] = w;
-        }
-    }
-}
-
 // Face and edge ghost images of node (ip, jp, kp) with value v, image rules only: along each
 // direction the ghosts whose source is this node, then every pair of directions (the composed image
 // of the x-then-y-then-z fill when every rule is an image rule).  Corner ghosts are not written: the
@@ -1106,479 +1053,6 @@ __global__ void __launch_bounds__(256) k_gcr_step(Lay L, Geo G, const double *__
     });
 }
 
-// ------------------------------------------------------------------------------------------------
-// the coarse end of the V-cycle in one workgroup: levels first..last of the down leg, the coarsest
-// solve and the up leg back to `first`, with every level's u and f held in LDS
-// (poisson.cc:239-279 restricted to those levels; poisson_d3.cc smooth/coarsen/solve/prolong)
-// ------------------------------------------------------------------------------------------------
-template <typename T>
-__device__ inline void blk_sweep(const Lay &L, T *u, const T *f, const T *cx, const T *cy, const T *cz, int color,
-                                 const Bc &bc, bool zero_start) {
-    int n = L.nx * L.ny * L.kh;
-    const Div3 dv = div3(L.ny, L.kh);
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        int ip, jp, h;
-        split3(dv, t, ip, jp, h);
-        ip += 1;
-        jp += 1;
-        int kb = (color + 1 + ip + jp) & 1;
-        int kp = 2 * h + kb;
-        if (kp < 1 || kp > L.nz) continue;
-        long rc = lay_row(L, ip, jp, color);
-        const T *X = cx + 4 * ip, *Y = cy + 4 * jp, *Z = cz + 4 * kp;
-        T num;
-        if (zero_start) {
-            num = -f[rc + h];
-        } else {
-            long ro = lay_row(L, ip, jp, color ^ 1);
-            long sx = 2L * (L.ny + 2) * L.khs, sy = 2L * L.khs;
-            num = X[0] * u[ro + sx + h] + X[1] * u[ro - sx + h] + Y[0] * u[ro + sy + h] + Y[1] * u[ro - sy + h] +
-                  Z[0] * u[ro + h + kb] + Z[1] * u[ro + h - 1 + kb] - f[rc + h];
-        }
-        T v = num / diag3<T>(X, Y, Z);
-        u[rc + h] = v;
-        write_images(L, u, ip, jp, kp, v, bc);
-    }
-    __syncthreads();
-}
-
-template <typename T>
-__device__ inline void blk_zero(const Lay &L, T *u) {
-    long n = lay_size(L);
-    for (long t = threadIdx.x; t < n; t += blockDim.x) u[t] = T(0);
-    __syncthreads();
-}
-
-// Residual of level L at padded node (ip, jp, kp) as the restriction reads it (residual-pad rules
-// tb).  The position is resolved without branches: a ghost position is mapped to the core node
-// whose residual it carries (periodic / mirror / antisymmetric image, factor +-1) or given factor 0
-// (zero pads), and the core residual f - L u (the expression of apply_lap) is evaluated there, so
-// the 27 evaluations of a restriction can overlap their loads.
-template <typename T>
-__device__ inline T blk_res_src(const Lay &L, const T *u, const T *f, const T *cx, const T *cy, const T *cz,
-                                const Bc &tb, int ip, int jp, int kp) {
-    const int n[3] = {L.nx, L.ny, L.nz};
-    int q[3] = {ip, jp, kp};
-    int fac = 1;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const int g = q[d], r = tb.rule[d];
-        const bool ghost = g == 0 || g == n[d] + 1;
-        const bool image = r <= G_ANTI;
-        fac = !ghost ? fac : !image ? 0 : r == G_ANTI ? -fac : fac;
-        q[d] = !ghost ? g : image ? ghost_src(r, g, n[d]) : 1;
-    }
-    const int sy = 2 * L.khs, sx = (L.ny + 2) * sy;
-    const int c = lay_color(q[0], q[1], q[2]);
-    const int base = (q[0] * (L.ny + 2) + q[1]) * sy;
-    const int rc = base + c * L.khs, ro = base + (c ^ 1) * L.khs;
-    const int h = q[2] >> 1, kb = q[2] & 1;
-    const T *X = cx + 4 * q[0], *Y = cy + 4 * q[1], *Z = cz + 4 * q[2];
-    T lu = X[0] * u[ro + sx + h] + X[1] * u[ro - sx + h] + Y[0] * u[ro + sy + h] + Y[1] * u[ro - sy + h] +
-           Z[0] * u[ro + h + kb] + Z[1] * u[ro + h - 1 + kb] - diag3<T>(X, Y, Z) * u[rc + h];
-    T res = f[rc + h] - lu;
-    return fac == 0 ? T(0) : fac < 0 ? -res : res;
-}
-
-// 27-point full weighting (poisson_d3.cc:250-298) of the residuals R(a, b, e) at the fine offsets
-// a, b, e in {-1, 0, 1} around a coarse node's fine position: faces 1/16, edges 1/32, vertices
-// 1/64, centre 1/8, summed in this order
-template <typename T, typename F>
-__device__ inline T full_weight27(F &&R) {
-    T facePoints = (R(1, 0, 0) + R(-1, 0, 0) + R(0, 1, 0) + R(0, -1, 0) + R(0, 0, 1) + R(0, 0, -1)) * T(0.0625);
-    T edgePoints = (R(1, 1, 0) + R(1, -1, 0) + R(-1, -1, 0) + R(-1, 1, 0) + R(0, 1, 1) + R(0, -1, 1) + R(0, -1, -1) +
-                    R(0, 1, -1) + R(1, 0, 1) + R(1, 0, -1) + R(-1, 0, -1) + R(-1, 0, 1)) *
-                   T(0.03125);
-    T vertPoints = (R(1, 1, 1) + R(1, 1, -1) + R(1, -1, 1) + R(-1, 1, 1) + R(1, -1, -1) + R(-1, 1, -1) + R(-1, -1, 1) +
-                    R(-1, -1, -1)) *
-                   T(0.015625);
-    return facePoints + edgePoints + vertPoints + R(0, 0, 0) * T(0.125);
-}
-
-// one thread per coarse node, its 27 fine residuals evaluated in turn
-template <typename T>
-__device__ inline void blk_restrict(const Lay &F, const T *uf, const T *ff, const T *cx, const T *cy, const T *cz,
-                                    const Bc &tb, const Lay &Cl, T *fc) {
-    int n = Cl.nx * Cl.ny * Cl.nz;
-    const Div3 dv = div3(Cl.ny, Cl.nz);
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        int fi = 2 * i + 1, fj = 2 * j + 1, fk = 2 * k + 1;
-        fc[lay_idx(Cl, i + 1, j + 1, k + 1)] = full_weight27<T>([&](int a, int b, int e) {
-            return blk_res_src<T>(F, uf, ff, cx, cy, cz, tb, fi + a, fj + b, fk + e);
-        });
-    }
-    __syncthreads();
-}
-
-// The same restriction with one thread per (coarse node, tap): rounds of kTapNodes coarse nodes,
-// whose 27 x kTapNodes fine residuals are evaluated at once into scr, then weighted by one thread
-// per node with the same arithmetic as blk_restrict.  For the smallest levels, where one thread
-// per coarse node leaves most of the workgroup idle behind 27 dependent residual evaluations.
-constexpr int kTapNodes = 37;
-constexpr int kTapScratch = 27 * kTapNodes;
-
-template <typename T>
-__device__ inline void blk_restrict_taps(const Lay &F, const T *uf, const T *ff, const T *cx, const T *cy,
-                                         const T *cz, const Bc &tb, const Lay &Cl, T *fc, T *scr) {
-    const int n = Cl.nx * Cl.ny * Cl.nz;
-    const Div3 dv = div3(Cl.ny, Cl.nz);
-    const int t = threadIdx.x;
-    for (int first = 0; first < n; first += kTapNodes) {
-        if (t < kTapScratch) {
-            int node = first + t / 27, tap = t % 27;
-            if (node < n) {
-                int i, j, k;
-                split3(dv, node, i, j, k);
-                scr[t] = blk_res_src<T>(F, uf, ff, cx, cy, cz, tb, 2 * i + tap / 9, 2 * j + (tap / 3) % 3,
-                                       2 * k + tap % 3);
-            }
-        }
-        __syncthreads();
-        if (t < kTapNodes && first + t < n) {
-            const T *R = scr + 27 * t;
-            int i, j, k;
-            split3(dv, first + t, i, j, k);
-            fc[lay_idx(Cl, i + 1, j + 1, k + 1)] =
-                full_weight27<T>([&](int a, int b, int e) { return R[(a + 1) * 9 + (b + 1) * 3 + (e + 1)]; });
-        }
-        __syncthreads();
-    }
-}
-
-// The red-black forms of the two restrictions above: after a red-black sweep that ended on colour 1
-// the colour-1 residual is zero, and of the 27 points only the coincident node and the 12 edge
-// points are colour 0 (k_restrict<T, true>): 13 residual evaluations per coarse node, weighted in
-// k_restrict<T, true>'s order.  kRbTaps lists the 12 edge offsets in that order, then the centre.
-__constant__ signed char kRbTaps[13][3] = {{1, 1, 0},  {1, -1, 0}, {-1, -1, 0}, {-1, 1, 0}, {0, 1, 1},
-                                           {0, -1, 1}, {0, -1, -1}, {0, 1, -1}, {1, 0, 1},  {1, 0, -1},
-                                           {-1, 0, -1}, {-1, 0, 1}, {0, 0, 0}};
-constexpr int kRbTapNodes = kTapScratch / 13;
-
-template <typename T, typename R>
-__device__ inline T rb_weight13(R &&res) {
-    T edgePoints = (res(0) + res(1) + res(2) + res(3) + res(4) + res(5) + res(6) + res(7) + res(8) + res(9) +
-                    res(10) + res(11)) *
-                   T(0.03125);
-    return edgePoints + res(12) * T(0.125);
-}
-
-template <typename T>
-__device__ inline void blk_restrict_rb(const Lay &F, const T *uf, const T *ff, const T *cx, const T *cy, const T *cz,
-                                       const Bc &tb, const Lay &Cl, T *fc) {
-    int n = Cl.nx * Cl.ny * Cl.nz;
-    const Div3 dv = div3(Cl.ny, Cl.nz);
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        int fi = 2 * i + 1, fj = 2 * j + 1, fk = 2 * k + 1;
-        fc[lay_idx(Cl, i + 1, j + 1, k + 1)] = rb_weight13<T>([&](int q) {
-            return blk_res_src<T>(F, uf, ff, cx, cy, cz, tb, fi + kRbTaps[q][0], fj + kRbTaps[q][1],
-                                  fk + kRbTaps[q][2]);
-        });
-    }
-    __syncthreads();
-}
-
-template <typename T>
-__device__ inline void blk_restrict_rb_taps(const Lay &F, const T *uf, const T *ff, const T *cx, const T *cy,
-                                            const T *cz, const Bc &tb, const Lay &Cl, T *fc, T *scr) {
-    const int n = Cl.nx * Cl.ny * Cl.nz;
-    const Div3 dv = div3(Cl.ny, Cl.nz);
-    const int t = threadIdx.x;
-    for (int first = 0; first < n; first += kRbTapNodes) {
-        if (t < 13 * kRbTapNodes) {
-            int node = first + t / 13, tap = t % 13;
-            if (node < n) {
-                int i, j, k;
-                split3(dv, node, i, j, k);
-                scr[t] = blk_res_src<T>(F, uf, ff, cx, cy, cz, tb, 2 * i + 1 + kRbTaps[tap][0],
-                                        2 * j + 1 + kRbTaps[tap][1], 2 * k + 1 + kRbTaps[tap][2]);
-            }
-        }
-        __syncthreads();
-        if (t < kRbTapNodes && first + t < n) {
-            const T *R = scr + 13 * t;
-            int i, j, k;
-            split3(dv, first + t, i, j, k);
-            fc[lay_idx(Cl, i + 1, j + 1, k + 1)] = rb_weight13<T>([&](int q) { return R[q]; });
-        }
-        __syncthreads();
-    }
-}
-
-// uf += P e on the core nodes of the fine level (trilinear, poisson_d3.cc:301-388).  The items
-// t, t + blockDim, t + 2 blockDim of a thread update distinct nodes, so their loads are all issued
-// before the first update is stored.  With `images` every updated node also rewrites its face-ghost
-// images (all smoothing ghost rules are images), which replaces a ghost fill of the whole level.
-constexpr int kBlkBatch = 3;
-
-template <typename T>
-__device__ inline void blk_prolong_add(const Lay &F, T *uf, const Lay &Cl, const T *e, const Bc &bc, bool images,
-                                       int color = -1) {
-    // color 1: the colour-1 nodes only (slots (i, j, h), kp = 2h + parity), the post-smoothing's first
-    // colour-0 half sweep overwrites the colour-0 nodes without reading them
-    const int kc = color == 1 ? (F.nz + 2) / 2 : F.nz;
-    const int n = F.nx * F.ny * kc;
-    const Div3 dv = div3(F.ny, kc);
-    for (int t0 = threadIdx.x; t0 < n; t0 += kBlkBatch * blockDim.x) {
-        T val[kBlkBatch];
-        int pi[kBlkBatch], pj[kBlkBatch], pk[kBlkBatch];
-        bool ok[kBlkBatch];
-#pragma unroll
-        for (int b = 0; b < kBlkBatch; b++) {
-            const int t = t0 + b * (int)blockDim.x;
-            ok[b] = false;
-            if (t >= n) continue;
-            int i, j, k;
-            split3(dv, t, i, j, k);
-            if (color == 1) {
-                const int kp = 2 * k + ((i + j) & 1);
-                if (kp < 1 || kp > F.nz) continue;
-                k = kp - 1;
-            }
-            ok[b] = true;
-            int io = i & 1, jo = j & 1, ko = k & 1;
-            int ci = i / 2 + 1, cj = j / 2 + 1, ck = k / 2 + 1;
-#define EE(a, b2, q) e[lay_idx(Cl, ci + (a), cj + (b2), ck + (q))]
-            T v;
-            if (io && jo && ko)
-                v = (EE(0, 0, 0) + EE(1, 0, 0) + EE(0, 1, 0) + EE(0, 0, 1) + EE(1, 1, 0) + EE(1, 0, 1) + EE(0, 1, 1) +
-                     EE(1, 1, 1)) / T(8.0);
-            else if (io && jo)
-                v = (EE(0, 0, 0) + EE(0, 1, 0) + EE(1, 0, 0) + EE(1, 1, 0)) / T(4.0);
-            else if (io && ko)
-                v = (EE(0, 0, 0) + EE(0, 0, 1) + EE(1, 0, 0) + EE(1, 0, 1)) / T(4.0);
-            else if (io)
-                v = (EE(0, 0, 0) + EE(1, 0, 0)) / T(2.0);
-            else if (jo && ko)
-                v = (EE(0, 0, 0) + EE(0, 0, 1) + EE(0, 1, 0) + EE(0, 1, 1)) / T(4.0);
-            else if (jo)
-                v = (EE(0, 0, 0) + EE(0, 1, 0)) / T(2.0);
-            else if (ko)
-                v = (EE(0, 0, 0) + EE(0, 0, 1)) / T(2.0);
-            else
-                v = EE(0, 0, 0);
-#undef EE
-            pi[b] = i + 1;
-            pj[b] = j + 1;
-            pk[b] = k + 1;
-            val[b] = uf[lay_idx(F, i + 1, j + 1, k + 1)] + v;
-        }
-#pragma unroll
-        for (int b = 0; b < kBlkBatch; b++) {
-            if (!ok[b]) continue;
-            uf[lay_idx(F, pi[b], pj[b], pk[b])] = val[b];
-            if (images) write_images(F, uf, pi[b], pj[b], pk[b], val[b], bc);
-        }
-    }
-    __syncthreads();
-}
-
-template <typename T>
-__device__ inline double blk_max_res(const Lay &L, const T *u, const T *f, const T *cx, const T *cy, const T *cz,
-                                     double *red) {
-    double m = -1.0e-10;
-    int nc = L.nx * L.ny * L.nz;
-    const Div3 dv = div3(L.ny, L.nz);
-    for (int t = threadIdx.x; t < nc; t += blockDim.x) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        int ip = i + 1, jp = j + 1, kp = k + 1;
-        int c = lay_color(ip, jp, kp);
-        long rc = lay_row(L, ip, jp, c), ro = lay_row(L, ip, jp, c ^ 1);
-        double lu = (double)apply_lap<T, T>(L, u, rc, ro, kp >> 1, kp & 1, cx + 4 * ip, cy + 4 * jp, cz + 4 * kp);
-        m = fmax(m, fabs((double)f[rc + (kp >> 1)] - lu));
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    double gm = red[0];
-    for (int w = 1; w < (int)(blockDim.x + 63) / 64; ++w) gm = fmax(gm, red[w]);
-    __syncthreads();
-    return gm;
-}
-
-template <typename T>
-__device__ inline void blk_project(const Lay &L, T *f, const double *wx, const double *wy, const double *wz,
-                                   double wsum, double *red) {
-    int n = L.nx * L.ny * L.nz;
-    double s = 0;
-    const Div3 dv = div3(L.ny, L.nz);
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        s += wx[i] * wy[j] * wz[k] * (double)f[lay_idx(L, i + 1, j + 1, k + 1)];
-    }
-    s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    double tot = 0;
-    for (int w = 0; w < (int)(blockDim.x + 63) / 64; ++w) tot += red[w];
-    __syncthreads();
-    double c = tot / wsum;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        long o = lay_idx(L, i + 1, j + 1, k + 1);
-        f[o] = (T)((double)f[o] - c);
-    }
-    __syncthreads();
-}
-
-// The coarsest-level iteration of the coarse cycle in one wavefront: the coarsest level has a few
-// dozen nodes, so one wave updates them with wave-level synchronisation instead of workgroup
-// barriers.  Same red-black order, same ghost composition, same stop rule as the whole-block path.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-template <typename T>
-__device__ inline void wv_fill_ghosts(const Lay &L, T *a, const Bc &bc, int lane) {
-    int NX = L.nx + 2, NY = L.ny + 2, NZ = L.nz + 2;
-    int n = NX * NY * NZ;
-    const Div3 dv = div3(NY, NZ);
-    for (int t = lane; t < n; t += 64) {
-        int ip, jp, kp;
-        split3(dv, t, ip, jp, kp);
-        bool ghost = ip == 0 || ip == NX - 1 || jp == 0 || jp == NY - 1 || kp == 0 || kp == NZ - 1;
-        T v;
-        if (ghost && ghost_resolve(L, a, ip, jp, kp, bc, v)) a[lay_idx(L, ip, jp, kp)] = v;
-    }
-    wave_sync();
-}
-
-template <typename T>
-__device__ inline void wv_sweep(const Lay &L, T *u, const T *f, const T *cx, const T *cy, const T *cz, int color,
-                                int lane) {
-    int n = L.nx * L.ny * L.nz;
-    const Div3 dv = div3(L.ny, L.nz);
-    for (int t = lane; t < n; t += 64) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        if (((i + j + k) & 1) != color) continue;
-        int ip = i + 1, jp = j + 1, kp = k + 1;
-        const T *X = cx + 4 * ip, *Y = cy + 4 * jp, *Z = cz + 4 * kp;
-        T num = X[0] * u[lay_idx(L, ip + 1, jp, kp)] + X[1] * u[lay_idx(L, ip - 1, jp, kp)] +
-                Y[0] * u[lay_idx(L, ip, jp + 1, kp)] + Y[1] * u[lay_idx(L, ip, jp - 1, kp)] +
-                Z[0] * u[lay_idx(L, ip, jp, kp + 1)] + Z[1] * u[lay_idx(L, ip, jp, kp - 1)] - f[lay_idx(L, ip, jp, kp)];
-        u[lay_idx(L, ip, jp, kp)] = num / diag3<T>(X, Y, Z);
-    }
-    wave_sync();
-}
-
-template <typename T>
-__device__ inline double wv_max_res(const Lay &L, const T *u, const T *f, const T *cx, const T *cy, const T *cz,
-                                    int lane) {
-    double m = -1.0e-10;
-    int nc = L.nx * L.ny * L.nz;
-    const Div3 dv = div3(L.ny, L.nz);
-    for (int t = lane; t < nc; t += 64) {
-        int i, j, k;
-        split3(dv, t, i, j, k);
-        int ip = i + 1, jp = j + 1, kp = k + 1;
-        int c = lay_color(ip, jp, kp);
-        long rc = lay_row(L, ip, jp, c), ro = lay_row(L, ip, jp, c ^ 1);
-        double lu = (double)apply_lap<T, T>(L, u, rc, ro, kp >> 1, kp & 1, cx + 4 * ip, cy + 4 * jp, cz + 4 * kp);
-        m = fmax(m, fabs((double)f[rc + (kp >> 1)] - lu));
-    }
-    return wave_max(m);
-}
-
-// The same coarsest-level iteration for a level of at most 64 core nodes and 256 padded entries:
-// each lane keeps one node's neighbour indices, coefficients and right-hand side in registers, and
-// up to four ghost entries with where they take their value, so an iteration is a few LDS reads
-// per lane instead of the index arithmetic and ghost composition of every pass.  The expressions
-// are those of wv_sweep and wv_max_res, and the order of the reference loop is kept: the ghosts
-// whose source has colour c are refilled after the colour-c half sweep, which is where the next
-// imposeBC would first change them, and the colour-1 ones only after the residual, which the
-// reference evaluates before its next imposeBC (poisson_d3.cc:190-247).  Returns the iteration count.
-template <typename T>
-__device__ inline int wv_coarsest_small(const Lay &L, T *u, const T *f, const T *cx, const T *cy, const T *cz,
-                                        const Bc &bc, double tol, int max_count, int lane) {
-    const int nc = L.nx * L.ny * L.nz;
-    const bool own = lane < nc;
-    long me = 0, nb[6] = {0, 0, 0, 0, 0, 0};
-    T co[6] = {T(0), T(0), T(0), T(0), T(0), T(0)}, dg = T(1), fm = T(0);
-    int col = 2;
-    if (own) {
-        int k = lane % L.nz, r = lane / L.nz;
-        int j = r % L.ny, i = r / L.ny;
-        int ip = i + 1, jp = j + 1, kp = k + 1;
-        me = lay_idx(L, ip, jp, kp);
-        nb[0] = lay_idx(L, ip + 1, jp, kp);
-        nb[1] = lay_idx(L, ip - 1, jp, kp);
-        nb[2] = lay_idx(L, ip, jp + 1, kp);
-        nb[3] = lay_idx(L, ip, jp - 1, kp);
-        nb[4] = lay_idx(L, ip, jp, kp + 1);
-        nb[5] = lay_idx(L, ip, jp, kp - 1);
-        const T *X = cx + 4 * ip, *Y = cy + 4 * jp, *Z = cz + 4 * kp;
-        co[0] = X[0]; co[1] = X[1]; co[2] = Y[0]; co[3] = Y[1]; co[4] = Z[0]; co[5] = Z[1];
-        dg = diag3<T>(X, Y, Z);
-        fm = f[me];
-        col = (i + j + k) & 1;
-    }
-    const int NX = L.nx + 2, NY = L.ny + 2, NZ = L.nz + 2;
-    const int np = NX * NY * NZ;
-    long gd[4] = {0, 0, 0, 0}, gs[4] = {0, 0, 0, 0};
-    T gsg[4] = {T(1), T(1), T(1), T(1)}, gc[4] = {T(0), T(0), T(0), T(0)};
-    int gk[4] = {0, 0, 0, 0}, gcol[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        int p = lane + 64 * q;
-        if (p >= np) continue;
-        int kp = p % NZ, r = p / NZ;
-        int jp = r % NY, ip = r / NY;
-        if (!(ip == 0 || ip == NX - 1 || jp == 0 || jp == NY - 1 || kp == 0 || kp == NZ - 1)) continue;
-        gk[q] = ghost_source<T>(L, ip, jp, kp, bc, gs[q], gsg[q], gc[q]);
-        gd[q] = lay_idx(L, ip, jp, kp);
-        if (gk[q] == 1) {
-            // colour of the source node (lay_idx's row carries it)
-            long row = gs[q] / L.khs;
-            gcol[q] = (int)(row & 1);
-        }
-    }
-    // colour c < 2: the ghosts whose source has colour c; c == 2: every ghost
-    auto fill = [&](int c) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            if (gk[q] == 1 && (c == 2 || gcol[q] == c)) u[gd[q]] = gsg[q] * u[gs[q]];
-            else if (gk[q] == 2) u[gd[q]] = gc[q];
-        }
-    };
-    fill(2);
-    wave_sync();
-    int it = 0;
-    while (true) {
-        if (col == 0)
-            u[me] = (co[0] * u[nb[0]] + co[1] * u[nb[1]] + co[2] * u[nb[2]] + co[3] * u[nb[3]] + co[4] * u[nb[4]] +
-                     co[5] * u[nb[5]] - fm) / dg;
-        wave_sync();
-        fill(0);
-        wave_sync();
-        if (col == 1)
-            u[me] = (co[0] * u[nb[0]] + co[1] * u[nb[1]] + co[2] * u[nb[2]] + co[3] * u[nb[3]] + co[4] * u[nb[4]] +
-                     co[5] * u[nb[5]] - fm) / dg;
-        wave_sync();
-        double m = -1.0e-10;
-        if (own) {
-            T c = u[me];
-            T lu = co[0] * u[nb[0]] + co[1] * u[nb[1]] + co[2] * u[nb[2]] + co[3] * u[nb[3]] + co[4] * u[nb[4]] +
-                   co[5] * u[nb[5]] - dg * c;
-            m = fmax(m, fabs((double)fm - (double)lu));
-        }
-        const double gm = wave_max(m);
-        fill(1);
-        wave_sync();
-        if (gm < tol) break;
-        it += 1;
-        if (it > max_count) break;
-    }
-    return it;
-}
-
 // u = P f on the core nodes of the coarsest level (P transposed: pt[j * nc + i] = P[i][j]), node
 // order (i, j, k) with k fastest; ghosts are left to the caller.  FP64 accumulation.
 template <typename T>
@@ -1609,147 +1083,6 @@ __device__ inline void blk_direct(const Lay &L, T *u, const T *f, const T *__res
         u[lay_idx(L, 1 + r / L.ny, 1 + r % L.ny, 1 + k)] = (T)acc;
     }
     __syncthreads();
-}
-
-template <typename T>
-__global__ void __launch_bounds__(1024) k_coarse_cycle(CoarseDesc D, T *__restrict__ u_first, const T *__restrict__ f_first,
-                                                       int *__restrict__ iters) {
-    extern __shared__ unsigned char smem[];
-    T *base = (T *)smem;
-    __shared__ double red[16];
-    const int nl = D.last - D.first + 1;
-    // the coarsest level's dense operator (exact coarsest solve), one entry per thread, loaded now and
-    // placed in the restriction scratch for the coarsest phase, where it fits
-    const int nc2 = D.pinv ? D.ncd * D.ncd : 0;
-    const bool pt_lds = D.off_s >= 0 && nc2 > 0 && nc2 <= kTapScratch;
-    const T ptv = pt_lds && (int)threadIdx.x < nc2 ? ((const T *)D.pinv)[threadIdx.x] : T(0);
-    // coefficients and the right-hand side of the first level into LDS; u(first) starts at zero.
-    // The global loads are issued in batches before their LDS stores (each is a round trip to L2
-    // or memory; the copies of one workgroup would otherwise run one after another).
-    {
-        T cv[8][3];
-#pragma unroll
-        for (int q = 0; q < 8; q++)
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                const int cnt = q < nl ? 4 * ((a == 0 ? D.L[q].nx : a == 1 ? D.L[q].ny : D.L[q].nz) + 2) : 0;
-                cv[q][a] = (int)threadIdx.x < cnt ? ((const T *)D.cg[q][a])[threadIdx.x] : T(0);
-            }
-#pragma unroll
-        for (int q = 0; q < 8; q++)
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                const int cnt = q < nl ? 4 * ((a == 0 ? D.L[q].nx : a == 1 ? D.L[q].ny : D.L[q].nz) + 2) : 0;
-                if ((int)threadIdx.x < cnt) base[D.off_c[q][a] + threadIdx.x] = cv[q][a];
-                // arrays longer than the workgroup (not met by the coarse levels) copy the rest
-                for (int t = (int)threadIdx.x + (int)blockDim.x; t < cnt; t += blockDim.x)
-                    base[D.off_c[q][a] + t] = ((const T *)D.cg[q][a])[t];
-            }
-    }
-    {
-        const long n = lay_size(D.L[0]);
-        T *f = base + D.off_f[0];
-        const long step = blockDim.x;
-        for (long t0 = threadIdx.x; t0 < n; t0 += 8 * step) {
-            T v[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) v[q] = t0 + q * step < n ? f_first[t0 + q * step] : T(0);
-#pragma unroll
-            for (int q = 0; q < 8; q++)
-                if (t0 + q * step < n) f[t0 + q * step] = v[q];
-        }
-    }
-    __syncthreads();
-#define CX(q) (base + D.off_c[q][0])
-#define CY(q) (base + D.off_c[q][1])
-#define CZ(q) (base + D.off_c[q][2])
-#define UU(q) (base + D.off_u[q])
-#define FF(q) (base + D.off_f[q])
-    // down leg
-    for (int q = 0; q + 1 < nl; q++) {
-        const Lay &L = D.L[q];
-        for (int s = 0; s < D.pre; s++) {
-            blk_sweep<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), 0, D.bc, s == 0);
-            blk_sweep<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), 1, D.bc, false);
-        }
-        if (D.pre == 0) {
-            blk_zero<T>(L, UU(q));
-        }
-        const Lay &C = D.L[q + 1];
-        if (D.pre > 0) {
-            // the pre-smoothing ended on colour 1: only the colour-0 residual points are restricted
-            if (D.off_s >= 0 && C.nx * C.ny * C.nz <= 4 * kRbTapNodes)
-                blk_restrict_rb_taps<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), D.tbc, C, FF(q + 1), base + D.off_s);
-            else
-                blk_restrict_rb<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), D.tbc, C, FF(q + 1));
-        } else if (D.off_s >= 0 && C.nx * C.ny * C.nz <= D.tap_max) {
-            blk_restrict_taps<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), D.tbc, C, FF(q + 1), base + D.off_s);
-        } else {
-            blk_restrict<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), D.tbc, C, FF(q + 1));
-        }
-    }
-    // coarsest solve (poisson_d3.cc:190-247 with the red-black sweep)
-    {
-        int q = nl - 1;
-        const Lay &L = D.L[q];
-        blk_zero<T>(L, UU(q));
-        if (D.pinv) {
-            const T *pt = (const T *)D.pinv;
-            if (pt_lds) {
-                if ((int)threadIdx.x < nc2) base[D.off_s + threadIdx.x] = ptv;
-                __syncthreads();
-                pt = base + D.off_s;
-            }
-            blk_direct<T>(L, UU(q), FF(q), pt, D.ncd);
-            lds_fill_ghosts(L, UU(q), D.bc);
-            if (threadIdx.x == 0) iters[0] = 0;
-        } else {
-        if (D.project) blk_project<T>(L, FF(q), D.wc[0], D.wc[1], D.wc[2], D.wcsum, red);
-        const bool small = L.nx * L.ny * L.nz <= 64 && (L.nx + 2) * (L.ny + 2) * (L.nz + 2) <= 256;
-        if (small && threadIdx.x < 64) {
-            const int it = wv_coarsest_small<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), D.bc, D.tol, D.max_count,
-                                                (int)threadIdx.x);
-            if (threadIdx.x == 0) iters[0] = it;
-        } else if (threadIdx.x < 64) {
-            const int lane = threadIdx.x;
-            int it = 0;
-            while (true) {
-                wv_fill_ghosts(L, UU(q), D.bc, lane);
-                wv_sweep(L, UU(q), FF(q), CX(q), CY(q), CZ(q), 0, lane);
-                wv_fill_ghosts(L, UU(q), D.bc, lane);
-                wv_sweep(L, UU(q), FF(q), CX(q), CY(q), CZ(q), 1, lane);
-                double gm = wv_max_res<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), lane);
-                if (gm < D.tol) break;
-                it += 1;
-                if (it > D.max_count) break;
-            }
-            wv_fill_ghosts(L, UU(q), D.bc, lane);
-            if (lane == 0) iters[0] = it;
-        }
-        __syncthreads();
-        }
-    }
-    // up leg
-    const bool images = D.bc.rule[0] <= G_ANTI && D.bc.rule[1] <= G_ANTI && D.bc.rule[2] <= G_ANTI;
-    for (int q = nl - 2; q >= 0; q--) {
-        const Lay &L = D.L[q];
-        blk_prolong_add<T>(L, UU(q), D.L[q + 1], UU(q + 1), D.bc, images, D.post > 0 ? 1 : -1);
-        if (!images) lds_fill_ghosts(L, UU(q), D.bc);
-        for (int s = 0; s < D.post; s++) {
-            blk_sweep<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), 0, D.bc, false);
-            blk_sweep<T>(L, UU(q), FF(q), CX(q), CY(q), CZ(q), 1, D.bc, false);
-        }
-    }
-    {
-        long n = lay_size(D.L[0]);
-        T *u = UU(0);
-        for (long t = threadIdx.x; t < n; t += blockDim.x) u_first[t] = u[t];
-    }
-#undef CX
-#undef CY
-#undef CZ
-#undef UU
-#undef FF
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2003,36 +1336,6 @@ void launch_coarsest_direct(const Lay &L, T *u, const T *f, const T *pt, int nc,
     hipLaunchKernelGGL(k_coarsest_direct<T>, dim3(1), dim3(1024), 0, s, L, u, f, pt, nc, bc, iters);
 }
 
-template <typename T>
-size_t coarse_cycle_plan(CoarseDesc &D, size_t limit) {
-    size_t off = 0;
-    auto take = [&](size_t n) { size_t o = off; off += (n + 7) & ~(size_t)7; return (int)o; };
-    for (int q = 0; q <= D.last - D.first; q++) {
-        const Lay &L = D.L[q];
-        D.off_u[q] = take((size_t)lay_size(L));
-        D.off_f[q] = take((size_t)lay_size(L));
-        D.off_c[q][0] = take(4 * (size_t)(L.nx + 2));
-        D.off_c[q][1] = take(4 * (size_t)(L.ny + 2));
-        D.off_c[q][2] = take(4 * (size_t)(L.nz + 2));
-    }
-    // scratch of the tap-parallel restriction, where it fits
-    D.off_s = -1;
-    D.tap_max = 4 * kTapNodes;
-    if ((off + kTapScratch + 8) * sizeof(T) <= limit) D.off_s = take(kTapScratch);
-    return off * sizeof(T);
-}
-
-template <typename T>
-void launch_coarse_cycle(const CoarseDesc &D, size_t lds, T *u_first, const T *f_first, int *iters, hipStream_t s) {
-    hipLaunchKernelGGL(k_coarse_cycle<T>, dim3(1), dim3(1024), lds, s, D, u_first, f_first, iters);
-}
-
-template <typename T>
-int coarse_cycle_attr(size_t lds) {
-    return hipFuncSetAttribute((const void *)k_coarse_cycle<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==
-                   hipSuccess ? 0 : 1;
-}
-
 // explicit instantiations
 #define SR_INST(T)                                                                                          \
     template void launch_fill_ghosts<T>(const Lay &, T *, const Bc &, hipStream_t);                        \
@@ -2058,12 +1361,6 @@ int coarse_cycle_attr(size_t lds) {
                                           double, hipStream_t);
 SR_INST(double)
 SR_INST(float)
-template size_t coarse_cycle_plan<double>(CoarseDesc &, size_t);
-template size_t coarse_cycle_plan<float>(CoarseDesc &, size_t);
-template void launch_coarse_cycle<double>(const CoarseDesc &, size_t, double *, const double *, int *, hipStream_t);
-template void launch_coarse_cycle<float>(const CoarseDesc &, size_t, float *, const float *, int *, hipStream_t);
-template int coarse_cycle_attr<double>(size_t);
-template int coarse_cycle_attr<float>(size_t);
 #undef SR_INST
 
 template void launch_residual<double, double>(const Lay &, const double *, const double *, double *,

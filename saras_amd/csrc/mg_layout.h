@@ -63,7 +63,8 @@ struct CoarseDesc {
     int first, last;
     Lay L[8];
     int off_u[8], off_f[8], off_c[8][3];
-    const void *cg[8][3];
+    const void *coef;   // the levels' coefficient arrays in one block, as LDS holds them from off_c[0][0]
+    int ncoef;          // its elements
     int pre, post;
     Bc bc;       // smoothing ghosts of the coarse levels (zeroBC = 1)
     Bc tbc;      // residual pads read by the restriction
@@ -74,8 +75,7 @@ struct CoarseDesc {
     double wcsum;
     const void *pinv;   // dense coarsest inverse, transposed (T), or null: Gauss-Seidel to tol
     int ncd;            // coarsest core nodes (rows of pinv)
-    int off_s;          // scratch of the tap-parallel restriction, or -1 (none)
-    int tap_max;        // coarse levels of at most this many core nodes use it
+    int off_s;          // scratch: one colour of the first level
 };
 
 // Buffers of a two-stage final reduction (k_gcr_coef_mb): FINAL_STAGE doubles

@@ -61,6 +61,8 @@ struct sr_mg {
     int coarse_first64 = 1 << 20, coarse_first32 = 1 << 20;
     sr::CoarseDesc cdesc64{}, cdesc32{};
     size_t clds64 = 0, clds32 = 0;
+    double *ccoef64 = nullptr;   // the coarse levels' coefficients in LDS order
+    float *ccoef32 = nullptr;
     int coarse_enable = 1;
     long lds_limit = 0;
     hipGraph_t graph_mixed_g[2] = {nullptr, nullptr};

@@ -8,7 +8,8 @@ import numpy as np
 import pytest
 
 from helpers import Problem, r2_walls
-from test_mg_gpu import _vcycle_iterates
+from oracle import pyoracle as po
+from test_mg_gpu import RTOL
 
 pytestmark = pytest.mark.gpu
 
@@ -28,19 +29,55 @@ CASES = [
     ((7, 5, 5), "PPN", "UUD", 2, 2, False),
 ]
 
+# the one-workgroup coarse end (saras_amd/csrc/mg_coarse.hip): its first level with one and three entries
+# per thread and with more items than threads, no pre- or post-smoothing, coarsest levels of one wave, of
+# the workgroup and (17 x 17 x 5 nodes) of more nodes than the workgroup has threads, which are solved
+# outside it
+COARSE = [
+    ((4, 4, 4), "PPN", "UUD", 2, 2, False, None),
+    ((5, 5, 5), "NNN", "DDD", 2, 1, False, None),
+    ((5, 5, 5), "PPP", "UUU", 0, 2, False, None),
+    ((5, 5, 5), "NPN", "DUD", 1, 0, False, None),
+    ((5, 5, 5), "PNP", "UDU", 0, 0, False, None),
+    ((6, 6, 5), "PPN", "UUD", 2, 2, False, 3),
+    ((6, 5, 4), "NNN", "UUU", 3, 2, True, None),
+    ((5, 6, 5), "NNP", "UUU", 2, 2, True, None),
+    ((5, 5, 5), "NNN", "UUU", 0, 2, True, None),
+    ((6, 6, 4), "PPN", "UUD", 2, 2, False, 2),
+]
 
-def _problem(ind, domain, mesh, pre, post, walls, **kw):
+
+def _problem(ind, domain, mesh, pre, post, walls, depth=None, **kw):
     n = [(1 << k) + 1 for k in ind]
     m = min(ind)
     return Problem(ind=ind, domain=domain, mesh=mesh, L=tuple(float(1 << (k - m)) for k in ind), pre=pre, post=post,
-                   test_poisson=walls, walls=r2_walls(n) if walls else None, **kw)
+                   depth=depth, test_poisson=walls, walls=r2_walls(n) if walls else None, **kw)
 
 
-@pytest.mark.parametrize("case", CASES, ids=str)
+@pytest.mark.parametrize("case", CASES + COARSE, ids=str)
 def test_vcycle_matches_oracle(case):
+    """Three iterates within the per-operator bar.  Without Dirichlet walls the operator is singular and
+    the coarsest iteration runs to its limit (up to 2000 times here), each step moving the level of the
+    iterate by its rounding: as for the pressures of a time step, the level is taken out."""
     pb = _problem(*case)
     o, g = pb.oracle(), pb.gpu()
-    _vcycle_iterates(pb, o, g)
+    P0, F0 = np.random.default_rng(7).standard_normal(pb.shape), pb.random_rhs(8)
+    o.level = 0
+    o.array(po.P, 0)[...] = P0
+    o.array(po.R, 0)[...] = F0
+    g.upload(po.P, 0, P0)
+    g.upload(po.R, 0, F0)
+    for it in range(3):
+        o.vcycle()
+        g.vCycle()
+        o.set_zero_bc(0)
+        g.set_zeroBC(0)
+        o.impose_bc()
+        g.imposeBC()
+        exp, d = o.array(po.P, 0), g.download(po.P, 0) - o.array(po.P, 0)
+        if not case[5]:
+            d = d - d[1:-1, 1:-1, 1:-1].mean()
+        assert np.max(np.abs(d)) <= RTOL * np.max(np.abs(exp)), (it, np.max(np.abs(d)), np.max(np.abs(exp)))
     g.close()
 
 
