@@ -307,7 +307,7 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
         for (int q = 0; q < 2; q++) launch_fill<float>(m->zdir[q], sz, 0.0f, m->stream);
     }
     if (d->coarseDirect) RETCHK(build_coarse_direct(m));
-    if (rb_pass_attr()) return set_err(SR_ERR_HIP, "LDS size of the sweep kernels refused");
+    if (rb_pass_attr() || march_outer_attr()) return set_err(SR_ERR_HIP, "LDS size of the sweep kernels refused");
     // coarse end of the cycle in LDS
     {
         int dev = 0, lds_max = 65536;
@@ -366,6 +366,7 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
     int nparts = norm_parts(F);
     HIPCHK(hipMalloc((void **)&m->part, sizeof(double) * 4 * (size_t)nparts));
     HIPCHK(hipMalloc((void **)&m->part2, sizeof(double) * 2 * (size_t)norm_res_parts(F)));
+    HIPCHK(hipMalloc((void **)&m->mpart, sizeof(double) * (6 * (size_t)march_parts(F) + 1)));
     HIPCHK(hipMalloc((void **)&m->fterms, sizeof(double) * 4));
     HIPCHK(hipMalloc((void **)&m->fstage, sizeof(double) * FINAL_STAGE));
     HIPCHK(hipMalloc((void **)&m->fcount, sizeof(unsigned)));
@@ -416,7 +417,7 @@ extern "C" int sr_mg_destroy(sr_mg *m) {
     }
     for (int q = 0; q < 6; q++) (void)hipFree(m->wall[q]);
     for (int a = 0; a < 3; a++) (void)hipFree(m->wvec[a]);
-    (void)hipFree(m->part); (void)hipFree(m->part2); (void)hipFree(m->fterms); (void)hipFree(m->fstage); (void)hipFree(m->fcount); (void)hipFree(m->dres); (void)hipFree(m->diters); (void)hipFree(m->stage);
+    (void)hipFree(m->part); (void)hipFree(m->part2); (void)hipFree(m->mpart); (void)hipFree(m->fterms); (void)hipFree(m->fstage); (void)hipFree(m->fcount); (void)hipFree(m->dres); (void)hipFree(m->diters); (void)hipFree(m->stage);
     (void)hipFree(m->stage2); (void)hipFree(m->r32);
     if (m->hres) (void)hipHostFree(m->hres);
     if (m->ev0) (void)hipEventDestroy(m->ev0);

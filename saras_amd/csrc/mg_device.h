@@ -68,4 +68,46 @@ __device__ inline void write_images(const Lay &L, T *u, int ip, int jp, int kp, 
     }
 }
 
+__device__ inline double wave_sum(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+__device__ inline double wave_max(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// Whether this workgroup is the last of the grid to get here (a device-scope counter, zero before the
+// launch, which the caller resets): what the others wrote before is then visible to it.
+__device__ inline bool last_block_done(unsigned *counter) {
+    __shared__ bool last;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        last = atomicAdd(counter, 1u) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (last) __threadfence();
+    return last;
+}
+
+// alpha, beta of the step from the block sums; coef = {alpha, beta, (r q), (q q), (q p), (r p), (p p)}.
+// When the orthogonalised direction has lost most of its norm to cancellation (or there is no
+// previous direction) the step falls back to the minimal-residual step along e.
+__device__ inline void gcr_coef_from(const double (&t)[5], double *coef) {
+    double rq = t[0], qq = t[1], qp = t[2], rp = t[3], pp = t[4];
+    double beta = pp > 0.0 ? qp / pp : 0.0;
+    double qn = qq - 2.0 * beta * qp + beta * beta * pp;
+    if (!(qn >= 1e-3 * qq)) {
+        beta = 0.0;
+        qn = qq;
+    }
+    double alpha = qn > 0.0 ? (rq - beta * rp) / qn : 0.0;
+    coef[0] = alpha;
+    coef[1] = beta;
+    for (int i = 0; i < 5; i++) coef[2 + i] = t[i];
+}
+
 }  // namespace sr

@@ -91,6 +91,26 @@ void launch_gcr_dots(const Lay &L, const float *e, const float *z, const float *
                      const FinalBufs *fb = nullptr);
 void launch_gcr_step(const Lay &L, const double *x_in, const float *e, const float *z, const double *coef,
                      double *x_out, float *z_next, const Bc &bc, const Bc &ebc, hipStream_t s);
+// The same steps and norms as marches over x with their reductions inside (mg_outer.hip), for the sizes
+// and ghost rules of march_outer_ok.  Ghosts are neither read nor written; S.out gets the four
+// quantities of computeError, as does S.host (pinned, may be null), so that no copy is needed.  e and
+// z select the step (see there); r32 null: norms only, color0: of colour 0.
+struct MarchSums {
+    double *part;        // 6 doubles per march_parts(L)
+    unsigned *counter;   // zero between launches
+    const double *fterms;
+    double *out, *host;
+};
+bool march_outer_ok(const Lay &L, const Bc &bc);
+int march_parts(const Lay &L);
+int march_outer_attr();   // once per device, before the first launch
+void launch_march_residual(const Lay &L, const double *x_in, const float *e, const float *z, const double *coef,
+                           const double *f, double *x_out, float *z_next, float *r32, const double *cx,
+                           const double *cy, const double *cz, const Bc &bc, bool color0, const MarchSums &S,
+                           hipStream_t s);
+void launch_march_dots(const Lay &L, const float *e, const float *z, const float *r32, const float *cx, const float *cy,
+                       const float *cz, const Bc &bc, bool q1r, double *part, unsigned *counter, double *coef,
+                       hipStream_t s);
 // exact coarsest solve u = P f with the dense inverse (transposed, nc x nc), ghosts filled by bc
 template <typename T>
 void launch_coarsest_direct(const Lay &L, T *u, const T *f, const T *pt, int nc, const Bc &bc, int *iters,

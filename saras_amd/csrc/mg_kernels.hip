@@ -437,17 +437,6 @@ __global__ void __launch_bounds__(256) k_unpack(Lay L, const TS *__restrict__ sr
 // ------------------------------------------------------------------------------------------------
 constexpr int NQ = 4;   // quantities per partial
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-__device__ inline double wave_max(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // q[0] += sum, q[1] += sum, q[2] = max, q[3] = max over the block; written to part[block*NQ + i]
 __device__ inline void block_reduce4(double s0, double s1, double m2, double m3, double *part) {
     __shared__ double sh[4][4];
@@ -569,19 +558,6 @@ __global__ void __launch_bounds__(1024) k_norm_combine(const double *__restrict_
 // depend on the order in which the workgroups finish.
 constexpr int FINAL_BLOCKS = 16;
 static_assert(FINAL_BLOCKS * 5 <= FINAL_STAGE, "stage buffer of the two-stage finals");
-
-__device__ inline bool last_block_done(unsigned *counter) {
-    __shared__ bool last;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        last = atomicAdd(counter, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (last) __threadfence();
-    return last;
-}
-
 
 // sum f^2 over the core and max |f| over every padded node
 template <typename T>
@@ -961,23 +937,6 @@ __global__ void __launch_bounds__(256) k_gcr_dots(Lay L, Geo G, const float *__r
         for (int w = 0; w < 4; w++) a += sh[w][threadIdx.x];
         part[5 * (long)blockIdx.x + threadIdx.x] = a;
     }
-}
-
-// alpha, beta of the step from the block sums; coef = {alpha, beta, (r q), (q q), (q p), (r p), (p p)}.
-// When the orthogonalised direction has lost most of its norm to cancellation (or there is no
-// previous direction) the step falls back to the minimal-residual step along e.
-__device__ inline void gcr_coef_from(const double (&t)[5], double *coef) {
-    double rq = t[0], qq = t[1], qp = t[2], rp = t[3], pp = t[4];
-    double beta = pp > 0.0 ? qp / pp : 0.0;
-    double qn = qq - 2.0 * beta * qp + beta * beta * pp;
-    if (!(qn >= 1e-3 * qq)) {
-        beta = 0.0;
-        qn = qq;
-    }
-    double alpha = qn > 0.0 ? (rq - beta * rp) / qn : 0.0;
-    coef[0] = alpha;
-    coef[1] = beta;
-    for (int i = 0; i < 5; i++) coef[2 + i] = t[i];
 }
 
 __global__ void __launch_bounds__(1024) k_gcr_coef(const double *__restrict__ part, int nb, double *__restrict__ coef) {

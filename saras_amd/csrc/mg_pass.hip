@@ -2,8 +2,8 @@
 //
 // Two half sweeps (k_rb_sweep) read the neighbour values of every node through seven vector loads and
 // are held by the address unit, not by HBM: 121 us (FP64) and 63 us (FP32) a sweep at 257^3, where a
-// sweep has to move 323 and 161 MB with its halos.  This kernel takes 56 and 39 us, 82 and 45 us as the
-// last sweep of a smoothing, which stores colour 0 too: 4.7-5.8 TB/s in FP64, about the rate of a large
+// sweep has to move 323 and 161 MB with its halos.  This kernel takes 55 and 40 us, 71 and 47 us as the
+// last sweep of a smoothing, which stores colour 0 too: 5.4-5.9 TB/s in FP64, about the rate of a large
 // copy; in FP32 it is bound by its instructions (190 vector instructions per four nodes).
 //
 // A workgroup marches over the planes of a chunk of x with a tile of y rows and the whole of z.  Each
@@ -22,54 +22,12 @@
 // written, as k_rb_sweep writes them.
 #include "mg_kernels.h"
 
-#include "mg_device.h"
+#include "mg_march.h"
 #include "xcd.h"
 
 namespace sr {
-namespace {
-
-template <typename T> struct Pair { T a, b; };
-
-// two consecutive entries at a 32-bit byte offset from a base that is the same for the whole wave
-template <typename T>
-__device__ __forceinline__ Pair<T> ld2(const T *base, unsigned off) {
-    typedef T V2 __attribute__((ext_vector_type(2)));
-    const V2 v = *reinterpret_cast<const V2 *>(reinterpret_cast<const char *>(base) + off);
-    return Pair<T>{v.x, v.y};
-}
-template <typename T>
-__device__ __forceinline__ void st2(T *base, unsigned off, const Pair<T> &v) {
-    typedef T V2 __attribute__((ext_vector_type(2)));
-    V2 w;
-    w.x = v.a;
-    w.y = v.b;
-    *reinterpret_cast<V2 *>(reinterpret_cast<char *>(base) + off) = w;
-}
-template <typename T>
-__device__ __forceinline__ void st1(T *base, unsigned off, T v) {
-    *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off) = v;
-}
-
-// coefficients of one direction at one index: c+, c- and, in FP32, the separately rounded centre
-// (see diag3)
-template <typename T> struct Co;
-template <> struct alignas(16) Co<double> { double p, m; };
-template <> struct alignas(16) Co<float> { float p, m, c, pad; };
-__device__ __forceinline__ double cen(const Co<double> &q) { return q.p + q.m; }
-__device__ __forceinline__ float cen(const Co<float> &q) { return q.c; }
-__device__ __forceinline__ Co<double> ldco(const double *q) { return Co<double>{q[0], q[1]}; }
-__device__ __forceinline__ Co<float> ldco(const float *q) { return Co<float>{q[0], q[1], q[2], 0.0f}; }
-
-}  // namespace
-
-struct PassGeo {
-    int ntile, nch, tpr;      // row tiles, chunks of x, threads per row
-    int tq, tr, cq, cr;       // rows per tile and planes per chunk: quotient and remainder
-    float inv_tpr;
-};
-
 template <typename T, bool ZERO, bool LAST, bool ZPER>
-__global__ void __launch_bounds__(1024) k_rb_pass(Lay L, PassGeo G, const T *__restrict__ ub, T *__restrict__ u,
+__global__ void __launch_bounds__(1024) k_rb_pass(Lay L, MarchGeo G, const T *__restrict__ ub, T *__restrict__ u,
                                                   T *__restrict__ bo, const T *__restrict__ f,
                                                   const T *__restrict__ cx, const T *__restrict__ cy,
                                                   const T *__restrict__ cz, Bc bc) {
@@ -156,7 +114,7 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, PassGeo G, const T *__r
     const bool yi0 = sj == ghost_src(bc.rule[1], 0, ny), yimg = yi0 || sj == ghost_src(bc.rule[1], ny + 1, ny);
     // colour c at core plane i, with the face-ghost images of all directions where they are wanted
     auto store = [&](T *dst, int i, int c, const Pair<T> &v, bool kb) {
-        const unsigned o = c ? vo1 : vo0;
+        const unsigned o = here(c ? vo1 : vo0);
         store_row(dst + i * ps, o, v, kb);
         if (!LAST) return;
         if (yimg)
@@ -187,15 +145,15 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, PassGeo G, const T *__r
         if (p == i0 - 1 || s != p || (p == i0 && i0 == 1)) {
             // the first plane, and the planes at a ghost plane, load all that their update needs
             X = ldco(cx + 4 * s);
-            f0 = ld2(f + s * ps, vo0);
+            f0 = ld2(f + s * ps, here(vo0));
             if (!ZERO) {
                 const int sm = src(0, s - 1, nx), sp = src(0, s + 1, nx);
-                Bm = ld2(ub + sm * ps, vo1);
-                Bc_ = ld2(ub + s * ps, vo1);
-                Bp = ld2(ub + sp * ps, vo1);
+                Bm = ld2(ub + sm * ps, here(vo1));
+                Bc_ = ld2(ub + s * ps, here(vo1));
+                Bp = ld2(ub + sp * ps, here(vo1));
                 if (halo) {
-                    Ym[par] = ld2(ub + s * ps, vom);
-                    Yp[par] = ld2(ub + s * ps, vop);
+                    Ym[par] = ld2(ub + s * ps, here(vom));
+                    Yp[par] = ld2(ub + s * ps, here(vop));
                 }
                 if (antix && sm != s - 1) Bm = Pair<T>{-Bm.a, -Bm.b};
                 if (antix && sp != s + 1) Bp = Pair<T>{-Bp.a, -Bp.b};
@@ -217,15 +175,15 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, PassGeo G, const T *__r
         if (p < i1) {
             const int s1 = src(0, p + 1, nx);
             Xn = ldco(cx + 4 * s1);
-            f0n = ld2(f + s1 * ps, vo0);
+            f0n = ld2(f + s1 * ps, here(vo0));
             if (!ZERO) {
-                Bn = ld2(ub + src(0, min(p + 2, nx + 1), nx) * ps, vo1);
+                Bn = ld2(ub + src(0, min(p + 2, nx + 1), nx) * ps, here(vo1));
                 if (halo) {
-                    Ym[par ^ 1] = ld2(ub + s1 * ps, vom);
-                    Yp[par ^ 1] = ld2(ub + s1 * ps, vop);
+                    Ym[par ^ 1] = ld2(ub + s1 * ps, here(vom));
+                    Yp[par ^ 1] = ld2(ub + s1 * ps, here(vop));
                 }
             }
-            f1n = ld2(f + s * ps, vo1);
+            f1n = ld2(f + s * ps, here(vo1));
         }
         const bool kb = (1 + p + jp) & 1;
         const Co<T> Z0 = lz[(kb ? G.tpr : 0) + t], Z1 = lz[(kb ? 3 * G.tpr : 2 * G.tpr) + t];
@@ -263,50 +221,11 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, PassGeo G, const T *__r
     if (!halo) store(bo, i1 - 1, 1, Bs, (1 + i1 + jp) & 1);
 }
 
-namespace {
-
-struct Plan {
-    PassGeo g;
-    int R;
-    size_t lds;
-};
-
-// Tiles of up to 13 rows (15 thread rows with the halo rows: 15 % of colour 0 updated twice) and as
-// many chunks of x as give every CU its share of workgroups: one of 1024 threads (257 nodes along z:
-// 240 workgroups of 21 planes), two of half that.  More chunks cost two planes each, fewer leave CUs
-// idle.  Measured (us per solve or step, R = 15 / 11 / 19 rows with 512 workgroups): 129^3 step
-// 3077 / 3135 / 3343, 65^3 GCR solve 1424 / 1446 / 1499; 15 rows with 256 workgroups 3140 and 1464.
-// At 257^3 in FP64 1024 threads and 256 workgroups take 12.56 ms per solve, 512 threads and 512
-// workgroups 12.85 ms, 715 threads and 512 workgroups 13.26 ms.
-template <typename T>
-Plan plan(const Lay &L) {
-    Plan P{};
-    P.g.tpr = L.kh / 2;
-    P.g.inv_tpr = 1.0f / (float)P.g.tpr;
-    int R = 1024 / P.g.tpr;
-    if (R > 15) R = 15;
-    if (R > L.ny + 2) R = L.ny + 2;
-    P.g.ntile = (L.ny + R - 3) / (R - 2);
-    P.g.tq = L.ny / P.g.ntile;
-    P.g.tr = L.ny % P.g.ntile;
-    P.R = P.g.tq + (P.g.tr > 0) + 2;
-    P.g.nch = (P.R * P.g.tpr > 512 ? 256 : 512) / P.g.ntile;
-    if (P.g.nch < 1) P.g.nch = 1;
-    if (P.g.nch > L.nx) P.g.nch = L.nx;
-    P.g.cq = L.nx / P.g.nch;
-    P.g.cr = L.nx % P.g.nch;
-    P.lds = 4 * (size_t)P.R * L.khs * sizeof(T) + 4 * (size_t)P.g.tpr * sizeof(Co<T>);
-    return P;
-}
-
-}  // namespace
-
-// Image rules only; rows of an even number of entries of which at least six fit a workgroup (a z
-// direction of at most 513 nodes; beyond that the halo rows outweigh the tile).
+// Image rules only (and march_ok's sizes).
 bool rb_pass_ok(const Lay &L, const Bc &bc) {
     for (int d = 0; d < 3; d++)
         if (bc.rule[d] > G_ANTI) return false;
-    return L.kh % 2 == 0 && L.nx >= 5 && L.ny >= 5 && L.nz >= 5 && L.kh / 2 <= 170;
+    return march_ok(L);
 }
 
 template <typename T, bool ZERO, bool LAST, bool ZPER>
@@ -325,9 +244,10 @@ int rb_pass_attr() { return attr8<double>() | attr8<float>(); }
 template <typename T>
 void launch_rb_pass(const Lay &L, const T *ub, T *u, T *bo, const T *f, const T *cx, const T *cy, const T *cz,
                     const Bc &bc, bool zero, bool last, hipStream_t s) {
-    const Plan P = plan<T>(L);
-    const dim3 grid(P.g.ntile * P.g.nch), blk(P.R * P.g.tpr);
-    auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, blk, P.lds, s, L, P.g, ub, u, bo, f, cx, cy, cz, bc); };
+    const MarchPlan P = march_plan(L);
+    const dim3 grid(P.blocks()), blk(P.threads());
+    const size_t lds = 4 * (size_t)P.R * L.khs * sizeof(T) + 4 * (size_t)P.g.tpr * sizeof(Co<T>);
+    auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, blk, lds, s, L, P.g, ub, u, bo, f, cx, cy, cz, bc); };
     const bool zper = bc.rule[2] == G_PERIODIC;
     if (zero && last) zper ? go(k_rb_pass<T, true, true, true>) : go(k_rb_pass<T, true, true, false>);
     else if (zero) zper ? go(k_rb_pass<T, true, false, true>) : go(k_rb_pass<T, true, false, false>);

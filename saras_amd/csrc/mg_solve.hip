@@ -92,12 +92,31 @@ static int norm_order(const sr_mg *m) {
     return m->d.semantics == SR_SEM_PROJECTED ? 2 : m->d.resType;
 }
 
+// Whether level 0 takes the marching kernels (mg_outer.hip), which leave the reduced quantities in the
+// host mirror themselves.
+static bool march0(const sr_mg *m) { return march_outer_ok(m->lv[0].L, pressure_bc(m, 0, 0)); }
+
+// One outer step as a march: from x_in, with e (refinement) or e and z (GCR) into x_out; without r32 the
+// norms of f - L x_in alone.
+static void march_step(sr_mg *m, const double *x_in, const float *e, const float *z, double *x_out, float *z_next,
+                       float *r32, bool color0 = false) {
+    Level &V = m->lv[0];
+    const MarchSums S{m->mpart, m->fcount, m->fterms, m->dres, m->hres};
+    launch_march_residual(V.L, x_in, e, z, m->gcoef, V.f, x_out, z_next, r32, V.c64[0], V.c64[1], V.c64[2],
+                          pressure_bc(m, 0, 0), color0, S, m->stream);
+}
+
 // one FP64 cycle plus its norm and the read-back of the reduced quantities
 static void cycle_fp64(sr_mg *m) {
     vcycle_fp64(m);
     // a Gauss-Seidel cycle ends on a colour-1 half sweep of level 0, which leaves the colour-1
     // residual zero (up to the rounding of f - Lu): the norm is taken over colour 0
-    norm_level0(m, m->d.gsSmooth && m->d.postSmooth > 0 ? 0 : -1);
+    const bool color0 = m->d.gsSmooth && m->d.postSmooth > 0;
+    if (march0(m)) {
+        march_step(m, m->lv[0].u, nullptr, nullptr, nullptr, nullptr, nullptr, color0);
+        return;
+    }
+    norm_level0(m, color0 ? 0 : -1);
     read_back(m);
 }
 
@@ -195,6 +214,7 @@ static int solve_fp64(sr_mg *m, int &cycles, double &res, bool &conv, double &sw
 static void mixed_body_ab(sr_mg *m) {
     Level &V = m->lv[0];
     vcycle_fp32(m);
+    if (march0(m)) return march_step(m, V.u, V.u32, nullptr, V.t, nullptr, V.f32);
     launch_outer_residual(V.L, V.u, V.u32, V.f, V.t, V.f32, V.c64[0], V.c64[1], V.c64[2], pressure_bc(m, 0, 0),
                           m->part2, m->fterms, m->dres, m->stream);
     read_back(m);
@@ -203,6 +223,7 @@ static void mixed_body_ab(sr_mg *m) {
 static void mixed_body_ba(sr_mg *m) {
     Level &V = m->lv[0];
     vcycle_fp32(m);
+    if (march0(m)) return march_step(m, V.t, V.u32, nullptr, V.u, nullptr, V.f32);
     launch_outer_residual(V.L, V.t, V.u32, V.f, V.u, V.f32, V.c64[0], V.c64[1], V.c64[2], pressure_bc(m, 0, 0),
                           m->part2, m->fterms, m->dres, m->stream);
     read_back(m);
@@ -223,13 +244,18 @@ static int solve_mixed(sr_mg *m, int &cycles, double &res, bool &conv, double &s
     RETCHK(ensure_fp32(m));
     Level &V = m->lv[0];
     long sz = lay_size(V.L);
-    // ghosts of the initial guess under its own BCs (Dirichlet walls included), then the second
-    // buffer of the pair inherits them; wall ghosts are never rewritten afterwards
-    launch_fill_ghosts<double>(V.L, V.u, pressure_bc(m, 0, 0), m->stream);
-    HIPCHK(hipMemcpyAsync(V.t, V.u, sizeof(double) * sz, hipMemcpyDeviceToDevice, m->stream));
-    launch_outer_residual(V.L, V.u, nullptr, V.f, nullptr, V.f32, V.c64[0], V.c64[1], V.c64[2],
-                          pressure_bc(m, 0, 0), m->part2, m->fterms, m->dres, m->stream);
-    HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, m->stream));
+    if (march0(m)) {
+        march_step(m, V.u, nullptr, nullptr, nullptr, nullptr, V.f32);
+        HIPCHK(hipGetLastError());
+    } else {
+        // ghosts of the initial guess under its own BCs (Dirichlet walls included), then the second
+        // buffer of the pair inherits them; wall ghosts are never rewritten afterwards
+        launch_fill_ghosts<double>(V.L, V.u, pressure_bc(m, 0, 0), m->stream);
+        HIPCHK(hipMemcpyAsync(V.t, V.u, sizeof(double) * sz, hipMemcpyDeviceToDevice, m->stream));
+        launch_outer_residual(V.L, V.u, nullptr, V.f, nullptr, V.f32, V.c64[0], V.c64[1], V.c64[2],
+                              pressure_bc(m, 0, 0), m->part2, m->fterms, m->dres, m->stream);
+        HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, m->stream));
+    }
     HIPCHK(hipStreamSynchronize(m->stream));
     int nt = norm_order(m);
     double r = error_from(m, m->hres, nt);
@@ -285,6 +311,12 @@ static void gcr_body(sr_mg *m, int cur) {
     // above the bottom of the cycle and has post-smoothing sweeps
     const int Lc = m->coarse_enable ? m->coarse_first32 : (1 << 20);
     const bool q1r = std::min(Lc, m->depth) >= 1 && m->post32 > 0;
+    if (march0(m)) {
+        launch_march_dots(V.L, V.u32, z, V.f32, V.c32[0], V.c32[1], V.c32[2], error_bc(m, 0, 0), q1r, m->mpart,
+                          m->fcount, m->gcoef, s);
+        march_step(m, x_in, V.u32, z, x_out, z_next, V.f32);
+        return;
+    }
     launch_gcr_dots(V.L, V.u32, z, V.f32, V.c32[0], V.c32[1], V.c32[2], m->gpart, m->gcoef, q1r, s,
                     &m->fb_coef);
     launch_gcr_step(V.L, x_in, V.u32, z, m->gcoef, x_out, z_next, pressure_bc(m, 0, 0), error_bc(m, 0, 0), s);
@@ -311,16 +343,22 @@ static int solve_gcr(sr_mg *m, int &cycles, double &res, bool &conv, double &swe
     long sz = lay_size(V.L);
     hipStream_t s = m->stream;
     Bc bc0 = pressure_bc(m, 0, 0);
-    launch_fill_ghosts<double>(V.L, V.u, bc0, s);
+    const bool march = march0(m);
+    if (!march) launch_fill_ghosts<double>(V.L, V.u, bc0, s);
     // the second iterate buffer needs the fixed wall ghosts only; every other face ghost is
     // rewritten as an image by each update
     if (bc0.rule[0] == G_WALL || bc0.rule[1] == G_WALL || bc0.rule[2] == G_WALL)
         HIPCHK(hipMemcpyAsync(V.t, V.u, sizeof(double) * sz, hipMemcpyDeviceToDevice, s));
     // no previous direction: the first step is the minimal-residual step along the cycle's result
     launch_fill<float>(m->zdir[0], sz, 0.0f, s);
-    launch_outer_residual(V.L, V.u, nullptr, V.f, nullptr, V.f32, V.c64[0], V.c64[1], V.c64[2],
-                          pressure_bc(m, 0, 0), m->part2, m->fterms, m->dres, s);
-    HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, s));
+    if (march) {
+        march_step(m, V.u, nullptr, nullptr, nullptr, nullptr, V.f32);
+        HIPCHK(hipGetLastError());
+    } else {
+        launch_outer_residual(V.L, V.u, nullptr, V.f, nullptr, V.f32, V.c64[0], V.c64[1], V.c64[2],
+                              pressure_bc(m, 0, 0), m->part2, m->fterms, m->dres, s);
+        HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, s));
+    }
     HIPCHK(hipStreamSynchronize(s));
     int nt = norm_order(m);
     double r = error_from(m, m->hres, nt);
@@ -366,9 +404,15 @@ extern "C" int sr_mg_residual(sr_mg *m, const double *p, const double *rhs, doub
     if (!m || !p || !rhs) return set_err(SR_ERR_ARG, "null argument");
     Level &V = m->lv[0];
     load_level0(m, rhs, p);
-    launch_fill_ghosts<double>(V.L, V.u, pressure_bc(m, 0, 0), m->stream);
-    norm_level0(m);
-    HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, m->stream));
+    const bool march = march0(m);
+    if (r || !march) launch_fill_ghosts<double>(V.L, V.u, pressure_bc(m, 0, 0), m->stream);
+    if (march) {
+        poison_hres(m);
+        march_step(m, V.u, nullptr, nullptr, nullptr, nullptr, nullptr);
+    } else {
+        norm_level0(m);
+        HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, m->stream));
+    }
     if (r) {
         residual_level(m, 0);
         launch_unpack<double, double>(V.L, V.t, r, m->stream);

@@ -45,6 +45,7 @@ struct sr_mg {
     double wsum = 0;
     double *part = nullptr;      // reduction partials
     double *part2 = nullptr;     // per-block (sum, max) partials of the level-0 residual norm
+    double *mpart = nullptr;     // per-workgroup sums of the marching kernels
     double *fterms = nullptr;    // right-hand side terms of computeError (device, 4 doubles)
     double *fstage = nullptr;    // stage of the GCR coefficients' two-stage final (FINAL_STAGE doubles)
     unsigned *fcount = nullptr;  // its counter (zero between launches)

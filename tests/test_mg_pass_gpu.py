@@ -95,3 +95,59 @@ def test_fp32_cycles_follow_fp64(case):
         g.close()
     tol = 4 * max(pb.n) ** 2 * 6e-8
     assert len(hist[0]) == 2 and np.max(np.abs(hist[0] - hist[1])) <= tol * max(1.0, hist[0][0]), (hist, tol)
+
+
+# marching outer step (saras_amd/csrc/mg_outer.hip): also no post-smoothing, whose L e is formed on both colours
+OUTER = [c for c in CASES if not c[5]] + [((5, 5, 4), "NPN", "DUD", 2, 0, False), ((4, 5, 3), "PNP", "UDU", 2, 0, False)]
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["fp64", "refinement", "gcr"])
+@pytest.mark.parametrize("case", OUTER, ids=str)
+def test_residual_norms_match_oracle(case, precision):
+    """The norm of the guess, the norm of every cycle and what the cycle left, against the oracle's
+    computeError of the same iterate.  Both round r = f - L x to some 10 units of |L| |x| per node, which
+    bounds the difference of the relative norms.  A GCR step is the best one along its directions, so
+    that its first is no worse than the refinement step up to the rounding of L e in FP32."""
+    from saras_amd import _lib
+    lens = []
+    for count in (1, 2, 3):
+        pb = _problem(*case, vc_count=count, rel_tol=1e-30)
+        f, x = pb.random_rhs(5), 1e-3 * pb.random_rhs(6)
+        o = pb.oracle()
+        o.level = 0
+        fp = o.project_rhs(f.copy())
+        size = 0.0
+        for d in range(3):
+            ax, h = po.grid_axis(pb.n[d], pb.L[d], pb.gtype[d], pb.beta[d]), 1.0 / (pb.n[d] - 1)
+            size += 4 * np.max(np.abs(ax["xix2"])) / h**2 + np.max(np.abs(ax["xixx"])) / h
+
+        def check(got, p):
+            o.array(po.P, 0)[...] = p
+            o.impose_bc()
+            o.array(po.R, 0)[...] = fp
+            want = o.compute_error(2)
+            tol = 16 * 2.2e-16 * size * np.max(np.abs(p)) * np.sqrt(np.prod(pb.n)) / np.linalg.norm(fp[1:-1, 1:-1, 1:-1])
+            assert abs(got - want) <= tol + 1e-12 * want, (count, got, want, tol)
+
+        g = pb.gpu(precision=precision, coarse_direct=1 if np.prod([k >> (pb.depth) for k in pb.n]) < 100 else 0)
+        bufs = [_lib.DeviceArray(pb.shape) for _ in range(2)]
+        bufs[0].upload(x)
+        bufs[1].upload(f)
+        check(g.residual_device(bufs[0].ptr, bufs[1].ptr), x)
+        p = x.copy()
+        st = g.mgSolve(p, f)
+        if precision:
+            check(st.residual0, x)
+        hist = g.history()
+        assert len(hist) == count
+        check(hist[-1], p)
+        lens.append(hist)
+        g.close()
+    assert lens[0][0] == lens[1][0] == lens[2][0] and lens[1][1] == lens[2][1]   # the same steps each time
+    if precision == 2:
+        g = pb.gpu(precision=1, coarse_direct=1 if np.prod([k >> (pb.depth) for k in pb.n]) < 100 else 0)
+        g.mgSolve(x.copy(), f)
+        hist = lens[2]
+        assert hist[0] <= g.history()[0] * (1 + 1e-5)
+        assert np.all(hist[1:] <= hist[:-1] * (1 + 1e-5)), hist
+        g.close()
