@@ -3,10 +3,9 @@
 // gradient (vfield.cc:104-320, sfield.cc:86-171), the boundary classes with syncData, and the
 // implicit Jacobi solves of hydro_d3 / scalar_d3.
 //
-// Kernels here work on one field at a time over the reference's padded natural layout (k
-// fastest), one thread per entry, k across the lanes of a wavefront so that every stencil load is
-// a coalesced row; the fused time step (ts_kernels.hip) keeps its own copies of the same
-// expressions.  All are HBM-bound (well under one FP64 flop per byte).
+// Kernels here march along x over the reference's padded natural layout (k fastest, columns.h), all
+// components of a field operator in one launch, so that computeNLin reads each V_d once for the three
+// components that it advects.  All are HBM-bound (well under one FP64 flop per byte).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -18,7 +17,7 @@
 #include "../../include/saras_field.h"
 #include "../../include/saras_mg.h"
 #include "ghost_waves.h"
-#include "xcd.h"
+#include "columns.h"
 #include "mg_state.h"
 #include "ts_kernels.h"
 
@@ -55,175 +54,408 @@ namespace {
 
 __host__ __device__ inline long fsz(const FShape &f) { return (long)(f.n[0] + 2) * (f.n[1] + 2) * (f.n[2] + 2); }
 
-__device__ inline long fix(const FShape &f, int i, int j, int k) {
-    return ((long)(i + 1) * (f.n[1] + 2) + (j + 1)) * (f.n[2] + 2) + (k + 1);
+// entry t of a padded plane with rows of n entries -> (j, k), counted from -1
+__device__ inline void in_plane(unsigned t, int n, int &j, int &k) {
+    const unsigned r = t / (unsigned)n;
+    j = (int)r - 1;
+    k = (int)(t - r * (unsigned)n) - 1;
 }
-__device__ inline double mt(const Metrics &M, int d, int node, int q, int i) { return M.m[d][node ? 0 : 1][q][i + 1]; }
-
-// padded entry t -> logical (i, j, k), each in -1..n (32-bit: a padded array has < 2^32 entries)
-__device__ inline void unflat(const FShape &f, unsigned t, int &i, int &j, int &k) {
-    unsigned n2 = (unsigned)f.n[2] + 2u, n1 = (unsigned)f.n[1] + 2u;
-    unsigned r = t / n2;
-    k = (int)(t - r * n2) - 1;
-    unsigned q = r / n1;
-    j = (int)(r - q * n1) - 1;
-    i = (int)q - 1;
-}
-// core entry t -> logical (i, j, k), each in 0..n-1
-__device__ inline void unflat_core(const FShape &f, unsigned t, int &i, int &j, int &k) {
-    unsigned n2 = (unsigned)f.n[2], n1 = (unsigned)f.n[1];
-    unsigned r = t / n2;
-    k = (int)(t - r * n2);
-    unsigned q = r / n1;
-    j = (int)(r - q * n1);
-    i = (int)q;
-}
-// the thread's entry: logical workgroups in XCD order (each XCD a contiguous range of rows)
-__device__ inline unsigned entry() { return xcd_block() * 256u + threadIdx.x; }
+__device__ inline long plane_of(const FShape &f) { return (long)(f.n[1] + 2) * (f.n[2] + 2); }
 
 // calcDerivative1 / 2 along d over the whole padded array: the core range along d gets the
 // derivative, the two pad layers along d get 0
-__global__ void __launch_bounds__(256) k_fd_deriv(FShape f, Metrics M, const double *__restrict__ F,
-                                                  double *__restrict__ out, int order, int d, double ih, double half) {
-    const unsigned t = entry();
-    if ((long)t >= fsz(f)) return;
-    int idx[3];
-    unflat(f, t, idx[0], idx[1], idx[2]);
-    int r = idx[d];
-    if (r < 0 || r >= f.n[d]) {
-        out[t] = 0.0;
-        return;
-    }
-    long st = d == 0 ? (long)(f.n[1] + 2) * (f.n[2] + 2) : d == 1 ? (long)(f.n[2] + 2) : 1;
-    double fp = F[t + st], fm = F[t - st];
-    if (order == 1) {
-        double v = (fp - fm) / 2.0;
-        v *= ih;
-        out[t] = mt(M, d, f.s[d], 1, r) * v;
-    } else {
-        double ih2 = ih * ih;
-        double tmp = (fp - fm) / 2.0 * ih;
-        double sec = (fp - 2.0 * F[t] + fm) * ih2;
-        out[t] = mt(M, d, f.s[d], 2, r) * tmp + half * mt(M, d, f.s[d], 3, r) * sec;
-    }
-}
-
-// computeDiff of one field: H(core) += d2xx, += d2yy, += d2zz in that order
-__global__ void __launch_bounds__(256) k_fd_diff(FShape f, Metrics M, const double *__restrict__ F,
-                                                 double *__restrict__ H, double ih0, double ih1, double ih2,
-                                                 double half) {
-    const unsigned t = entry();
-    if ((long)t >= (long)f.n[0] * f.n[1] * f.n[2]) return;
-    int idx[3];
-    unflat_core(f, t, idx[0], idx[1], idx[2]);
-    long q = fix(f, idx[0], idx[1], idx[2]);
-    long st[3] = {(long)(f.n[1] + 2) * (f.n[2] + 2), (long)(f.n[2] + 2), 1};
-    double ihh[3] = {ih0, ih1, ih2};
-    double acc = H[q];
-    double f0 = F[q];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        double ih = ihh[d];
-        double ih2 = ih * ih;
-        double fp = F[q + st[d]], fm = F[q - st[d]];
-        double tmp = (fp - fm) / 2.0 * ih;
-        double sec = (fp - 2.0 * f0 + fm) * ih2;
-        double dd = mt(M, d, f.s[d], 2, idx[d]) * tmp + half * mt(M, d, f.s[d], 3, idx[d]) * sec;
-        acc += dd;
-    }
-    H[q] = acc;
-}
-
-// computeNLin of one field at location loc (0 node, 1..3 face of component loc - 1), advected by
-// (Vx, Vy, Vz): for d = x, y, z, H(core) -= (sum of the slices of V_d) d_d F / nslices.  Slices of
-// V_d onto component c's location: the core index alone when d == c, else {core, d-1, c+1,
-// (c+1, d-1)}; onto the nodes: {core, d-1} (field.cc:309-575)
-__global__ void __launch_bounds__(256) k_fd_nlin(int loc, FShape f, FShape fx, FShape fy, FShape fz, Metrics M,
-                                                 const double *__restrict__ F, const double *__restrict__ Vx,
-                                                 const double *__restrict__ Vy, const double *__restrict__ Vz,
-                                                 double *__restrict__ H, double ih0, double ih1, double ih2) {
-    const unsigned t = entry();
-    if ((long)t >= (long)f.n[0] * f.n[1] * f.n[2]) return;
-    int i, j, k;
-    unflat_core(f, t, i, j, k);
-    int idx[3] = {i, j, k};
-    long q = fix(f, i, j, k);
-    long st[3] = {(long)(f.n[1] + 2) * (f.n[2] + 2), (long)(f.n[2] + 2), 1};
-    double ihh[3] = {ih0, ih1, ih2};
-    const double *V[3] = {Vx, Vy, Vz};
-    const FShape *FS[3] = {&fx, &fy, &fz};
-    const int c = loc - 1;
-    double acc = H[q];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        const FShape &fd = *FS[d];
-        const double *Vd = V[d];
-        double inter = 0.0;
-        int ns;
-        if (loc == 0) {
-            int o[3] = {i, j, k};
-            o[d] -= 1;
-            inter += Vd[fix(fd, i, j, k)];
-            inter += Vd[fix(fd, o[0], o[1], o[2])];
-            ns = 2;
-        } else if (d == c) {
-            inter += Vd[fix(fd, i, j, k)];
-            ns = 1;
-        } else {
-            int o1[3] = {i, j, k}, o2[3] = {i, j, k}, o3[3] = {i, j, k};
-            o1[d] -= 1;
-            o2[c] += 1;
-            o3[c] += 1;
-            o3[d] -= 1;
-            inter += Vd[fix(fd, i, j, k)];
-            inter += Vd[fix(fd, o1[0], o1[1], o1[2])];
-            inter += Vd[fix(fd, o2[0], o2[1], o2[2])];
-            inter += Vd[fix(fd, o3[0], o3[1], o3[2])];
-            ns = 4;
+template <int ORDER, bool ALONGX>
+__global__ void __launch_bounds__(kColThreads) k_fd_deriv(ColGeo G, FShape f, Metrics M, const double *__restrict__ F,
+                                                          double *__restrict__ out, int d, double ih, double half) {
+    const Col C = column(G);
+    const long ps = plane_of(f);
+    // metrics of the planes (along x) or of this column
+    __shared__ double lx[2][kColPlanes];
+    if (ALONGX) {
+        for (int q = (int)threadIdx.x; q < C.i1 - C.i0; q += kColThreads) {
+            const int r = max(0, min(C.i0 - 1 + q, f.n[0] - 1));
+            lx[0][q] = ORDER == 1 ? met1(M, 0, f.s[0], r, ih) : met2(M, 0, f.s[0], r, ih);
+            lx[1][q] = ORDER == 1 ? 0.0 : met3(M, 0, f.s[0], r, ih, half);
         }
-        double ih = ihh[d];
-        double dv = (F[q + st[d]] - F[q - st[d]]) / 2.0;
-        dv *= ih;
-        double deriv = mt(M, d, f.s[d], 1, idx[d]) * dv;
-        // / ns with ns = 1, 2 or 4: the same as * (1 / ns), exactly
-        acc -= inter * deriv * (ns == 1 ? 1.0 : ns == 2 ? 0.5 : 0.25);
+        __syncthreads();
     }
-    H[q] = acc;
+    if ((long)C.t >= ps) return;
+    int j, k;
+    in_plane(C.t, f.n[2] + 2, j, k);
+    const int r = d == 1 ? j : k, n = d == 1 ? f.n[1] : f.n[2], sd = d == 1 ? f.s[1] : f.s[2];
+    const bool column_in = ALONGX || (r >= 0 && r < n);
+    // a pad entry along d takes part in the loads of the core entry next to it
+    const int rc = max(0, min(r, n - 1)), st2 = d == 1 ? f.n[2] + 2 : 1;
+    const unsigned o = C.t * 8u, os = ALONGX ? o : (unsigned)((int)C.t + (rc - r) * st2) * 8u;
+    const long st = ALONGX ? ps : st2;
+    double a2 = 0.0, a3 = 0.0;
+    if (!ALONGX) {
+        a2 = d == 1 ? met(M, 1, sd, ORDER, rc) : met(M, 2, sd, ORDER, rc);
+        a2 *= 0.5 * ih;
+        if (ORDER == 2) a3 = half * (d == 1 ? met(M, 1, sd, 3, rc) : met(M, 2, sd, 3, rc)) * (ih * ih);
+    }
+    for (int p0 = C.i0; p0 < C.i1; p0 += kColAhead) {
+        double fp[kColAhead], fm[kColAhead], fc[kColAhead];
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            const int p = ALONGX ? max(1, min(p0 + u, f.n[0])) : min(p0 + u, C.i1 - 1);
+            const double *const c = F + p * ps;
+            fp[u] = ldd(c + st, os);
+            fm[u] = ldd(c - st, os);
+            if (ORDER == 2) fc[u] = ldd(c, os);
+        }
+        loaded(fp);
+        loaded(fm);
+        if (ORDER == 2) loaded(fc);
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            const int p = p0 + u;
+            if (p >= C.i1) break;
+            const bool in = ALONGX ? p >= 1 && p <= f.n[0] : column_in;
+            const double b2 = ALONGX ? lx[0][p - C.i0] : a2, b3 = ALONGX ? lx[1][p - C.i0] : a3;
+            const double v = ORDER == 1 ? b2 * (fp[u] - fm[u]) : b2 * (fp[u] - fm[u]) + b3 * (fp[u] - 2.0 * fc[u] + fm[u]);
+            std_(out + p * ps, o, in ? v : 0.0);
+        }
+    }
 }
 
-// gradient component c on its core: G = xi_c(face) (F(+1) - F) / h_c
-__global__ void __launch_bounds__(256) k_fd_gradient(int c, FShape fc, FShape fp, Metrics M,
-                                                     const double *__restrict__ F, double *__restrict__ G, double hc) {
-    const unsigned t = entry();
-    if ((long)t >= (long)fc.n[0] * fc.n[1] * fc.n[2]) return;
-    int i, j, k;
-    unflat_core(fc, t, i, j, k);
-    int idx[3] = {i, j, k};
-    long sp = c == 0 ? (long)(fp.n[1] + 2) * (fp.n[2] + 2) : c == 1 ? (long)(fp.n[2] + 2) : 1;
-    long pq = fix(fp, i, j, k);
-    G[fix(fc, i, j, k)] = mt(M, c, 0, 1, idx[c]) * (F[pq + sp] - F[pq]) / hc;
+// up to three fields with their own shapes, one per grid row
+struct Fields {
+    const double *F[3];
+    double *H[3];
+    FShape f[3];
+};
+
+// computeDiff: H(core) += d2xx, += d2yy, += d2zz in that order.  At 257^3 the field and H are read and
+// H is written, 0.41 GB: 163 -> 116 us.
+__global__ void __launch_bounds__(kColThreads) k_fd_diff(ColGeo G, Fields A, Metrics M, ColMet W) {
+    const FShape f = A.f[blockIdx.y];
+    const Col C = column(G);
+    __shared__ double lx[2][kColPlanes];
+    for (int q = (int)threadIdx.x; q < C.i1 - C.i0; q += kColThreads) {
+        const int i = min(C.i0 + q, f.n[0] - 1);
+        lx[0][q] = met2(M, 0, f.s[0], i, W.ih[0]);
+        lx[1][q] = met3(M, 0, f.s[0], i, W.ih[0], W.half);
+    }
+    __syncthreads();
+    int j, k;
+    const int row = f.n[2] + 2, i1 = min(C.i1, f.n[0]);
+    in_plane(C.t, row, j, k);
+    if (j < 0 || k < 0 || j >= f.n[1] || k >= f.n[2] || C.i0 >= i1) return;
+    const long ps = plane_of(f);
+    const unsigned o = C.t * 8u;
+    const double y2 = met2(M, 1, f.s[1], j, W.ih[1]), y3 = met3(M, 1, f.s[1], j, W.ih[1], W.half);
+    const double z2 = met2(M, 2, f.s[2], k, W.ih[2]), z3 = met3(M, 2, f.s[2], k, W.ih[2], W.half);
+    const double *F = A.F[blockIdx.y] + (C.i0 + 1) * ps;
+    double *H = A.H[blockIdx.y] + (C.i0 + 1) * ps;
+    Cross u;
+    u.xm = ldd(F - ps, o);
+    u.c = ldd(F, o);
+    for (int i = C.i0; i < i1; i += kColAhead, F += kColAhead * ps, H += kColAhead * ps) {
+        double xp[kColAhead], h[kColAhead];
+#pragma unroll
+        for (int w = 0; w < kColAhead; w++) {
+            const long q = min(w, i1 - 1 - i) * ps;
+            xp[w] = ldd(F + q + ps, o);
+            h[w] = ldd(H + q, o);
+        }
+        loaded(xp);
+        loaded(h);
+#pragma unroll
+        for (int w = 0; w < kColAhead; w++) {
+            if (i + w >= i1) break;
+            const double *const f = F + w * ps;
+            u.xp = xp[w];
+            u.yp = ldd(f + row, o);
+            u.ym = ldd(f - row, o);
+            u.zp = ldd(f + 1, o);
+            u.zm = ldd(f - 1, o);
+            const int q = i + w - C.i0;
+            std_(H + w * ps, o, diffuse(h[w], u, lx[0][q], lx[1][q], y2, y3, z2, z3));
+            u.xm = u.c;
+            u.c = u.xp;
+        }
+    }
+}
+
+// computeNLin of a vector field U advected by V: for d = x, y, z, H(core) -= (sum of the slices of V_d)
+// d_d U / nslices.  Slices of V_d onto component c's location: the core index alone when d == c, else
+// {core, d-1, c+1, (c+1, d-1)} (field.cc:309-575).  SELF: U is V, whose loads then serve both.  which: the
+// components to do, as bits.  At 257^3 three fields and three H are read and H is written, 1.22 GB: 560 ->
+// 350 us for the three components.
+template <bool SELF>
+__global__ void __launch_bounds__(kColThreads) k_fd_nlin(ColGeo G, VelGeo S, Metrics M, const double *__restrict__ Ux,
+                                                 const double *__restrict__ Uy, const double *__restrict__ Uz,
+                                                 const double *__restrict__ Vx, const double *__restrict__ Vy,
+                                                 const double *__restrict__ Vz, double *__restrict__ Hx,
+                                                 double *__restrict__ Hy, double *__restrict__ Hz, ColMet W, int which) {
+    const Col C = column(G);
+    __shared__ double lx[2][kColPlanes];   // x metrics of faces (one slice) and a quarter of those of nodes
+    for (int q = (int)threadIdx.x; q < C.i1 - C.i0; q += kColThreads) {
+        lx[0][q] = met1(M, 0, 0, min(C.i0 + q, S.N[0] - 2), W.ih[0]);
+        lx[1][q] = 0.25 * met1(M, 0, 1, C.i0 + q, W.ih[0]);
+    }
+    __syncthreads();
+    int j, k;
+    const int row = S.N[2] + 2, rz = S.N[2] + 1;
+    in_plane(C.t, row, j, k);
+    if (j < 0 || k < 0 || j >= S.N[1] || k >= S.N[2]) return;
+    const long sx = S.sx(), sy = S.sy(), sz = S.sz();
+    const unsigned o = C.t * 8u, oz = (unsigned)((j + 1) * rz + k + 1) * 8u;
+    const bool cy = (which & 2) && j < S.N[1] - 1, cz = (which & 4) && k < S.N[2] - 1;
+    const double yf = met1(M, 1, 0, min(j, S.N[1] - 2), W.ih[1]), yn = 0.25 * met1(M, 1, 1, j, W.ih[1]);
+    const double zf = met1(M, 2, 0, min(k, S.N[2] - 2), W.ih[2]), zn = 0.25 * met1(M, 2, 1, k, W.ih[2]);
+    const long i0 = C.i0 + 1;
+    Vx += i0 * sx;
+    Vy += i0 * sy;
+    Vz += i0 * sz;
+    Ux += i0 * sx;
+    Uy += i0 * sy;
+    Uz += i0 * sz;
+    Hx += i0 * sx;
+    Hy += i0 * sy;
+    Hz += i0 * sz;
+    Vels v;
+    vels_begin(v, Vx, Vy, Vz, S, o, oz, SELF);
+    Cross ux, uy, uz;
+    if (!SELF) {
+        ux.xm = ldd(Ux - sx, o);
+        ux.c = ldd(Ux, o);
+        uy.xm = ldd(Uy - sy, o);
+        uy.c = ldd(Uy, o);
+        uz.xm = ldd(Uz - sz, oz);
+        uz.c = ldd(Uz, oz);
+    }
+    for (int i = C.i0; i < C.i1; ++i) {
+        const bool cx = i < S.N[0] - 1;
+        vels_load(v, Vx, Vy, Vz, S, o, oz, SELF, !cx);
+        if (SELF) {
+            ux = cross_x(v);
+            uy = cross_y(v);
+            uz = cross_z(v);
+        } else {
+            ux.xp = ldd(cx ? Ux + sx : Ux, o);
+            ux.yp = ldd(Ux + row, o);
+            ux.ym = ldd(Ux - row, o);
+            ux.zp = ldd(Ux + 1, o);
+            ux.zm = ldd(Ux - 1, o);
+            uy.xp = ldd(Uy + sy, o);
+            uy.yp = ldd(Uy + row, o);
+            uy.ym = ldd(Uy - row, o);
+            uy.zp = ldd(Uy + 1, o);
+            uy.zm = ldd(Uy - 1, o);
+            uz.xp = ldd(Uz + sz, oz);
+            uz.yp = ldd(Uz + rz, oz);
+            uz.ym = ldd(Uz - rz, oz);
+            uz.zp = ldd(Uz + 1, oz);
+            uz.zm = ldd(Uz - 1, oz);
+        }
+        const double hx = ldd(Hx, o), hy = ldd(Hy, o), hz = ldd(Hz, oz);
+        const double xf = lx[0][i - C.i0], xn = lx[1][i - C.i0];
+        if (cx && (which & 1)) std_(Hx, o, advect<0>(hx, v, ux, xf, yn, zn));
+        if (cy) std_(Hy, o, advect<1>(hy, v, uy, xn, yf, zn));
+        if (cz) std_(Hz, oz, advect<2>(hz, v, uz, xn, yn, zf));
+        vels_next(v);
+        if (!SELF) {
+            ux.xm = ux.c;
+            ux.c = ux.xp;
+            uy.xm = uy.c;
+            uy.c = uy.xp;
+            uz.xm = uz.c;
+            uz.c = uz.xp;
+        }
+        Vx += sx;
+        Vy += sy;
+        Vz += sz;
+        Ux += sx;
+        Uy += sy;
+        Uz += sz;
+        Hx += sx;
+        Hy += sy;
+        Hz += sz;
+    }
+}
+
+// computeNLin of a node field: the slices of V_d are {core, d-1}
+__global__ void __launch_bounds__(kColThreads) k_fd_nlin_node(ColGeo G, VelGeo S, Metrics M, const double *__restrict__ F,
+                                                      const double *__restrict__ Vx, const double *__restrict__ Vy,
+                                                      const double *__restrict__ Vz, double *__restrict__ H, ColMet W) {
+    const Col C = column(G);
+    __shared__ double lx[kColPlanes];
+    for (int q = (int)threadIdx.x; q < C.i1 - C.i0; q += kColThreads) lx[q] = 0.5 * met1(M, 0, 1, C.i0 + q, W.ih[0]);
+    __syncthreads();
+    int j, k;
+    const int row = S.N[2] + 2, rz = S.N[2] + 1;
+    in_plane(C.t, row, j, k);
+    if (j < 0 || k < 0 || j >= S.N[1] || k >= S.N[2]) return;
+    const long sx = S.sx(), sy = S.sy(), sz = S.sz(), i0 = C.i0 + 1;
+    const unsigned o = C.t * 8u, oz = (unsigned)((j + 1) * rz + k + 1) * 8u;
+    const double ay = 0.5 * met1(M, 1, 1, j, W.ih[1]), az = 0.5 * met1(M, 2, 1, k, W.ih[2]);
+    F += i0 * sx;
+    H += i0 * sx;
+    Vx += i0 * sx;
+    Vy += i0 * sy;
+    Vz += i0 * sz;
+    double fm = ldd(F - sx, o), f0 = ldd(F, o), xm = ldd(Vx - sx, o);
+    for (int i = C.i0; i < C.i1; i += kColAhead) {
+        double fp[kColAhead], x[kColAhead], acc[kColAhead], y[kColAhead], ym[kColAhead], z[kColAhead], zm[kColAhead];
+        double fy[kColAhead], fym[kColAhead], fz[kColAhead], fzm[kColAhead];
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            const long q = min(u, C.i1 - 1 - i);
+            const double *const f = F + q * sx, *const Y = Vy + q * sy, *const Z = Vz + q * sz;
+            fp[u] = ldd(f + sx, o);
+            x[u] = ldd(Vx + q * sx, o);
+            acc[u] = ldd(H + q * sx, o);
+            y[u] = ldd(Y, o);
+            ym[u] = ldd(Y - row, o);
+            z[u] = ldd(Z, oz);
+            zm[u] = ldd(Z - 1, oz);
+            fy[u] = ldd(f + row, o);
+            fym[u] = ldd(f - row, o);
+            fz[u] = ldd(f + 1, o);
+            fzm[u] = ldd(f - 1, o);
+        }
+        loaded(fp);
+        loaded(x);
+        loaded(acc);
+        loaded(y);
+        loaded(z);
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            if (i + u >= C.i1) break;
+            acc[u] -= (x[u] + xm) * (lx[i + u - C.i0] * (fp[u] - fm));
+            acc[u] -= (y[u] + ym[u]) * (ay * (fy[u] - fym[u]));
+            acc[u] -= (z[u] + zm[u]) * (az * (fz[u] - fzm[u]));
+            std_(H + u * sx, o, acc[u]);
+            fm = f0;
+            f0 = fp[u];
+            xm = x[u];
+        }
+        F += kColAhead * sx;
+        H += kColAhead * sx;
+        Vx += kColAhead * sx;
+        Vy += kColAhead * sy;
+        Vz += kColAhead * sz;
+    }
+}
+
+// gradient on the cores of its components: G_c = xi_c(face) (F(+1) - F) / h_c; which: the components to
+// do, as bits.  One launch reads F once: 213 -> 134 us at 257^3.
+__global__ void __launch_bounds__(kColThreads) k_fd_gradient(ColGeo G, VelGeo S, Metrics M, const double *__restrict__ F,
+                                                     double *__restrict__ Gx, double *__restrict__ Gy,
+                                                     double *__restrict__ Gz, ColMet W, int which) {
+    const Col C = column(G);
+    __shared__ double lx[kColPlanes];
+    for (int q = (int)threadIdx.x; q < C.i1 - C.i0; q += kColThreads)
+        lx[q] = met(M, 0, 0, 1, min(C.i0 + q, S.N[0] - 2)) * W.ih[0];
+    __syncthreads();
+    int j, k;
+    const int row = S.N[2] + 2, rz = S.N[2] + 1;
+    in_plane(C.t, row, j, k);
+    if (j < 0 || k < 0 || j >= S.N[1] || k >= S.N[2]) return;
+    const long sx = S.sx(), sy = S.sy(), sz = S.sz(), i0 = C.i0 + 1;
+    const unsigned o = C.t * 8u, oz = (unsigned)((j + 1) * rz + k + 1) * 8u;
+    const bool cy = (which & 2) && j < S.N[1] - 1, cz = (which & 4) && k < S.N[2] - 1;
+    const double ay = met(M, 1, 0, 1, min(j, S.N[1] - 2)) * W.ih[1], az = met(M, 2, 0, 1, min(k, S.N[2] - 2)) * W.ih[2];
+    F += i0 * sx;
+    Gx += i0 * sx;
+    Gy += i0 * sy;
+    Gz += i0 * sz;
+    double f0 = ldd(F, o);
+    for (int i = C.i0; i < C.i1; i += kColAhead) {
+        double fp[kColAhead], fy[kColAhead], fz[kColAhead];
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            const double *const f = F + min(u, C.i1 - 1 - i) * sx;
+            fp[u] = ldd(f + sx, o);
+            fy[u] = ldd(f + row, o);
+            fz[u] = ldd(f + 1, o);
+        }
+        loaded(fp);
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            if (i + u >= C.i1) break;
+            if (i + u < S.N[0] - 1 && (which & 1)) std_(Gx + u * sx, o, lx[i + u - C.i0] * (fp[u] - f0));
+            if (cy) std_(Gy + u * sy, o, ay * (fy[u] - f0));
+            if (cz) std_(Gz + u * sz, oz, az * (fz[u] - f0));
+            f0 = fp[u];
+        }
+        F += kColAhead * sx;
+        Gx += kColAhead * sx;
+        Gy += kColAhead * sy;
+        Gz += kColAhead * sz;
+    }
 }
 
 // divergence over the whole padded node array: core from the face differences, pads 0
-__global__ void __launch_bounds__(256) k_fd_divergence(FShape fp, FShape fx, FShape fy, FShape fz, Metrics M,
-                                                       const double *__restrict__ Vx, const double *__restrict__ Vy,
-                                                       const double *__restrict__ Vz, double *__restrict__ out,
-                                                       double h0, double h1, double h2) {
-    const unsigned t = entry();
-    if ((long)t >= fsz(fp)) return;
-    int i, j, k;
-    unflat(fp, t, i, j, k);
-    if (i < 0 || j < 0 || k < 0 || i >= fp.n[0] || j >= fp.n[1] || k >= fp.n[2]) {
-        out[t] = 0.0;
-        return;
+__global__ void __launch_bounds__(kColThreads) k_fd_divergence(ColGeo G, VelGeo S, Metrics M, const double *__restrict__ Vx,
+                                                       const double *__restrict__ Vy, const double *__restrict__ Vz,
+                                                       double *__restrict__ out, ColMet W) {
+    const Col C = column(G);   // padded planes
+    __shared__ double lx[kColPlanes];
+    for (int q = (int)threadIdx.x; q < C.i1 - C.i0; q += kColThreads)
+        lx[q] = met(M, 0, 1, 1, max(0, min(C.i0 - 1 + q, S.N[0] - 1))) * W.ih[0];
+    __syncthreads();
+    const long sx = S.sx(), sy = S.sy(), sz = S.sz();
+    if ((long)C.t >= sx) return;
+    int j, k;
+    const int row = S.N[2] + 2, rz = S.N[2] + 1;
+    in_plane(C.t, row, j, k);
+    const bool in = j >= 0 && k >= 0 && j < S.N[1] && k < S.N[2];
+    const unsigned po = C.t * 8u;
+    // a pad entry takes part in the loads of the core entry next to it
+    j = max(0, min(j, S.N[1] - 1));
+    k = max(0, min(k, S.N[2] - 1));
+    const unsigned o = (unsigned)((j + 1) * row + k + 1) * 8u, oz = (unsigned)((j + 1) * rz + k + 1) * 8u;
+    const double ay = met(M, 1, 1, 1, j) * W.ih[1], az = met(M, 2, 1, 1, k) * W.ih[2];
+    double xm = ldd(Vx + max(C.i0 - 1, 0) * sx, o);
+    for (int p0 = C.i0; p0 < C.i1; p0 += kColAhead) {
+        double x[kColAhead], y[kColAhead], ym[kColAhead], z[kColAhead], zm[kColAhead];
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            const long p = min(p0 + u, S.N[0]);   // the last plane of Vx
+            x[u] = ldd(Vx + p * sx, o);
+            y[u] = ldd(Vy + p * sy, o);
+            ym[u] = ldd(Vy + p * sy - row, o);
+            z[u] = ldd(Vz + p * sz, oz);
+            zm[u] = ldd(Vz + p * sz - 1, oz);
+        }
+        loaded(x);
+        loaded(y);
+        loaded(z);
+#pragma unroll
+        for (int u = 0; u < kColAhead; u++) {
+            const int p = p0 + u;
+            if (p >= C.i1) break;
+            const double a = lx[p - C.i0] * (x[u] - xm), b = ay * (y[u] - ym[u]);
+            const double v = a + b + az * (z[u] - zm[u]);
+            std_(out + p * sx, po, in && p >= 1 && p <= S.N[0] ? v : 0.0);
+            xm = x[u];
+        }
     }
-    double a = mt(M, 0, 1, 1, i) * (Vx[fix(fx, i, j, k)] - Vx[fix(fx, i - 1, j, k)]) / h0;
-    double b = mt(M, 1, 1, 1, j) * (Vy[fix(fy, i, j, k)] - Vy[fix(fy, i, j - 1, k)]) / h1;
-    double cz = mt(M, 2, 1, 1, k) * (Vz[fix(fz, i, j, k)] - Vz[fix(fz, i, j, k - 1)]) / h2;
-    out[t] = a + b + cz;
 }
 
-inline unsigned nblocks(long n) { return (unsigned)((n + 255) / 256); }
+ColMet col_met(const sr_fgrid *g) {
+    // the inverse grid spacings are formed on the host, like derivative's ihx, ihy, ihz (derivative.cc:66-68)
+    return ColMet{{1.0 / g->h[0], 1.0 / g->h[1], 1.0 / g->h[2]}, g->half};
+}
+VelGeo vel_geo(const sr_fgrid *g) { return VelGeo{{g->N[0], g->N[1], g->N[2]}}; }
+// Whether the components' outputs H can be written by one launch that reads the inputs U: no output shares
+// memory with another one or with another component's input.  A caller may let them (the components are
+// then done in order, as if one by one).
+bool one_launch(const sr_fgrid *g, double *const H[3], const double *const *U) {
+    auto apart = [&](const double *a, int la, const double *b, int lb) {
+        return a + fsz(g->shape[la]) <= b || b + fsz(g->shape[lb]) <= a;
+    };
+    for (int c = 0; c < 3; c++)
+        for (int e = 0; e < 3; e++)
+            if (e != c && (!apart(H[c], SR_LOC_VX + c, H[e], SR_LOC_VX + e) ||
+                           (U && !apart(H[c], SR_LOC_VX + c, U[e], SR_LOC_VX + e))))
+                return false;
+    return true;
+}
+ColGeo node_geo(const sr_fgrid *g, int planes) { return col_geo(vel_geo(g).sx(), planes); }
 
 int check_loc(const sr_fgrid *g, int loc) {
     if (!g) return set_err(SR_ERR_ARG, "null handle");
@@ -385,9 +617,11 @@ static int deriv(sr_fgrid *g, int loc, int order, int dim, const double *F, doub
     if (!F || !out) return set_err(SR_ERR_ARG, "null array");
     if ((const double *)out == F) return set_err(SR_ERR_ARG, "out must not alias F");
     const FShape &f = g->shape[loc];
-    // the inverse grid spacings are formed on the host, like derivative's ihx, ihy, ihz (derivative.cc:66-68)
-    hipLaunchKernelGGL(k_fd_deriv, dim3(nblocks(fsz(f))), dim3(256), 0, g->s, f, g->M, F, out, order, dim,
-                       1.0 / g->h[dim], g->half);
+    const ColGeo G = col_geo((long)(f.n[1] + 2) * (f.n[2] + 2), f.n[0] + 2);
+    auto *const k = order == 1 ? (dim == 0 ? k_fd_deriv<1, true> : k_fd_deriv<1, false>)
+                               : (dim == 0 ? k_fd_deriv<2, true> : k_fd_deriv<2, false>);
+    hipLaunchKernelGGL(k, dim3(col_blocks(G)), dim3(kColThreads), 0, g->s, G, f, g->M, F, out, dim, 1.0 / g->h[dim],
+                       g->half);
     HIPCHK(hipGetLastError());
     return SR_OK;
 }
@@ -399,13 +633,18 @@ extern "C" int sr_deriv2(sr_fgrid *g, int loc, int dim, const double *F, double 
     return deriv(g, loc, 2, dim, F, out);
 }
 
-static int diff(sr_fgrid *g, int loc, const double *F, double *H) {
-    if (!F || !H) return set_err(SR_ERR_ARG, "null array");
-    if ((const double *)H == F) return set_err(SR_ERR_ARG, "H must not alias the field");
-    const FShape &f = g->shape[loc];
-    long n = (long)f.n[0] * f.n[1] * f.n[2];
-    hipLaunchKernelGGL(k_fd_diff, dim3(nblocks(n)), dim3(256), 0, g->s, f, g->M, F, H, 1.0 / g->h[0], 1.0 / g->h[1],
-                       1.0 / g->h[2], g->half);
+// computeDiff of n fields at locations loc, loc + 1, ...
+static int diff(sr_fgrid *g, int loc, int n, const double *const *F, double *const *H) {
+    Fields A{};
+    for (int c = 0; c < n; c++) {
+        if (!F[c] || !H[c]) return set_err(SR_ERR_ARG, "null array");
+        if ((const double *)H[c] == F[c]) return set_err(SR_ERR_ARG, "H must not alias the field");
+        A.F[c] = F[c];
+        A.H[c] = H[c];
+        A.f[c] = g->shape[loc + c];
+    }
+    const ColGeo G = node_geo(g, g->N[0]);
+    hipLaunchKernelGGL(k_fd_diff, dim3(col_blocks(G), n), dim3(kColThreads), 0, g->s, G, A, g->M, col_met(g));
     HIPCHK(hipGetLastError());
     return SR_OK;
 }
@@ -413,35 +652,23 @@ static int diff(sr_fgrid *g, int loc, const double *F, double *H) {
 extern "C" int sr_vf_diff(sr_fgrid *g, const double *Vx, const double *Vy, const double *Vz, double *Hx, double *Hy,
                           double *Hz) {
     if (!g) return set_err(SR_ERR_ARG, "null handle");
-    RETCHK(diff(g, SR_LOC_VX, Vx, Hx));
-    RETCHK(diff(g, SR_LOC_VY, Vy, Hy));
-    RETCHK(diff(g, SR_LOC_VZ, Vz, Hz));
+    const double *F[3] = {Vx, Vy, Vz};
+    double *H[3] = {Hx, Hy, Hz};
+    if (one_launch(g, H, F)) return diff(g, SR_LOC_VX, 3, F, H);
+    for (int c = 0; c < 3; c++) RETCHK(diff(g, SR_LOC_VX + c, 1, F + c, H + c));
     return SR_OK;
 }
 
 extern "C" int sr_sf_diff(sr_fgrid *g, const double *F, double *H) {
     if (!g) return set_err(SR_ERR_ARG, "null handle");
-    return diff(g, SR_LOC_NODE, F, H);
-}
-
-static int nlin(sr_fgrid *g, int loc, const double *F, const double *const V[3], double *H) {
-    if (!F || !H || !V[0] || !V[1] || !V[2]) return set_err(SR_ERR_ARG, "null array");
-    if ((const double *)H == F || (const double *)H == V[0] || (const double *)H == V[1] || (const double *)H == V[2])
-        return set_err(SR_ERR_ARG, "H must not alias an input");
-    const FShape &f = g->shape[loc];
-    long n = (long)f.n[0] * f.n[1] * f.n[2];
-    hipLaunchKernelGGL(k_fd_nlin, dim3(nblocks(n)), dim3(256), 0, g->s, loc, f, g->shape[SR_LOC_VX],
-                       g->shape[SR_LOC_VY], g->shape[SR_LOC_VZ], g->M, F, V[0], V[1], V[2], H, 1.0 / g->h[0],
-                       1.0 / g->h[1], 1.0 / g->h[2]);
-    HIPCHK(hipGetLastError());
-    return SR_OK;
+    return diff(g, SR_LOC_NODE, 1, &F, &H);
 }
 
 extern "C" int sr_vf_nlin(sr_fgrid *g, const double *Ux, const double *Uy, const double *Uz, const double *Vx,
                           const double *Vy, const double *Vz, double *Hx, double *Hy, double *Hz) {
     if (!g) return set_err(SR_ERR_ARG, "null handle");
     // each component's H is written from U_c and the three V_d; H_c must alias none of them,
-    // including the other components' inputs that later launches read
+    // including the other components' inputs
     const double *V[3] = {Vx, Vy, Vz};
     const double *U[3] = {Ux, Uy, Uz};
     double *H[3] = {Hx, Hy, Hz};
@@ -449,15 +676,28 @@ extern "C" int sr_vf_nlin(sr_fgrid *g, const double *Ux, const double *Uy, const
         for (int e = 0; e < 3; e++)
             if ((const double *)H[c] == U[e] || (const double *)H[c] == V[e])
                 return set_err(SR_ERR_ARG, "H must not alias an input");
-    for (int c = 0; c < 3; c++) RETCHK(nlin(g, SR_LOC_VX + c, U[c], V, H[c]));
+    for (int c = 0; c < 3; c++)
+        if (!U[c] || !V[c] || !H[c]) return set_err(SR_ERR_ARG, "null array");
+    const ColGeo G = node_geo(g, g->N[0]);
+    const bool self = Ux == Vx && Uy == Vy && Uz == Vz;
+    for (int part = 0, one = one_launch(g, H, nullptr); part < (one ? 1 : 3); part++)
+        hipLaunchKernelGGL((self ? k_fd_nlin<true> : k_fd_nlin<false>), dim3(col_blocks(G)), dim3(kColThreads), 0, g->s, G,
+                           vel_geo(g), g->M, Ux, Uy, Uz, Vx, Vy, Vz, Hx, Hy, Hz, col_met(g), one ? 7 : 1 << part);
+    HIPCHK(hipGetLastError());
     return SR_OK;
 }
 
 extern "C" int sr_sf_nlin(sr_fgrid *g, const double *Vx, const double *Vy, const double *Vz, const double *F,
                           double *H) {
     if (!g) return set_err(SR_ERR_ARG, "null handle");
-    const double *V[3] = {Vx, Vy, Vz};
-    return nlin(g, SR_LOC_NODE, F, V, H);
+    if (!F || !H || !Vx || !Vy || !Vz) return set_err(SR_ERR_ARG, "null array");
+    if ((const double *)H == F || (const double *)H == Vx || (const double *)H == Vy || (const double *)H == Vz)
+        return set_err(SR_ERR_ARG, "H must not alias an input");
+    const ColGeo G = node_geo(g, g->N[0]);
+    hipLaunchKernelGGL(k_fd_nlin_node, dim3(col_blocks(G)), dim3(kColThreads), 0, g->s, G, vel_geo(g), g->M, F, Vx, Vy, Vz, H,
+                       col_met(g));
+    HIPCHK(hipGetLastError());
+    return SR_OK;
 }
 
 extern "C" int sr_divergence(sr_fgrid *g, const double *Vx, const double *Vy, const double *Vz, double *div) {
@@ -465,9 +705,9 @@ extern "C" int sr_divergence(sr_fgrid *g, const double *Vx, const double *Vy, co
     if (!Vx || !Vy || !Vz || !div) return set_err(SR_ERR_ARG, "null array");
     if ((const double *)div == Vx || (const double *)div == Vy || (const double *)div == Vz)
         return set_err(SR_ERR_ARG, "div must not alias an input");
-    const FShape &fp = g->shape[SR_LOC_NODE];
-    hipLaunchKernelGGL(k_fd_divergence, dim3(nblocks(fsz(fp))), dim3(256), 0, g->s, fp, g->shape[SR_LOC_VX],
-                       g->shape[SR_LOC_VY], g->shape[SR_LOC_VZ], g->M, Vx, Vy, Vz, div, g->h[0], g->h[1], g->h[2]);
+    const ColGeo G = node_geo(g, g->N[0] + 2);
+    hipLaunchKernelGGL(k_fd_divergence, dim3(col_blocks(G)), dim3(kColThreads), 0, g->s, G, vel_geo(g), g->M, Vx, Vy, Vz, div,
+                       col_met(g));
     HIPCHK(hipGetLastError());
     return SR_OK;
 }
@@ -478,12 +718,10 @@ extern "C" int sr_gradient(sr_fgrid *g, const double *F, double *Gx, double *Gy,
     if (!F || !Gx || !Gy || !Gz) return set_err(SR_ERR_ARG, "null array");
     for (int c = 0; c < 3; c++)
         if ((const double *)G[c] == F) return set_err(SR_ERR_ARG, "the gradient must not alias F");
-    for (int c = 0; c < 3; c++) {
-        const FShape &fc = g->shape[SR_LOC_VX + c];
-        long n = (long)fc.n[0] * fc.n[1] * fc.n[2];
-        hipLaunchKernelGGL(k_fd_gradient, dim3(nblocks(n)), dim3(256), 0, g->s, c, fc, g->shape[SR_LOC_NODE], g->M, F,
-                           G[c], g->h[c]);
-    }
+    const ColGeo C = node_geo(g, g->N[0]);
+    for (int part = 0, one = one_launch(g, G, nullptr); part < (one ? 1 : 3); part++)
+        hipLaunchKernelGGL(k_fd_gradient, dim3(col_blocks(C)), dim3(kColThreads), 0, g->s, C, vel_geo(g), g->M, F, Gx, Gy, Gz,
+                           col_met(g), one ? 7 : 1 << part);
     HIPCHK(hipGetLastError());
     return SR_OK;
 }

@@ -412,11 +412,8 @@ static void build_rhs(sr_ts *t) {
     const double *Vc[3] = {t->V[0], t->V[1], t->V[2]};
     // hydro_d3 multiplies the diffusion by 1/Re (hydro_d3.cc:259-262), scalar_d3 by nu
     const double visc = t->d.scalar ? t->nu : 1.0 / t->d.Re;
-    for (int c = 0; c < 3; c++) {
-        ts_build_rhs(c, t->fv, t->fp, t->M, Vc, t->P, t->H[c], t->h, visc, t->d.dt, t->d.scalar ? t->T : nullptr,
-                     t->Fb, t->s);
-        ts_ghost_wave(t->fv[c], t->H[c], t->sync_v[c], t->s);
-    }
+    ts_build_rhs(t->fp, t->M, Vc, t->P, t->H, t->h, visc, t->d.dt, t->d.scalar ? t->T : nullptr, t->Fb, t->s);
+    for (int c = 0; c < 3; c++) ts_ghost_wave(t->fv[c], t->H[c], t->sync_v[c], t->s);
 }
 
 extern "C" int sr_ts_build_rhs(sr_ts *t) {
@@ -577,7 +574,7 @@ extern "C" int sr_ts_time_advance(sr_ts *t, sr_ts_stats *st) {
     if (t->d.scalar) {
         // the temperature equation with the projected velocity (scalar_d3.cc:349-363)
         const double *Vp[3] = {t->V[0], t->V[1], t->V[2]};
-        ts_build_trhs(t->fp, t->fv, t->M, Vp, t->T, t->Trhs, t->h, t->kappa, dt, t->s);
+        ts_build_trhs(t->fp, t->M, Vp, t->T, t->Trhs, t->h, t->kappa, dt, t->s);
         ts_ghost_wave(t->fp, t->Trhs, t->sync_p, t->s);
         RETCHK(solve_t(t, nullptr));
     }
@@ -660,7 +657,7 @@ extern "C" int sr_ts_impose_tbc(sr_ts *t) {
 extern "C" int sr_ts_build_trhs(sr_ts *t) {
     RETCHK(need_scalar(t));
     const double *Vc[3] = {t->V[0], t->V[1], t->V[2]};
-    ts_build_trhs(t->fp, t->fv, t->M, Vc, t->T, t->Trhs, t->h, t->kappa, t->d.dt, t->s);
+    ts_build_trhs(t->fp, t->M, Vc, t->T, t->Trhs, t->h, t->kappa, t->d.dt, t->s);
     ts_ghost_wave(t->fp, t->Trhs, t->sync_p, t->s);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(t->s));
@@ -724,8 +721,9 @@ extern "C" int sr_ts_kernel_bytes(const sr_ts *t, int kernel, double *bytes) {
     const double w = 8.0;
     double b = 0.0;
     switch (kernel) {
-        case 0:   // nseRHS of the three components: V_c, the two other components' slices, P read, H_c written
-            for (int c = 0; c < 3; c++) b += 5.0 * w * (double)core_n(t->fv[c]);
+        case 0:   // nseRHS of the three components: V, P read, H written
+            b = w * (double)fsize(t->fp);
+            for (int c = 0; c < 3; c++) b += 2.0 * w * (double)fsize(t->fv[c]);
             break;
         case 1: b = 3.0 * w * (double)fsize(t->fv[0]); break;           // Jacobi sweep of Vx: V, R read, G written
         case 2: {                                                       // its residual over the bulk: V, R read
@@ -758,9 +756,8 @@ extern "C" int sr_ts_time_kernel(sr_ts *t, int kernel, int reps, double *avg_ms)
     auto launch = [&]() {
         switch (kernel) {
             case 0:
-                for (int c = 0; c < 3; c++)
-                    ts_build_rhs(c, t->fv, t->fp, t->M, Vc, t->P, t->H[c], t->h, visc, t->d.dt,
-                                 t->d.scalar ? t->T : nullptr, t->Fb, t->s);
+                ts_build_rhs(t->fp, t->M, Vc, t->P, t->H, t->h, visc, t->d.dt, t->d.scalar ? t->T : nullptr, t->Fb,
+                             t->s);
                 break;
             case 1: ts_jacobi(t->fv[0], t->M, B, t->V[0], t->H[0], t->G[0], J, t->s); break;
             case 2: ts_jacobi_res(t->fv[0], t->M, B, t->V[0], t->H[0], J, t->part, t->dmax, t->s); break;

@@ -58,14 +58,13 @@ struct GhostWave {
 
 void ts_deriv(const FShape &f, const Metrics &M, const double *F, double *out, int order, int d, double h,
               hipStream_t s);
-// nseRHS of component c; visc multiplies the diffusion (1/Re or nu); with T != null the
+// nseRHS of the three components; visc multiplies the diffusion (1/Re or nu); with T != null the
 // buoyancy Fb (T(k) + T(k+1)) / 2 is added to the z component
-void ts_build_rhs(int c, const FShape *fv, const FShape &fp, const Metrics &M, const double *const *V,
-                  const double *P, double *H, const double *h, double visc, double dt, const double *T, double Fb,
-                  hipStream_t s);
+void ts_build_rhs(const FShape &fp, const Metrics &M, const double *const *V, const double *P, double *const *H,
+                  const double *h, double visc, double dt, const double *T, double Fb, hipStream_t s);
 // tmpRHS of the temperature (scalar_d3.cc:349-357)
-void ts_build_trhs(const FShape &fp, const FShape *fv, const Metrics &M, const double *const *V, const double *T,
-                   double *R, const double *h, double kappa, double dt, hipStream_t s);
+void ts_build_trhs(const FShape &fp, const Metrics &M, const double *const *V, const double *T, double *R,
+                   const double *h, double kappa, double dt, hipStream_t s);
 void ts_nusselt(const FShape &fp, const FShape &fz, const Metrics &M, const double *Vz, const double *T,
                 const double *h, double *part, double *out, hipStream_t s);
 void ts_jacobi(const FShape &f, const Metrics &M, const Bulk &B, const double *V, const double *R, double *G,
