@@ -18,7 +18,7 @@
 namespace sr {
 
 constexpr int kColThreads = 256;
-// workgroups of kColThreads columns per plane, chunks of planes, planes per chunk (quotient, remainder)
+// workgroups of a number of columns per plane, chunks of planes, planes per chunk (quotient, remainder)
 struct ColGeo {
     int nb, nch, cq, cr;
 };
@@ -28,10 +28,10 @@ constexpr int kColAhead = 2;
 
 // Eight workgroups per CU where the planes suffice, and at most kColPlanes planes each.  The 257^3
 // operators with 1024 / 2048 / 4096 / 8192 / 16384 workgroups: 1611 / 1586 / 1571 / 1590 / 1683 us.
-inline ColGeo col_geo(long plane, int planes) {
+inline ColGeo col_geo(long plane, int planes, int threads = kColThreads) {
     ColGeo G;
-    G.nb = (int)((plane + kColThreads - 1) / kColThreads);
-    int nch = 2048 / G.nb;
+    G.nb = (int)((plane + threads - 1) / threads);
+    int nch = 2048 * 256 / threads / G.nb;
     if (nch < (planes + kColPlanes - 1) / kColPlanes) nch = (planes + kColPlanes - 1) / kColPlanes;
     if (nch > planes) nch = planes;
     G.nch = nch;
@@ -50,7 +50,7 @@ struct Col {
 __device__ inline Col column(const ColGeo &G) {
     const unsigned b = xcd_block(), tile = b / (unsigned)G.nch, chunk = b - tile * (unsigned)G.nch;
     Col C;
-    C.t = tile * (unsigned)kColThreads + threadIdx.x;
+    C.t = tile * blockDim.x + threadIdx.x;
     C.i0 = (int)chunk * G.cq + min((int)chunk, G.cr);
     C.i1 = C.i0 + G.cq + ((int)chunk < G.cr);
     return C;

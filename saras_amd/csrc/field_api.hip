@@ -45,8 +45,8 @@ struct sr_fgrid {
     double *dmet = nullptr;
     Metrics M{};
     hipStream_t s = nullptr;
-    double *part = nullptr;              // block maxima of the Jacobi residual
-    unsigned long long *dmax = nullptr, *hmax = nullptr;
+    JacobiSync *jsync = nullptr;
+    unsigned long long *dmax = nullptr, *hmax = nullptr;   // JacobiIO
     hipEvent_t jev = nullptr;            // marks a Jacobi residual's read-back
 };
 
@@ -550,11 +550,10 @@ static int fgrid_create_impl(const sr_fgrid_desc *desc, sr_fgrid *g) {
                 g->M.m[k][face][q] = g->dmet + off;
                 off += v.size();
             }
-    long nparts = ts_jacobi_res_parts();
-    for (int loc = 0; loc < 4; loc++) nparts = std::max(nparts, ts_jacobi_vres_parts(g->shape[loc]));
-    HIPCHK(hipMalloc((void **)&g->part, sizeof(double) * nparts));
     HIPCHK(hipEventCreateWithFlags(&g->jev, hipEventDisableTiming));
     HIPCHK(hipMalloc((void **)&g->dmax, sizeof(unsigned long long)));
+    HIPCHK(hipMalloc((void **)&g->jsync, sizeof(JacobiSync)));
+    HIPCHK(hipMemset(g->jsync, 0, sizeof(JacobiSync)));
     HIPCHK(hipHostMalloc((void **)&g->hmax, sizeof(unsigned long long), hipHostMallocDefault));
     return SR_OK;
 }
@@ -578,8 +577,8 @@ extern "C" int sr_fgrid_destroy(sr_fgrid *g) {
     if (g->s) (void)hipStreamSynchronize(g->s);
     if (g->dmet) (void)hipFree(g->dmet);
     if (g->jev) (void)hipEventDestroy(g->jev);
-    if (g->part) (void)hipFree(g->part);
     if (g->dmax) (void)hipFree(g->dmax);
+    if (g->jsync) (void)hipFree(g->jsync);
     if (g->hmax) (void)hipHostFree(g->hmax);
     if (g->s) (void)hipStreamDestroy(g->s);
     delete g;
@@ -756,7 +755,7 @@ extern "C" int sr_jacobi_visc(sr_fgrid *g, int loc, const sr_jacobi_desc *jd, co
     Bulk B = jacobi_bulk(f, per);
     long maxIterations = (long)(g->N[0] - 1) * (g->N[1] - 1) * (g->N[2] - 1);
     double *a = F, *b = G;
-    JacobiIO io{g->part, g->dmax, g->hmax, g->jev, g->s};
+    JacobiIO io{g->jsync, g->dmax, g->hmax, g->jev, g->s};
     int sweeps = 0;
     hipError_t err = hipSuccess;
     int st = ts_jacobi_loop(f, g->M, B, a, b, R, J, ws.data(), (int)ws.size(), io, jd->cnTolerance, maxIterations,

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/saras_mg.h"
+#include "grid_last.h"
 #include "mg_kernels.h"
 #include "mg_state.h"
 
@@ -372,6 +373,8 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
     HIPCHK(hipMalloc((void **)&m->fcount, sizeof(unsigned)));
     HIPCHK(hipMemsetAsync(m->fcount, 0, sizeof(unsigned), m->stream));
     m->fb_coef = FinalBufs{m->fstage, m->fcount};
+    HIPCHK(hipMalloc((void **)&m->mcount, sizeof(unsigned) * kGridWords));
+    HIPCHK(hipMemsetAsync(m->mcount, 0, sizeof(unsigned) * kGridWords, m->stream));
     launch_fill<double>(m->fterms, 4, 0.0, m->stream);
     HIPCHK(hipMalloc((void **)&m->dres, sizeof(double) * 16));
     HIPCHK(hipMalloc((void **)&m->diters, sizeof(int) * 4));
@@ -417,7 +420,7 @@ extern "C" int sr_mg_destroy(sr_mg *m) {
     }
     for (int q = 0; q < 6; q++) (void)hipFree(m->wall[q]);
     for (int a = 0; a < 3; a++) (void)hipFree(m->wvec[a]);
-    (void)hipFree(m->part); (void)hipFree(m->part2); (void)hipFree(m->mpart); (void)hipFree(m->fterms); (void)hipFree(m->fstage); (void)hipFree(m->fcount); (void)hipFree(m->dres); (void)hipFree(m->diters); (void)hipFree(m->stage);
+    (void)hipFree(m->part); (void)hipFree(m->part2); (void)hipFree(m->mpart); (void)hipFree(m->fterms); (void)hipFree(m->fstage); (void)hipFree(m->fcount); (void)hipFree(m->mcount); (void)hipFree(m->dres); (void)hipFree(m->diters); (void)hipFree(m->stage);
     (void)hipFree(m->stage2); (void)hipFree(m->r32);
     if (m->hres) (void)hipHostFree(m->hres);
     if (m->ev0) (void)hipEventDestroy(m->ev0);

@@ -17,6 +17,7 @@
 // to the node it copies.  (Dirichlet walls keep the kernels of mg_kernels.hip.)
 #include "mg_kernels.h"
 
+#include "grid_last.h"
 #include "mg_march.h"
 #include "xcd.h"
 
@@ -105,11 +106,8 @@ __device__ inline void block_sums(double (&s)[W], double &m) {
         }
 }
 
-// Partials of all workgroups, combined by the last of them in a fixed order: true there, in thread 0,
-// with the totals.  The partials travel as device-scope atomics, whose results are waited for before
-// the workgroup counts itself in, so that no fence is needed: a device-scope fence writes back the L2
-// with all that the workgroup stored (20.6 against 13.0 us for a 129 x 65 x 33 refinement step of 510
-// workgroups; 15.4 against 10.7 us for a 65^3 GCR step).
+// Partials of all workgroups, combined by the last of them (grid_last.h) in a fixed order: true there,
+// in thread 0, with the totals.
 template <int W>
 __device__ inline bool grid_sums(double (&s)[W], double &m, double *part, unsigned *counter) {
     __shared__ bool last;
@@ -123,8 +121,8 @@ __device__ inline bool grid_sums(double (&s)[W], double &m, double *part, unsign
                                            (unsigned long long)__double_as_longlong(i < W ? s[i < W ? i : 0] : m),
                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int i = 0; i <= W; i++) asm volatile("" : : "v"(old[i]) : "memory");
-        last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        for (int i = 0; i <= W; i++) arrived(old[i]);
+        last = grid_last(counter);
     }
     __syncthreads();
     if (!last) return false;
@@ -142,7 +140,6 @@ __device__ inline bool grid_sums(double (&s)[W], double &m, double *part, unsign
         m = fmax(m, v[W]);
     }
     block_sums<W>(s, m);
-    if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return threadIdx.x == 0;
 }
 

@@ -101,7 +101,7 @@ static bool march0(const sr_mg *m) { return march_outer_ok(m->lv[0].L, pressure_
 static void march_step(sr_mg *m, const double *x_in, const float *e, const float *z, double *x_out, float *z_next,
                        float *r32, bool color0 = false) {
     Level &V = m->lv[0];
-    const MarchSums S{m->mpart, m->fcount, m->fterms, m->dres, m->hres};
+    const MarchSums S{m->mpart, m->mcount, m->fterms, m->dres, m->hres};
     launch_march_residual(V.L, x_in, e, z, m->gcoef, V.f, x_out, z_next, r32, V.c64[0], V.c64[1], V.c64[2],
                           pressure_bc(m, 0, 0), color0, S, m->stream);
 }
@@ -313,7 +313,7 @@ static void gcr_body(sr_mg *m, int cur) {
     const bool q1r = std::min(Lc, m->depth) >= 1 && m->post32 > 0;
     if (march0(m)) {
         launch_march_dots(V.L, V.u32, z, V.f32, V.c32[0], V.c32[1], V.c32[2], error_bc(m, 0, 0), q1r, m->mpart,
-                          m->fcount, m->gcoef, s);
+                          m->mcount, m->gcoef, s);
         march_step(m, x_in, V.u32, z, x_out, z_next, V.f32);
         return;
     }

@@ -49,6 +49,7 @@ struct sr_mg {
     double *fterms = nullptr;    // right-hand side terms of computeError (device, 4 doubles)
     double *fstage = nullptr;    // stage of the GCR coefficients' two-stage final (FINAL_STAGE doubles)
     unsigned *fcount = nullptr;  // its counter (zero between launches)
+    unsigned *mcount = nullptr;  // grid_last words of the marches (mg_outer.hip)
     sr::FinalBufs fb_coef{};
     double *dres = nullptr;      // reduced quantities (device)
     double *hres = nullptr;      // pinned host mirror

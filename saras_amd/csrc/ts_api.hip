@@ -45,6 +45,7 @@ struct sr_ts {
     double *P = nullptr, *Pp = nullptr, *mgRHS = nullptr, *divV = nullptr;
     double *scratch = nullptr;                    // derivative output of the parity entry point
     double *part = nullptr, *dred = nullptr, *hred = nullptr;
+    JacobiSync *jsync = nullptr;
     unsigned long long *dmax = nullptr, *hmax = nullptr;
     hipEvent_t jev = nullptr;                    // marks a Jacobi residual's read-back
     std::vector<GhostWave> vbc[3];               // imposeU/V/WBCs as ordered waves
@@ -254,13 +255,13 @@ static int create_impl(const sr_ts_desc *desc, sr_ts *t) {
         t->tbc = tbc_waves(d, t->fp);
     }
     size_t nparts = std::max<size_t>(2 * (size_t)ts_energy_parts(t->fp), ts_jacobi_res_parts());
-    nparts = std::max<size_t>(nparts, (size_t)ts_jacobi_vres_parts(t->fp));
-    for (int c = 0; c < 3; c++) nparts = std::max<size_t>(nparts, (size_t)ts_jacobi_vres_parts(t->fv[c]));
     HIPCHK(hipMalloc((void **)&t->part, sizeof(double) * nparts));
     HIPCHK(hipEventCreateWithFlags(&t->jev, hipEventDisableTiming));
     HIPCHK(hipMalloc((void **)&t->dred, sizeof(double) * 4));
     HIPCHK(hipHostMalloc((void **)&t->hred, sizeof(double) * 4, hipHostMallocDefault));
     HIPCHK(hipMalloc((void **)&t->dmax, sizeof(unsigned long long)));
+    HIPCHK(hipMalloc((void **)&t->jsync, sizeof(JacobiSync)));
+    HIPCHK(hipMemset(t->jsync, 0, sizeof(JacobiSync)));
     HIPCHK(hipHostMalloc((void **)&t->hmax, sizeof(unsigned long long), hipHostMallocDefault));
     for (int c = 0; c < 3; c++) {
         t->vbc[c] = vbc_waves(d, t->fv[c], c);
@@ -285,6 +286,7 @@ extern "C" int sr_ts_destroy(sr_ts *t) {
         if (t->G[c]) (void)hipFree(t->G[c]);
     }
     if (t->dmax) (void)hipFree(t->dmax);
+    if (t->jsync) (void)hipFree(t->jsync);
     if (t->jev) (void)hipEventDestroy(t->jev);
     if (t->hred) (void)hipHostFree(t->hred);
     if (t->hmax) (void)hipHostFree(t->hmax);
@@ -435,7 +437,7 @@ static int jacobi(sr_ts *t, const FShape &f, double *&F, double *&G, const doubl
     int per[3] = {t->d.xPer, t->d.yPer, t->d.zPer};
     Bulk B = jacobi_bulk(f, per);
     long maxIterations = (long)(t->N[0] - 1) * (t->N[1] - 1) * (t->N[2] - 1);
-    JacobiIO io{t->part, t->dmax, t->hmax, t->jev, t->s};
+    JacobiIO io{t->jsync, t->dmax, t->hmax, t->jev, t->s};
     int sweeps = 0;
     hipError_t err = hipSuccess;
     int st = ts_jacobi_loop(f, t->M, B, F, G, R, J, bc.data(), (int)bc.size(), io, t->d.cnTolerance, maxIterations,
@@ -766,7 +768,7 @@ extern "C" int sr_ts_time_kernel(sr_ts *t, int kernel, int reps, double *avg_ms)
                 for (int c = 0; c < 3; c++) ts_project(c, t->fv[c], t->fp, t->M, t->Pp, t->V[c], t->h[c], t->d.dt, t->s);
                 break;
             case 5: ts_energy(t->fp, t->fv, t->M, Vc, t->h, t->part, t->dred, t->s); break;
-            case 6: ts_jacobi_vres(t->fv[0], t->M, B, t->V[0], t->H[0], t->G[0], J, t->part, t->dmax, t->s); break;
+            case 6: ts_jacobi_vres(t->fv[0], t->M, B, t->V[0], t->H[0], t->G[0], J, t->jsync, t->dmax, nullptr, t->s); break;
         }
     };
     hipEvent_t e0, e1;

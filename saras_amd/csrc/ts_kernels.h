@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "grid_last.h"
+
 namespace sr {
 
 // core sizes of a padded field and its staggering per direction (1 node, 0 face)
@@ -75,10 +77,15 @@ int ts_jacobi_res_parts();
 void ts_jacobi_res(const FShape &f, const Metrics &M, const Bulk &B, const double *V, const double *R,
                    const JacobiCoef &J, double *part, unsigned long long *out, hipStream_t s);
 // G = one Jacobi sweep of V (as ts_jacobi) and the max |residual| of V itself over the bulk (as
-// ts_jacobi_res) in one pass; part holds ts_jacobi_vres_parts(f) doubles
-long ts_jacobi_vres_parts(const FShape &f);
+// ts_jacobi_res) in one pass, in out[0] and, when given, the pinned host word; sync is 0 before the
+// first call
+struct JacobiSync {
+    unsigned words[kGridWords];
+    unsigned long long max[16 * kGridGroups];   // a cache line for each group of workgroups
+};
 void ts_jacobi_vres(const FShape &f, const Metrics &M, const Bulk &B, const double *V, const double *R, double *G,
-                    const JacobiCoef &J, double *part, unsigned long long *out, hipStream_t s);
+                    const JacobiCoef &J, JacobiSync *sync, unsigned long long *out, unsigned long long *host,
+                    hipStream_t s);
 void ts_ghost_wave(const FShape &f, double *F, const GhostWave &W, hipStream_t s);
 
 // The grid factors of the Jacobi solves (hydro_d3.cc:56-61: hx2hy2 = hx^2 hy^2 ...) for spacings h,
@@ -97,10 +104,9 @@ Bulk jacobi_bulk(const FShape &f, const int per[3]);
 // the sweep count are those of the sweep-then-check loop.  F and G are swapped as the iterates
 // move; on return F holds the converged iterate, or with status 1 the last one whose residual was
 // read after max_iter + 1 checks without convergence.  Returns 0 or 1, or -1 with *err set when a
-// HIP call failed.  part holds max(ts_jacobi_vres_parts(f), 1) doubles; G's BC waves may still be
-// queued on s on return.
+// HIP call failed.  G's BC waves may still be queued on s on return.
 struct JacobiIO {
-    double *part;
+    JacobiSync *sync;
     unsigned long long *dmax, *hmax;   // device maximum and its pinned host mirror
     hipEvent_t ev;
     hipStream_t s;
