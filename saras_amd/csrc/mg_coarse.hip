@@ -82,7 +82,7 @@ __device__ __forceinline__ T nb_sum(const Lvl<T> &V, const Node &N, const T *X, 
         w[q] = V.u[N.nb[q]];
         if (ANTI && (N.ghosts >> (8 + q) & 1u)) w[q] = -w[q];
     }
-    return X[0] * w[0] + X[1] * w[1] + Y[0] * w[2] + Y[1] * w[3] + Z[0] * w[4] + Z[1] * w[5];
+    return six(X[0], w[0], X[1], w[1], Y[0], w[2], Y[1], w[3], Z[0], w[4], Z[1], w[5]);
 }
 
 // Gauss-Seidel update of one node
@@ -186,7 +186,7 @@ __device__ __forceinline__ void column_sums(const Lay &L, const Lvl<T> &V, const
             yp *= C.syp;
             ym *= C.sym;
         }
-        s[q] = C.X0 * xp + C.X1 * xm + C.Y0 * yp + C.Y1 * ym + C.Z0[c][q] * z[q + 1] + C.Z1[c][q] * z[q];
+        s[q] = six(C.X0, xp, C.X1, xm, C.Y0, yp, C.Y1, ym, C.Z0[c][q], z[q + 1], C.Z1[c][q], z[q]);
     }
 }
 
@@ -427,7 +427,7 @@ __device__ inline int gs_wave(const Lay &L, const Lvl<T> &V, const Bc &bc, doubl
             if (ANTI && (N.ghosts >> (8 + q) & 1u)) o[q] = -o[q];
         }
     };
-    auto sum = [&](const T (&o)[6]) { return c0 * o[0] + c1 * o[1] + c2 * o[2] + c3 * o[3] + c4 * o[4] + c5 * o[5]; };
+    auto sum = [&](const T (&o)[6]) { return six(c0, o[0], c1, o[1], c2, o[2], c3, o[3], c4, o[4], c5, o[5]); };
     int it = 0;
     gather(x);
     while (true) {
@@ -476,8 +476,8 @@ __device__ inline int gs_block(const Lay &L, const Lvl<T> &V, const Bc &bc, doub
             if (!(col == 0 && (N.ghosts >> e & 1u))) w[e] = V.u[N.nb[e]];
             if (ANTI && (N.ghosts >> (8 + e) & 1u)) w[e] = -w[e];
         }
-        const T lu = X[0] * w[0] + X[1] * w[1] + Y[0] * w[2] + Y[1] * w[3] + Z[0] * w[4] + Z[1] * w[5] -
-                     diag3<T>(X, Y, Z) * V.u[N.own];
+        const T lu = fma(-diag3<T>(X, Y, Z), V.u[N.own],
+                         six(X[0], w[0], X[1], w[1], Y[0], w[2], Y[1], w[3], Z[0], w[4], Z[1], w[5]));
         const double m = fmax(-1.0e-10, fabs((double)V.f[N.own] - (double)lu));
         if (!__syncthreads_or(own && !(m < tol))) break;
         it += 1;

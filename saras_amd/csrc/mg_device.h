@@ -42,6 +42,19 @@ __device__ __forceinline__ T diag3(const T *X, const T *Y, const T *Z) {
     else return X[2] + Y[2] + Z[2];
 }
 
+// The six neighbour products of L u.  The roundings are written out (x- rounded, the others fused onto it in
+// order): left to the compiler they came out differently from kernel to kernel, and a refinement's
+// iterates then differ by FP32 roundings, which a poorly conditioned grid amplifies to 1e-8.
+template <typename T>
+__device__ __forceinline__ T six(T x0, T xp, T x1, T xm, T y0, T yp, T y1, T ym, T z0, T zp, T z1, T zm) {
+    T s = x1 * xm;
+    s = fma(x0, xp, s);
+    s = fma(y0, yp, s);
+    s = fma(y1, ym, s);
+    s = fma(z0, zp, s);
+    return fma(z1, zm, s);
+}
+
 // Face-ghost images of an updated node: a node whose padded index is the source of a ghost of a
 // periodic / mirror / anti direction writes that ghost (same colour, so no other thread of this
 // half sweep reads it).  Edge and corner ghosts are not read by the 7-point stencil.

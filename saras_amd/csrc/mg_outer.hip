@@ -79,8 +79,8 @@ __device__ __forceinline__ Pair<T> lap2(const Place &P, int kh, bool zper, bool 
     const T zm0 = kb ? lo : ext, zp0 = kb ? hi : own.a;
     const T zm1 = kb ? own.b : own.a, zp1 = kb ? ext : own.b;
     const T d0 = cen(X) + cen(Y) + cen(Z0), d1 = cen(X) + cen(Y) + cen(Z1);
-    return Pair<T>{X.p * xp.a + X.m * xm.a + Y.p * yp.a + Y.m * ym.a + Z0.p * zp0 + Z0.m * zm0 - d0 * c.a,
-                   X.p * xp.b + X.m * xm.b + Y.p * yp.b + Y.m * ym.b + Z1.p * zp1 + Z1.m * zm1 - d1 * c.b};
+    return Pair<T>{fma(-d0, c.a, six(X.p, xp.a, X.m, xm.a, Y.p, yp.a, Y.m, ym.a, Z0.p, zp0, Z0.m, zm0)),
+                   fma(-d1, c.b, six(X.p, xp.b, X.m, xm.b, Y.p, yp.b, Y.m, ym.b, Z1.p, zp1, Z1.m, zm1))};
 }
 
 // sums of W quantities and one maximum over the workgroup (a multiple of 64 threads), in thread 0

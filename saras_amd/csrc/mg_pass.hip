@@ -89,8 +89,8 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, MarchGeo G, const T *__
         }
         const T zm0 = kb ? lo : ext, zp0 = kb ? hi : own.a;
         const T zm1 = kb ? own.b : own.a, zp1 = kb ? ext : own.b;
-        T n0 = X.p * xp.a + X.m * xm.a + Y.p * yp.a + Y.m * ym.a + Z0.p * zp0 + Z0.m * zm0 - fv.a;
-        T n1 = X.p * xp.b + X.m * xm.b + Y.p * yp.b + Y.m * ym.b + Z1.p * zp1 + Z1.m * zm1 - fv.b;
+        const T n0 = six(X.p, xp.a, X.m, xm.a, Y.p, yp.a, Y.m, ym.a, Z0.p, zp0, Z0.m, zm0) - fv.a;
+        const T n1 = six(X.p, xp.b, X.m, xm.b, Y.p, yp.b, Y.m, ym.b, Z1.p, zp1, Z1.m, zm1) - fv.b;
         return Pair<T>{n0 / (cen(X) + cen(Y) + cen(Z0)), n1 / (cen(X) + cen(Y) + cen(Z1))};
     };
     // the entries of one colour's row at byte offset o.  Beside the core nodes a row holds its ghost
