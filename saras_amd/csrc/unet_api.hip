@@ -40,9 +40,15 @@ static int dalloc(sr_guess *g, T **p, long n) {
     return SR_OK;
 }
 
-static void repack(sr_guess *g, int l) {
-    launch_pack(g->W[l], kLayers[l].cin, kLayers[l].cout, 0, g->pf[l], g->s);
-    if (l > 0) launch_pack(g->W[l], kLayers[l].cin, kLayers[l].cout, 1, g->pb[l], g->s);
+static_assert(2 * SR_GUESS_LAYERS <= kMaxSegs, "segments");
+// layers l0 to l1 - 1
+static void repack(sr_guess *g, int l0, int l1) {
+    PackSegs P;
+    for (int l = l0; l < l1; l++) {
+        add_pack(P, g->W[l], kLayers[l].cin, kLayers[l].cout, 0, g->pf[l]);
+        if (l > 0) add_pack(P, g->W[l], kLayers[l].cin, kLayers[l].cout, 1, g->pb[l]);
+    }
+    launch_pack(P, g->s);
 }
 
 // SplitMix64 -> uniform -> Box-Muller
@@ -106,7 +112,7 @@ static int create_impl(const sr_guess_desc *desc, sr_guess *g) {
     long tmax = std::max(n0 * 16, std::max(n1 * 32, n2 * 64));
     RETCHK(dalloc(g, &g->tF, tmax));
     RETCHK(dalloc(g, &g->tM, tmax));
-    RETCHK(dalloc(g, &g->dy16, n0 * 16));
+    RETCHK(dalloc(g, &g->dy16, tmax));
     RETCHK(dalloc(g, &g->part, partmax));
     RETCHK(dalloc(g, &g->bpart, bpartmax));
     RETCHK(dalloc(g, &g->stage, n0 * SR_GUESS_IN_CH));
@@ -147,7 +153,7 @@ static int create_impl(const sr_guess_desc *desc, sr_guess *g) {
         }
         HIPCHK(hipMemcpyAsync(g->W[l], w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice, g->s));
         HIPCHK(hipStreamSynchronize(g->s));
-        repack(g, l);
+        repack(g, l, l + 1);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(g->s));
@@ -191,7 +197,7 @@ extern "C" int sr_guess_set_layer(sr_guess *g, int l, const float *W, const floa
     if (!g || !W || !b || l < 0 || l >= SR_GUESS_LAYERS) return set_err(SR_ERR_ARG, "bad argument");
     HIPCHK(hipMemcpyAsync(g->W[l], W, sizeof(float) * wsize(l), hipMemcpyHostToDevice, g->s));
     HIPCHK(hipMemcpyAsync(g->b[l], b, sizeof(float) * kLayers[l].cout, hipMemcpyHostToDevice, g->s));
-    repack(g, l);
+    repack(g, l, l + 1);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(g->s));
     return SR_OK;
@@ -218,15 +224,19 @@ extern "C" int sr_guess_get_grad(sr_guess *g, int l, float *dW, float *db) {
 // ------------------------------------------------------------------------------------------------
 static int conv(sr_guess *g, int l, const bf16_t *in, void *out, int mode) {
     const LayerSpec &L = kLayers[l];
-    if (launch_conv(L.cin, L.cout, g->lv[L.level], in, g->pf[l], g->b[l], out, mode, g->s) != 0)
+    if (launch_conv(L.cin, L.cout, g->lv[L.level], in, g->pf[l], g->b[l], out, mode, nullptr, g->s) != 0)
         return set_err(SR_ERR_ARG, "no convolution kernel for this channel pair");
     return SR_OK;
 }
 
-// adjoint convolution of layer l: dX (fp32, cin channels) from the bf16 gradient dY (cout channels)
-static int conv_adj(sr_guess *g, int l, const bf16_t *dY, float *dX) {
+// adjoint convolution of layer l from the bf16 gradient dY (cout channels): dX in fp32 (cin channels), or
+// behind the ReLU with the stored outputs act, in bf16
+static int conv_adj(sr_guess *g, int l, const bf16_t *dY, float *dX, const bf16_t *act = nullptr,
+                    bf16_t *dX16 = nullptr) {
     const LayerSpec &L = kLayers[l];
-    if (launch_conv(L.cout, L.cin, g->lv[L.level], dY, g->pb[l], nullptr, dX, CONV_F32, g->s) != 0)
+    void *out = act ? (void *)dX16 : (void *)dX;
+    if (launch_conv(L.cout, L.cin, g->lv[L.level], dY, g->pb[l], nullptr, out, act ? CONV_MASK : CONV_F32, act,
+                    g->s) != 0)
         return set_err(SR_ERR_ARG, "no adjoint convolution kernel for this channel pair");
     return SR_OK;
 }
@@ -266,48 +276,38 @@ int sr::guess_forward_device(sr_guess *g) {
 int sr::guess_backward_device(sr_guess *g) {
     const NetGrid *v = g->lv;
     hipStream_t s = g->s;
-    const long n0 = v[0].nvox(), n1 = v[1].nvox(), n2 = v[2].nvox(), n3 = v[3].nvox();
-    launch_expand_ch0(n0, g->dyd, g->dy16, s);
+    launch_expand_ch0(v[0].nvox(), g->dyd, g->dy16, s);
+    // a convolution cannot write over its input: the output's gradient is done with after layer 11
+    bf16_t *const other = g->dy16;
     RETCHK(wgrad(g, 11, g->dy16, g->T[G0]));
-    RETCHK(conv_adj(g, 11, g->dy16, g->tF));                 // d/dg0
-    launch_mask(n0 * 16, g->tF, g->T[G0], g->tM, s);
+    RETCHK(conv_adj(g, 11, g->dy16, nullptr, g->T[G0], g->tM));   // d/dg0
     RETCHK(wgrad(g, 10, g->tM, g->T[U0]));
     RETCHK(conv_adj(g, 10, g->tM, g->DS0));                  // d/du0 = d/ds0 (skip part)
-    launch_restrict_f32(v[0], v[1], 16, g->DS0, g->tF, 8.0f, s);   // prolongation adjoint = 8 R
-    launch_mask(n1 * 16, g->tF, g->T[G1], g->tM, s);
+    launch_restrict_mask(v[0], v[1], 16, g->DS0, g->T[G1], g->tM, 8.0f, s);   // prolongation adjoint = 8 R
     RETCHK(wgrad(g, 9, g->tM, g->T[U1]));
     RETCHK(conv_adj(g, 9, g->tM, g->DS1));                   // d/du1
-    launch_restrict_f32(v[1], v[2], 32, g->DS1, g->tF, 8.0f, s);
-    launch_mask(n2 * 32, g->tF, g->T[G2], g->tM, s);
+    launch_restrict_mask(v[1], v[2], 32, g->DS1, g->T[G2], g->tM, 8.0f, s);
     RETCHK(wgrad(g, 8, g->tM, g->T[U2]));
     RETCHK(conv_adj(g, 8, g->tM, g->DS2));                   // d/du2
-    launch_restrict_f32(v[2], v[3], 64, g->DS2, g->tF, 8.0f, s);
-    launch_mask(n3 * 64, g->tF, g->T[BB], g->tM, s);
+    launch_restrict_mask(v[2], v[3], 64, g->DS2, g->T[BB], g->tM, 8.0f, s);
     RETCHK(wgrad(g, 7, g->tM, g->T[A3]));
-    RETCHK(conv_adj(g, 7, g->tM, g->tF));                    // d/da3
-    launch_mask(n3 * 64, g->tF, g->T[A3], g->tM, s);
-    RETCHK(wgrad(g, 6, g->tM, g->T[X3]));
-    RETCHK(conv_adj(g, 6, g->tM, g->tF));                    // d/dx3
-    launch_prolong_add_f32(v[2], v[3], 64, g->tF, g->DS2, g->DS2, 0.125f, s);   // += R^T = P / 8
-    launch_mask(n2 * 64, g->DS2, g->T[S2], g->tM, s);
+    RETCHK(conv_adj(g, 7, g->tM, nullptr, g->T[A3], other));   // d/da3
+    RETCHK(wgrad(g, 6, other, g->T[X3]));
+    RETCHK(conv_adj(g, 6, other, g->tF));                    // d/dx3
+    launch_prolong_add_mask(v[2], v[3], 64, g->tF, g->DS2, g->T[S2], g->tM, 0.125f, s);   // += R^T = P / 8
     RETCHK(wgrad(g, 5, g->tM, g->T[A2]));
-    RETCHK(conv_adj(g, 5, g->tM, g->tF));
-    launch_mask(n2 * 64, g->tF, g->T[A2], g->tM, s);
-    RETCHK(wgrad(g, 4, g->tM, g->T[X2]));
-    RETCHK(conv_adj(g, 4, g->tM, g->tF));                    // d/dx2
-    launch_prolong_add_f32(v[1], v[2], 32, g->tF, g->DS1, g->DS1, 0.125f, s);
-    launch_mask(n1 * 32, g->DS1, g->T[S1], g->tM, s);
+    RETCHK(conv_adj(g, 5, g->tM, nullptr, g->T[A2], other));
+    RETCHK(wgrad(g, 4, other, g->T[X2]));
+    RETCHK(conv_adj(g, 4, other, g->tF));                    // d/dx2
+    launch_prolong_add_mask(v[1], v[2], 32, g->tF, g->DS1, g->T[S1], g->tM, 0.125f, s);
     RETCHK(wgrad(g, 3, g->tM, g->T[A1]));
-    RETCHK(conv_adj(g, 3, g->tM, g->tF));
-    launch_mask(n1 * 32, g->tF, g->T[A1], g->tM, s);
-    RETCHK(wgrad(g, 2, g->tM, g->T[X1]));
-    RETCHK(conv_adj(g, 2, g->tM, g->tF));                    // d/dx1
-    launch_prolong_add_f32(v[0], v[1], 16, g->tF, g->DS0, g->DS0, 0.125f, s);
-    launch_mask(n0 * 16, g->DS0, g->T[S0], g->tM, s);
+    RETCHK(conv_adj(g, 3, g->tM, nullptr, g->T[A1], other));
+    RETCHK(wgrad(g, 2, other, g->T[X1]));
+    RETCHK(conv_adj(g, 2, other, g->tF));                    // d/dx1
+    launch_prolong_add_mask(v[0], v[1], 16, g->tF, g->DS0, g->T[S0], g->tM, 0.125f, s);
     RETCHK(wgrad(g, 1, g->tM, g->T[A0]));
-    RETCHK(conv_adj(g, 1, g->tM, g->tF));
-    launch_mask(n0 * 16, g->tF, g->T[A0], g->tM, s);
-    RETCHK(wgrad(g, 0, g->tM, g->T[X0]));
+    RETCHK(conv_adj(g, 1, g->tM, nullptr, g->T[A0], other));
+    RETCHK(wgrad(g, 0, other, g->T[X0]));
     return SR_OK;
 }
 
@@ -315,12 +315,13 @@ int sr::guess_adam_device(sr_guess *g) {
     g->adam_t += 1;
     const double b1 = g->d.beta1, b2 = g->d.beta2;
     const float lr_t = (float)(g->d.lr * std::sqrt(1.0 - std::pow(b2, g->adam_t)) / (1.0 - std::pow(b1, g->adam_t)));
+    AdamSegs A;
     for (int l = 0; l < SR_GUESS_LAYERS; l++) {
-        launch_adam(wsize(l), g->W[l], g->dW[l], g->mW[l], g->vW[l], lr_t, g->d.beta1, g->d.beta2, g->d.eps, g->s);
-        launch_adam(kLayers[l].cout, g->b[l], g->db[l], g->mb[l], g->vb[l], lr_t, g->d.beta1, g->d.beta2, g->d.eps,
-                    g->s);
-        repack(g, l);
+        add_adam(A, (int)wsize(l), g->W[l], g->dW[l], g->mW[l], g->vW[l]);
+        add_adam(A, kLayers[l].cout, g->b[l], g->db[l], g->mb[l], g->vb[l]);
     }
+    launch_adam(A, lr_t, g->d.beta1, g->d.beta2, g->d.eps, g->s);
+    repack(g, 0, SR_GUESS_LAYERS);
     return SR_OK;
 }
 

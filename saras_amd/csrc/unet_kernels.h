@@ -22,16 +22,27 @@ inline NetGrid net_grid(int nx, int ny, int nz) {
     return g;
 }
 
-enum ConvOut { CONV_BF16_RELU = 0, CONV_F32 = 1, CONV_F32_CH0 = 2 };
+enum ConvOut { CONV_BF16_RELU = 0, CONV_F32 = 1, CONV_F32_CH0 = 2, CONV_MASK = 3 };
 
 // packed-weight size (bf16 elements) of a convolution CIN -> COUT
 long conv_pack_elems(int cin, int cout);
 // W (27, COUT, CIN) fp32 master weights -> packed bf16 fragments of the convolution; with
-// transpose, the packing of the adjoint convolution (COUT -> CIN, taps mirrored)
-void launch_pack(const float *W, int cin, int cout, int transpose, bf16_t *packed, hipStream_t s);
-// out = conv(in) (+ bias, ReLU, bf16) or raw fp32
+// transpose, the packing of the adjoint convolution (COUT -> CIN, taps mirrored).  Any number of
+// layers in one launch: workgroups first[q] to first[q + 1] - 1 take segment q.
+constexpr int kMaxSegs = 24;   // two for each layer
+struct PackSegs {
+    int n = 0, first[kMaxSegs + 1] = {};
+    const float *W[kMaxSegs];
+    bf16_t *packed[kMaxSegs];
+    int cin[kMaxSegs], cout[kMaxSegs], transpose[kMaxSegs];
+    long total[kMaxSegs];
+};
+void add_pack(PackSegs &P, const float *W, int cin, int cout, int transpose, bf16_t *packed);
+void launch_pack(const PackSegs &P, hipStream_t s);
+// out = conv(in) (+ bias, ReLU, bf16), raw fp32, or (CONV_MASK) bf16(conv(in) * (act > 0)).  At 129^3 x 16
+// channels the gradient through a ReLU as fp32 and a second kernel took 71 + 98 us, 74 this way.
 int launch_conv(int cin, int cout, const NetGrid &g, const bf16_t *in, const bf16_t *wpack, const float *bias,
-                void *out, int mode, hipStream_t s);
+                void *out, int mode, const bf16_t *act, hipStream_t s);
 // weight gradient: partials per slot, then the fixed-order sum into dW (27, COUT, CIN) fp32
 int wgrad_slots(int cin, int cout, const NetGrid &g);
 long wgrad_part_elems(int cin, int cout, const NetGrid &g);
@@ -42,22 +53,29 @@ int launch_wgrad(int cin, int cout, const NetGrid &g, const bf16_t *dy, const bf
 // transfer operators on channels-last tensors (C a multiple of 4)
 void launch_restrict_bf16(const NetGrid &fine, const NetGrid &coarse, int C, const bf16_t *in, bf16_t *out,
                           hipStream_t s);
-void launch_restrict_f32(const NetGrid &fine, const NetGrid &coarse, int C, const float *in, float *out, float scale,
-                         hipStream_t s);
+// out = bf16(scale R(in) * (act > 0))
+void launch_restrict_mask(const NetGrid &fine, const NetGrid &coarse, int C, const float *in, const bf16_t *act,
+                          bf16_t *out, float scale, hipStream_t s);
 // out = bf16(P(coarse) + skip)
 void launch_prolong_add_bf16(const NetGrid &fine, const NetGrid &coarse, int C, const bf16_t *coarse_in,
                              const bf16_t *skip, bf16_t *out, hipStream_t s);
-// out = acc + scale P(coarse)   (fp32; acc may alias out)
-void launch_prolong_add_f32(const NetGrid &fine, const NetGrid &coarse, int C, const float *coarse_in,
-                            const float *acc, float *out, float scale, hipStream_t s);
-// out = bf16(d * (y > 0))
-void launch_mask(long n, const float *d, const bf16_t *y, bf16_t *out, hipStream_t s);
+// out = bf16((acc + scale P(coarse)) * (act > 0)), the sum in fp32
+void launch_prolong_add_mask(const NetGrid &fine, const NetGrid &coarse, int C, const float *coarse_in,
+                             const float *acc, const bf16_t *act, bf16_t *out, float scale, hipStream_t s);
 void launch_f32_to_bf16(long n, const float *in, bf16_t *out, hipStream_t s);
 void launch_bf16_to_f32(long n, const bf16_t *in, float *out, hipStream_t s);
 // one channel of dy into a 16-channel bf16 tensor (the other channels zero)
 void launch_expand_ch0(long nvox, const float *dy, bf16_t *out16, hipStream_t s);
-// Adam on fp32 master weights (bias-corrected step sizes given by the host)
-void launch_adam(long n, float *w, const float *g, float *m, float *v, float lr_t, float beta1, float beta2,
-                 float eps, hipStream_t s);
+// Adam on fp32 master weights (bias-corrected step sizes given by the host), segments as in PackSegs: the
+// step of all layers took 47 launches with its packing, 480 us, and takes two
+struct AdamSegs {
+    int n = 0, first[kMaxSegs + 1] = {};
+    float *w[kMaxSegs];
+    const float *g[kMaxSegs];
+    float *m[kMaxSegs], *v[kMaxSegs];
+    int count[kMaxSegs];
+};
+void add_adam(AdamSegs &A, int n, float *w, const float *g, float *m, float *v);
+void launch_adam(const AdamSegs &A, float lr_t, float beta1, float beta2, float eps, hipStream_t s);
 
 }  // namespace sr

@@ -52,12 +52,20 @@ long conv_pack_elems(int cin, int cout) {
     return (long)(cin / ch) * conv_ns(cin) * (cout / 16) * 64 * 8;
 }
 
+// whether a ReLU passed: its stored output is positive
+__device__ __forceinline__ bool relu_on(unsigned y) { return y != 0 && !(y & 0x8000u); }
+
 // packed[(((c * NS + s) * NCB + cb) * 64 + lane) * 8 + i] = W'[tap][co][ci] with
 // co = cb * 16 + lane % 16, kk = s * 32 + 8 (lane / 16) + i, tap = kk / CH, ci = c * CH + kk % CH
-__global__ void k_pack(const float *__restrict__ W, int cin_l, int cout_l, int transpose, int cin, int cout,
-                       long total, bf16_t *__restrict__ packed) {
-    long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= total) return;
+__global__ void __launch_bounds__(256) k_pack(PackSegs P) {
+    int q = 0;
+    while (q + 1 < P.n && (int)blockIdx.x >= P.first[q + 1]) q++;
+    const float *__restrict__ W = P.W[q];
+    bf16_t *__restrict__ packed = P.packed[q];
+    const int transpose = P.transpose[q], cin_l = P.cin[q], cout_l = P.cout[q];
+    const int cin = transpose ? cout_l : cin_l, cout = transpose ? cin_l : cout_l;
+    const long e = (long)((int)blockIdx.x - P.first[q]) * 256 + threadIdx.x;
+    if (e >= P.total[q]) return;
     int ch = cin < 32 ? cin : 32;
     int ns = (27 * ch + 31) / 32, ncb = cout / 16;
     int i = (int)(e % 8);
@@ -82,7 +90,7 @@ __global__ void k_pack(const float *__restrict__ W, int cin_l, int cout_l, int t
 template <int CIN, int COUT>
 __global__ void __launch_bounds__(256) k_conv(NetGrid g, const bf16_t *__restrict__ in,
                                               const bf16_t *__restrict__ wpack, const float *__restrict__ bias,
-                                              void *__restrict__ out, int mode) {
+                                              void *__restrict__ out, int mode, const bf16_t *__restrict__ act) {
     using K = ConvShape<CIN>;
     constexpr int CH = K::CH, NCH = K::NCH, NS = K::NS, VS = K::VS, NCB = COUT / 16, PARTS = CH / 8;
     __shared__ __attribute__((aligned(16))) bf16_t halo[648 * VS];
@@ -148,6 +156,14 @@ __global__ void __launch_bounds__(256) k_conv(NetGrid g, const bf16_t *__restric
                 float r3 = fmaxf(acc[yy][cb][3] + bias[co0 + 3], 0.f);
                 u32x2 pk = {(unsigned)f2bf(r0) | ((unsigned)f2bf(r1) << 16),
                             (unsigned)f2bf(r2) | ((unsigned)f2bf(r3) << 16)};
+                *(u32x2 *)((bf16_t *)out + v * COUT + co0) = pk;
+            } else if (mode == CONV_MASK) {
+                const u32x2 y = *(const u32x2 *)(act + v * COUT + co0);
+                u32x2 pk;
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    pk[h] = (unsigned)f2bf(relu_on(y[h] & 0xffffu) ? acc[yy][cb][2 * h] : 0.f) |
+                            ((unsigned)f2bf(relu_on(y[h] >> 16) ? acc[yy][cb][2 * h + 1] : 0.f) << 16);
                 *(u32x2 *)((bf16_t *)out + v * COUT + co0) = pk;
             } else if (mode == CONV_F32) {
                 *(f32x4 *)((float *)out + v * COUT + co0) = acc[yy][cb];
@@ -375,11 +391,18 @@ __device__ __forceinline__ void store4(float *p, const float *v) {
     *(f32x4 *)p = u;
 }
 
+// x where the ReLU with the stored outputs act passed, else 0
+__device__ inline void mask4(const bf16_t *act, float (&x)[4]) {
+    const u32x2 y = *(const u32x2 *)act;
+#pragma unroll
+    for (int q = 0; q < 4; q++) x[q] = relu_on((y[q >> 1] >> (16 * (q & 1))) & 0xffffu) ? x[q] : 0.f;
+}
+
 // full weighting: coarse I = sum over fine 2I + (a, b, c), a, b, c in {-1, 0, 1}, of
 // w(a) w(b) w(c) (w(0) = 1/2, w(+-1) = 1/4), zero outside; times scale
 template <typename TI, typename TO>
 __global__ void __launch_bounds__(256) k_restrict(NetGrid f, NetGrid cg, int C, const TI *__restrict__ in,
-                                                  TO *__restrict__ out, float scale) {
+                                                  TO *__restrict__ out, float scale, const bf16_t *__restrict__ act) {
     const int C4 = C / 4;
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= cg.nvox() * C4) return;
@@ -406,6 +429,7 @@ __global__ void __launch_bounds__(256) k_restrict(NetGrid f, NetGrid cg, int C, 
         }
     }
     for (int q = 0; q < 4; q++) acc[q] *= scale;
+    if (act) mask4(act + v * C + c4 * 4, acc);
     store4(out + v * C + c4 * 4, acc);
 }
 
@@ -413,7 +437,7 @@ __global__ void __launch_bounds__(256) k_restrict(NetGrid f, NetGrid cg, int C, 
 // out = bf16(P(coarse) + skip)   or   out = acc + scale P(coarse)
 template <typename TI, typename TS, typename TO>
 __global__ void __launch_bounds__(256) k_prolong(NetGrid f, NetGrid cg, int C, const TI *__restrict__ cin,
-                                                 const TS *add, TO *out, float scale) {
+                                                 const TS *add, TO *out, float scale, const bf16_t *__restrict__ act) {
     const int C4 = C / 4;
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= f.nvox() * C4) return;
@@ -435,13 +459,8 @@ __global__ void __launch_bounds__(256) k_prolong(NetGrid f, NetGrid cg, int C, c
     float s[4];
     load4(add + v * C + c4 * 4, s);
     for (int q = 0; q < 4; q++) acc[q] = s[q] + scale * acc[q];
+    if (act) mask4(act + v * C + c4 * 4, acc);
     store4(out + v * C + c4 * 4, acc);
-}
-
-__global__ void __launch_bounds__(256) k_mask(long n, const float *__restrict__ d, const bf16_t *__restrict__ y,
-                                              bf16_t *__restrict__ out) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) out[t] = f2bf(y[t] != 0 && !(y[t] & 0x8000u) ? d[t] : 0.0f);
 }
 
 __global__ void __launch_bounds__(256) k_f32_to_bf16(long n, const float *__restrict__ in, bf16_t *__restrict__ out) {
@@ -459,11 +478,14 @@ __global__ void __launch_bounds__(256) k_expand_ch0(long nvox, const float *__re
     if (t < nvox * 16) out[t] = (t % 16) == 0 ? f2bf(dy[t / 16]) : (bf16_t)0;
 }
 
-__global__ void __launch_bounds__(256) k_adam(long n, float *__restrict__ w, const float *__restrict__ g,
-                                              float *__restrict__ m, float *__restrict__ v, float lr_t, float b1,
-                                              float b2, float eps) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
+// all layers' weights and biases in one launch
+__global__ void __launch_bounds__(256) k_adam(AdamSegs A, float lr_t, float b1, float b2, float eps) {
+    int q = 0;
+    while (q + 1 < A.n && (int)blockIdx.x >= A.first[q + 1]) q++;
+    float *__restrict__ w = A.w[q], *__restrict__ m = A.m[q], *__restrict__ v = A.v[q];
+    const float *__restrict__ g = A.g[q];
+    const int t = ((int)blockIdx.x - A.first[q]) * 256 + (int)threadIdx.x;
+    if (t >= A.count[q]) return;
     float gr = g[t];
     float mm = b1 * m[t] + (1.f - b1) * gr;
     float vv = b2 * v[t] + (1.f - b2) * gr * gr;
@@ -477,21 +499,30 @@ __global__ void __launch_bounds__(256) k_adam(long n, float *__restrict__ w, con
 // ------------------------------------------------------------------------------------------------
 static inline unsigned nblk(long n) { return (unsigned)((n + 255) / 256); }
 
-void launch_pack(const float *W, int cin, int cout, int transpose, bf16_t *packed, hipStream_t s) {
-    int ci = transpose ? cout : cin, co = transpose ? cin : cout;
-    long total = conv_pack_elems(ci, co);
-    hipLaunchKernelGGL(k_pack, dim3(nblk(total)), dim3(256), 0, s, W, cin, cout, transpose, ci, co, total, packed);
+void add_pack(PackSegs &P, const float *W, int cin, int cout, int transpose, bf16_t *packed) {
+    const int q = P.n++;
+    P.W[q] = W;
+    P.packed[q] = packed;
+    P.cin[q] = cin;
+    P.cout[q] = cout;
+    P.transpose[q] = transpose;
+    P.total[q] = conv_pack_elems(transpose ? cout : cin, transpose ? cin : cout);
+    P.first[q + 1] = P.first[q] + (int)nblk(P.total[q]);
+}
+
+void launch_pack(const PackSegs &P, hipStream_t s) {
+    hipLaunchKernelGGL(k_pack, dim3(P.first[P.n]), dim3(256), 0, s, P);
 }
 
 #define CONV_CASE(CI, CO)                                                                                  \
     if (cin == CI && cout == CO) {                                                                         \
         hipLaunchKernelGGL((k_conv<CI, CO>), dim3((unsigned)g.ntiles()), dim3(256), 0, s, g, in, wpack, bias, \
-                           out, mode);                                                                     \
+                           out, mode, act);                                                                \
         return 0;                                                                                          \
     }
 
 int launch_conv(int cin, int cout, const NetGrid &g, const bf16_t *in, const bf16_t *wpack, const float *bias,
-                void *out, int mode, hipStream_t s) {
+                void *out, int mode, const bf16_t *act, hipStream_t s) {
     CONV_CASE(8, 16)
     CONV_CASE(16, 16)
     CONV_CASE(16, 32)
@@ -545,29 +576,25 @@ int launch_wgrad(int cin, int cout, const NetGrid &g, const bf16_t *dy, const bf
 void launch_restrict_bf16(const NetGrid &fine, const NetGrid &coarse, int C, const bf16_t *in, bf16_t *out,
                           hipStream_t s) {
     hipLaunchKernelGGL((k_restrict<bf16_t, bf16_t>), dim3(nblk(coarse.nvox() * (C / 4))), dim3(256), 0, s, fine,
-                       coarse, C, in, out, 1.0f);
+                       coarse, C, in, out, 1.0f, nullptr);
 }
 
-void launch_restrict_f32(const NetGrid &fine, const NetGrid &coarse, int C, const float *in, float *out, float scale,
-                         hipStream_t s) {
-    hipLaunchKernelGGL((k_restrict<float, float>), dim3(nblk(coarse.nvox() * (C / 4))), dim3(256), 0, s, fine, coarse,
-                       C, in, out, scale);
+void launch_restrict_mask(const NetGrid &fine, const NetGrid &coarse, int C, const float *in, const bf16_t *act,
+                          bf16_t *out, float scale, hipStream_t s) {
+    hipLaunchKernelGGL((k_restrict<float, bf16_t>), dim3(nblk(coarse.nvox() * (C / 4))), dim3(256), 0, s, fine, coarse,
+                       C, in, out, scale, act);
 }
 
 void launch_prolong_add_bf16(const NetGrid &fine, const NetGrid &coarse, int C, const bf16_t *coarse_in,
                              const bf16_t *skip, bf16_t *out, hipStream_t s) {
     hipLaunchKernelGGL((k_prolong<bf16_t, bf16_t, bf16_t>), dim3(nblk(fine.nvox() * (C / 4))), dim3(256), 0, s, fine,
-                       coarse, C, coarse_in, skip, out, 1.0f);
+                       coarse, C, coarse_in, skip, out, 1.0f, nullptr);
 }
 
-void launch_prolong_add_f32(const NetGrid &fine, const NetGrid &coarse, int C, const float *coarse_in,
-                            const float *acc, float *out, float scale, hipStream_t s) {
-    hipLaunchKernelGGL((k_prolong<float, float, float>), dim3(nblk(fine.nvox() * (C / 4))), dim3(256), 0, s, fine,
-                       coarse, C, coarse_in, acc, out, scale);
-}
-
-void launch_mask(long n, const float *d, const bf16_t *y, bf16_t *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_mask, dim3(nblk(n)), dim3(256), 0, s, n, d, y, out);
+void launch_prolong_add_mask(const NetGrid &fine, const NetGrid &coarse, int C, const float *coarse_in,
+                             const float *acc, const bf16_t *act, bf16_t *out, float scale, hipStream_t s) {
+    hipLaunchKernelGGL((k_prolong<float, float, bf16_t>), dim3(nblk(fine.nvox() * (C / 4))), dim3(256), 0, s, fine,
+                       coarse, C, coarse_in, acc, out, scale, act);
 }
 
 void launch_f32_to_bf16(long n, const float *in, bf16_t *out, hipStream_t s) {
@@ -582,9 +609,18 @@ void launch_expand_ch0(long nvox, const float *dy, bf16_t *out16, hipStream_t s)
     hipLaunchKernelGGL(k_expand_ch0, dim3(nblk(nvox * 16)), dim3(256), 0, s, nvox, dy, out16);
 }
 
-void launch_adam(long n, float *w, const float *g, float *m, float *v, float lr_t, float beta1, float beta2,
-                 float eps, hipStream_t s) {
-    hipLaunchKernelGGL(k_adam, dim3(nblk(n)), dim3(256), 0, s, n, w, g, m, v, lr_t, beta1, beta2, eps);
+void add_adam(AdamSegs &A, int n, float *w, const float *g, float *m, float *v) {
+    const int q = A.n++;
+    A.w[q] = w;
+    A.g[q] = g;
+    A.m[q] = m;
+    A.v[q] = v;
+    A.count[q] = n;
+    A.first[q + 1] = A.first[q] + (int)nblk(n);
+}
+
+void launch_adam(const AdamSegs &A, float lr_t, float beta1, float beta2, float eps, hipStream_t s) {
+    hipLaunchKernelGGL(k_adam, dim3(A.first[A.n]), dim3(256), 0, s, A, lr_t, beta1, beta2, eps);
 }
 
 }  // namespace sr
