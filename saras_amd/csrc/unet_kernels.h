@@ -17,6 +17,25 @@ struct NetGrid {
     __host__ __device__ long ntiles() const { return (long)tx * ty * tz; }
 };
 
+// t = q n + r and t = (i n1 + j) n2 + k: in 32 bits where t has no more (64-bit divisions cost some hundred
+// instructions each)
+__device__ inline void split2(long t, int n, long &q, int &r) {
+    if (t >> 32) {
+        q = t / n;
+        r = (int)(t - q * n);
+    } else {
+        const unsigned u = (unsigned)t, a = u / (unsigned)n;
+        q = a;
+        r = (int)(u - a * (unsigned)n);
+    }
+}
+__device__ inline void node3(long t, int n1, int n2, int &i, int &j, int &k) {
+    long a, b;
+    split2(t, n2, a, k);
+    split2(a, n1, b, j);
+    i = (int)b;
+}
+
 inline NetGrid net_grid(int nx, int ny, int nz) {
     NetGrid g{nx, ny, nz, (nx + 3) / 4, (ny + 3) / 4, (nz + 15) / 16};
     return g;

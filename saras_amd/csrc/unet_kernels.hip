@@ -406,9 +406,10 @@ __global__ void __launch_bounds__(256) k_restrict(NetGrid f, NetGrid cg, int C, 
     const int C4 = C / 4;
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= cg.nvox() * C4) return;
-    int c4 = (int)(t % C4);
-    long v = t / C4;
-    int K = (int)(v % cg.nz), J = (int)((v / cg.nz) % cg.ny), I = (int)(v / ((long)cg.nz * cg.ny));
+    int c4, I, J, K;
+    long v;
+    split2(t, C4, v, c4);
+    node3(v, cg.ny, cg.nz, I, J, K);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     for (int a = -1; a <= 1; a++) {
         int i = 2 * I + a;
@@ -441,9 +442,10 @@ __global__ void __launch_bounds__(256) k_prolong(NetGrid f, NetGrid cg, int C, c
     const int C4 = C / 4;
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= f.nvox() * C4) return;
-    int c4 = (int)(t % C4);
-    long v = t / C4;
-    int k = (int)(v % f.nz), j = (int)((v / f.nz) % f.ny), i = (int)(v / ((long)f.nz * f.ny));
+    int c4, i, j, k;
+    long v;
+    split2(t, C4, v, c4);
+    node3(v, f.ny, f.nz, i, j, k);
     int ia[2] = {i >> 1, (i + 1) >> 1}, ja[2] = {j >> 1, (j + 1) >> 1}, ka[2] = {k >> 1, (k + 1) >> 1};
     int ni = (i & 1) ? 2 : 1, nj = (j & 1) ? 2 : 1, nk = (k & 1) ? 2 : 1;
     float wi = (i & 1) ? 0.5f : 1.0f, wj = (j & 1) ? 0.5f : 1.0f, wk = (k & 1) ? 0.5f : 1.0f;
@@ -474,8 +476,11 @@ __global__ void __launch_bounds__(256) k_bf16_to_f32(long n, const bf16_t *__res
 }
 
 __global__ void __launch_bounds__(256) k_expand_ch0(long nvox, const float *__restrict__ dy, bf16_t *__restrict__ out) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nvox * 16) out[t] = (t % 16) == 0 ? f2bf(dy[t / 16]) : (bf16_t)0;
+    long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nvox) return;
+    u32x4 *const o = (u32x4 *)(out + 16 * v);
+    o[0] = (u32x4){(unsigned)f2bf(dy[v]), 0u, 0u, 0u};
+    o[1] = (u32x4){0u, 0u, 0u, 0u};
 }
 
 // all layers' weights and biases in one launch
@@ -606,7 +611,7 @@ void launch_bf16_to_f32(long n, const bf16_t *in, float *out, hipStream_t s) {
 }
 
 void launch_expand_ch0(long nvox, const float *dy, bf16_t *out16, hipStream_t s) {
-    hipLaunchKernelGGL(k_expand_ch0, dim3(nblk(nvox * 16)), dim3(256), 0, s, nvox, dy, out16);
+    hipLaunchKernelGGL(k_expand_ch0, dim3(nblk(nvox)), dim3(256), 0, s, nvox, dy, out16);
 }
 
 void add_adam(AdamSegs &A, int n, float *w, const float *g, float *m, float *v) {
