@@ -34,10 +34,22 @@ sys.path.insert(0, ROOT)
 
 METRIC = "ms/Poisson solve to 1e-10 rel. residual, 257³ (learned+mixed vs FP64 MG)"
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch of the roofline kernels, from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE
-# (KiB per dispatch) scaled by what the same counters read for a device copy of known size
-# (FETCH_SIZE x 2.005, WRITE_SIZE x 1.0); the summaries and commands are in profiles/
-TRAFFIC_BYTES = {"k_rb_sweep<float> 257x257x257": 124.4e6, "k_rb_sweep<double> 257x257x257": 229.0e6}
+
+
+def half_sweep_bytes(solver, kernel):
+    """Algorithmic bytes of a finest half sweep within the one-launch sweeps of the pre-smoothing (two
+    sweeps, k_rb_pass).  Per node of a first and a last sweep, in words: f and colour 1 read, colour 1
+    written, 2; the same and colour 0 written, 2.5.  The FP32 cycle starts from zero and does not read
+    colour 1 first, 1.5.  kernel_bytes counts the 3 words per updated node of a single half sweep."""
+    return solver.kernel_bytes(kernel, 0) / 1.5 * ((2.0 + 2.5) if kernel == 0 else (1.5 + 2.5)) / 4.0
+
+
+def cycle_bytes(n_levels):
+    """Algorithmic bytes of one FP64 V(2,2) cycle: 90 B per node on every level above the coarsest (two
+    first sweeps, 16 B, two last ones, 20 B; residual read on colour 0 with its restriction, 8 B, and the
+    coarse right-hand side written, 1 B; prolongation onto colour 1, 9 B), 4 B less below the finest, whose
+    pre-smoothing starts from zero, + 12 B per finest node for the colour-0 norm."""
+    return 102.0 * n_levels[0] + 86.0 * sum(n_levels[1:-1])
 
 
 def host_info():
@@ -205,7 +217,7 @@ def tgv_bench(args):
     # the step kernels one by one (HIP events on the handle's stream) against their algorithmic
     # bytes; timed after the stepped state was read, since they overwrite what they write
     kernels = {}
-    for kid, name in ((0, "k_build_rhs x3"), (1, "k_jacobi_v (Vx)"), (2, "k_jacobi_res (Vx)"),
+    for kid, name in ((0, "k_build_rhs"), (1, "k_jacobi_v (Vx)"), (2, "k_jacobi_res (Vx)"),
                       (6, "k_jacobi_vres (Vx: sweep + residual of its input)"), (3, "k_divergence"),
                       (4, "k_project x3"), (5, "k_energy")):
         kms = h.time_kernel(kid, reps=20)
@@ -257,11 +269,11 @@ def tgv_bench(args):
                    "ke_trace_every_10": ke[::10], "max_divergence_end": maxdiv,
                    "ke_rel_diff_vs_oracle_first_steps": ke_check, "ke_steps_checked_vs_oracle": ke_steps_checked,
                    "step_kernels": kernels},
-        "roofline": {"bound": "hbm", "kernel": "k_build_rhs x3 (the largest non-multigrid kernel of the step)",
-                     "achieved": kernels["k_build_rhs x3"]["GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": kernels["k_build_rhs x3"]["frac"], "traffic": None,
-                     "bytes_per_launch": kernels["k_build_rhs x3"]["bytes"],
-                     "avg_launch_ms": kernels["k_build_rhs x3"]["ms"]},
+        "roofline": {"bound": "hbm", "kernel": "k_build_rhs (the largest non-multigrid kernel of the step)",
+                     "achieved": kernels["k_build_rhs"]["GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": kernels["k_build_rhs"]["frac"], "traffic": None,
+                     "bytes_per_launch": kernels["k_build_rhs"]["bytes"],
+                     "avg_launch_ms": kernels["k_build_rhs"]["ms"]},
         "cpu_baseline": cpu,
     }
     print(json.dumps(out))
@@ -356,13 +368,9 @@ def rbc_bench(args):
         sols[name] = h.download(ts.P)
         h.close()
     net.close()
-    # algorithmic bytes of one FP64 V(2,2) cycle: 114 B per node on every level above the coarsest
-    # (four sweeps of two half sweeps, 96 B; residual read on colour 0 with its restriction, 8 B, and
-    # the coarse right-hand side written, 1 B; prolongation onto colour 1, 9 B) + 12 B per finest
-    # node for the colour-0 norm
     depth = nz_ind - 1
     n_levels = [((n[0] - 1 >> l) + 1) * ((n[1] - 1 >> l) + 1) * ((n[2] - 1 >> l) + 1) for l in range(depth + 1)]
-    cyc_bytes = 114.0 * sum(n_levels[:-1]) + 12.0 * n_levels[0]
+    cyc_bytes = cycle_bytes(n_levels)
     a_, b_ = sol_l[1:-1, 1:-1, 1:-1], sols["fp64_warm"][1:-1, 1:-1, 1:-1]
     dP = (a_ - a_.mean()) - (b_ - b_.mean())
     base = out["fp64_warm"]["ms_per_solve"]
@@ -372,8 +380,7 @@ def rbc_bench(args):
     if nz_ind == 7:
         p.Lx, p.Ly = 2.0, 2.0
     solver = mg.Multigrid(mg.Grid(p), p)
-    bytes_sweep = solver.kernel_bytes(6, 0)
-    iso_ms = solver.time_kernel(6, 0, 20)
+    bytes_sweep = half_sweep_bytes(solver, 6)
     solver.close()
     sweep_ms = learned["sweep0_ms_mean"]
     achieved = bytes_sweep / (sweep_ms * 1e-3) / 1e9 if sweep_ms > 0 else None
@@ -419,12 +426,11 @@ def rbc_bench(args):
                                                                           np.linalg.norm(b_ - b_.mean())),
                    "train_seconds": round(train_s, 2), "train_loss_first": train_loss[:3],
                    "train_loss_last": train_loss[-3:], "nusselt_end": nu_end},
-        "roofline": {"bound": "hbm", "kernel": "k_rb_sweep<float> finest level (FP32 V-cycle)",
+        "roofline": {"bound": "hbm", "kernel": "k_rb_pass<float> finest level, per half sweep (FP32 V-cycle)",
                      "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
-                     "traffic": TRAFFIC_BYTES.get(f"k_rb_sweep<float> {n[0]}x{n[1]}x{n[2]}"),
-                     "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5),
-                     "avg_launch_ms_isolated": round(iso_ms, 5)},
+                     "traffic": None,
+                     "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5)},
         "cpu_baseline": cpu,
     }
     print(json.dumps(res))
@@ -483,11 +489,9 @@ def seq_bench(args):
     p.precision, p.coarseDirect = mg._L.SR_PREC_MIXED_GCR, 1
     solver = mg.Multigrid(seq.g, p)
     sweep_ms = lm["sweep0_ms_mean"]
-    bytes_sweep = solver.kernel_bytes(6, 0)
-    iso_ms = solver.time_kernel(6, 0, 20)
+    bytes_sweep = half_sweep_bytes(solver, 6)
     solver.close()
     achieved = bytes_sweep / (sweep_ms * 1e-3) / 1e9 if sweep_ms > 0 else None
-    traffic = TRAFFIC_BYTES.get("k_rb_sweep<float> 257x257x257")
     cpu = None
     if not args.no_cpu:
         pc, gc, fc = workloads.stretched_poisson(ind=8, beta=1.0, seed=0)
@@ -510,11 +514,10 @@ def seq_bench(args):
                    "learned_mixed_rel_l2_diff_vs_fp64_last_step": float(np.linalg.norm(dm) /
                                                                        np.linalg.norm(b - b.mean())),
                    "legs": res},
-        "roofline": {"bound": "hbm", "kernel": "k_rb_sweep<float> finest level (FP32 V-cycle)",
+        "roofline": {"bound": "hbm", "kernel": "k_rb_pass<float> finest level, per half sweep (FP32 V-cycle)",
                      "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None, "traffic": traffic,
-                     "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5),
-                     "avg_launch_ms_isolated": round(iso_ms, 5)},
+                     "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None, "traffic": None,
+                     "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5)},
         "cpu_baseline": cpu,
     }
     print(json.dumps(out))
@@ -811,16 +814,13 @@ def main():
     conv = all(s.converged for s in stats)
     sweep_ms = float(np.mean([s.sweep0_ms for s in stats]))
     # roofline of the dominant kernel: the finest-level red-black half sweep
-    bytes_sweep = solver.kernel_bytes(0, 0)
+    bytes_sweep = half_sweep_bytes(solver, 0)
     achieved = bytes_sweep / (sweep_ms * 1e-3) / 1e9 if sweep_ms > 0 else None
-    iso_ms = solver.time_kernel(0, 0, 20)
     plan = {"coarse_cycle_first_level_fp64": solver.info(0), "coarse_cycle_lds_bytes_fp64": solver.info(2),
             "lds_limit_per_workgroup": solver.info(4)}
     solver.close()
-    # whole-cycle algorithmic traffic (114 B per node per level: the residual on colour 0 only, 16 B,
-    # and the prolongation onto colour 1 only, 9 B; + 12 B per finest node for the colour-0 norm)
     n_levels = [((1 << (8 - l)) + 1) ** 3 for l in range(p.vcDepth + 1)]
-    cyc_bytes = 114.0 * sum(n_levels[:-1]) + 12.0 * n_levels[0]
+    cyc_bytes = cycle_bytes(n_levels)
     solve_gbs = cyc_bytes * np.mean(cycles) / (ms * 1e-3) / 1e9
 
     # mixed precision: FP32 V(2,2) cycles under FP64 iterative refinement, same stop rule
@@ -873,12 +873,11 @@ def main():
                    "cycles_per_solve": int(np.median(cycles)), "final_rel_residual": res, "converged": conv,
                    "solve_GBs_algorithmic": round(solve_gbs, 1), "mixed_precision": mixed,
                    "gcr_mixed_precision": gcr, "plan": plan},
-        "roofline": {"bound": "hbm", "kernel": "k_rb_sweep<double> finest level",
+        "roofline": {"bound": "hbm", "kernel": "k_rb_pass<double> finest level, per half sweep",
                      "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
-                     "traffic": TRAFFIC_BYTES.get("k_rb_sweep<double> 257x257x257"),
-                     "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5),
-                     "avg_launch_ms_isolated": round(iso_ms, 5)},
+                     "traffic": None,
+                     "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5)},
         "cpu_baseline": cpu,
     }
     print(json.dumps(out))
