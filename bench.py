@@ -217,8 +217,8 @@ def tgv_bench(args):
     # the step kernels one by one (HIP events on the handle's stream) against their algorithmic
     # bytes; timed after the stepped state was read, since they overwrite what they write
     kernels = {}
-    for kid, name in ((0, "k_build_rhs"), (1, "k_jacobi_v (Vx)"), (2, "k_jacobi_res (Vx)"),
-                      (6, "k_jacobi_vres (Vx: sweep + residual of its input)"), (3, "k_divergence"),
+    for kid, name in ((0, "k_build_rhs"), (1, "k_jacobi_march (Vx: sweep)"), (2, "k_jacobi_res (Vx)"),
+                      (6, "k_jacobi_march (Vx: sweep + residual of its input)"), (3, "k_divergence"),
                       (4, "k_project x3"), (5, "k_energy")):
         kms = h.time_kernel(kid, reps=20)
         kb = h.kernel_bytes(kid)
