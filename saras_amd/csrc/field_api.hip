@@ -730,7 +730,7 @@ extern "C" int sr_bc_fill(sr_fgrid *g, int loc, const sr_bc *bc, double *F) {
     if (!bc || !F) return set_err(SR_ERR_ARG, "null argument");
     std::vector<GhostWave> ws;
     RETCHK(bc_waves(g, g->shape[loc], bc, ws));
-    for (const GhostWave &w : ws) ts_ghost_wave(g->shape[loc], F, w, g->s);
+    ts_ghost_waves(g->shape[loc], F, ws.data(), (int)ws.size(), g->s);
     HIPCHK(hipGetLastError());
     return SR_OK;
 }

@@ -102,7 +102,7 @@ static std::vector<GhostWave> vbc_waves(const sr_ts_desc &d, const FShape &f, in
 }
 
 static void impose_vbc(sr_ts *t, int c) {
-    for (const GhostWave &w : t->vbc[c]) ts_ghost_wave(t->fv[c], t->V[c], w, t->s);
+    ts_ghost_waves(t->fv[c], t->V[c], t->vbc[c].data(), (int)t->vbc[c].size(), t->s);
 }
 
 // scalar::imposeTBCs (scalar.cc:240-255) with the walls of initTBC (scalar.cc:196-228): syncData,
@@ -133,7 +133,7 @@ static std::vector<GhostWave> tbc_waves(const sr_ts_desc &d, const FShape &f) {
 }
 
 static void impose_tbc(sr_ts *t) {
-    for (const GhostWave &w : t->tbc) ts_ghost_wave(t->fp, t->T, w, t->s);
+    ts_ghost_waves(t->fp, t->T, t->tbc.data(), (int)t->tbc.size(), t->s);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -87,6 +87,10 @@ void ts_jacobi_vres(const FShape &f, const Metrics &M, const Bulk &B, const doub
                     const JacobiCoef &J, JacobiSync *sync, unsigned long long *out, unsigned long long *host,
                     hipStream_t s);
 void ts_ghost_wave(const FShape &f, double *F, const GhostWave &W, hipStream_t s);
+// n waves in order.  Copies onto x and y pads followed by z walls (a grid without x and y walls: every
+// Taylor-Green and Rayleigh-Benard field) are one launch, 4.7 us at 129^3 (5.4 + 3.8 as two): 129^3 step
+// 2375 -> 2358 us, 257 x 257 x 129 convection step 6068 -> 5987.
+void ts_ghost_waves(const FShape &f, double *F, const GhostWave *W, int n, hipStream_t s);
 
 // The grid factors of the Jacobi solves (hydro_d3.cc:56-61: hx2hy2 = hx^2 hy^2 ...) for spacings h,
 // time step dt and Reynolds number Re (1 / Re = 0 when Re <= 0); form, vis and ms are the caller's.

@@ -6,7 +6,8 @@
 //   k_jacobi_march one Jacobi sweep of solveVx/Vy/Vz (hydro_d3.cc:375-391) into the second buffer, with
 //                  or without the residual of the current iterate from the same loads
 //   k_jacobi_res   the convergence residual of the same routines (hydro_d3.cc:396-410), max-reduced
-//   k_ghost_ops    a wave of ghost / wall operations (mpidata::syncData, lib/boundary/*.cc)
+//   k_ghost_ops    a wave of ghost / wall operations (mpidata::syncData, lib/boundary/*.cc); k_ghost_pair
+//                  syncData and the z walls in one launch
 //   k_divergence   vfield::divergence (vfield.cc:299-320), optionally scaled (mgRHS = div / dt)
 //   k_project      P += Pp and V -= dt grad Pp (hydro_d3.cc:354-362)
 //   k_energy       tseries energy (tseries.cc:158-169), deterministic two-pass sum
@@ -329,31 +330,78 @@ __global__ void __launch_bounds__(1024) k_jacobi_res_final(const double *__restr
 // ------------------------------------------------------------------------------------------------
 // ghost / wall operations: dst = a * F(src) + b over a plane (dim fixed) or a z-line (x, y fixed)
 // ------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_ghost_ops(FShape f, double *__restrict__ F, GhostWave W) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    int o = 0;
+// operation and place of thread t of a wave: destination p, source s; false past the last one
+__device__ inline bool ghost_place(const GhostWave &W, long t, int &o, int (&p)[3], int (&s)[3]) {
+    o = 0;
     while (o < W.nops && t >= W.ops[o].count) {
         t -= W.ops[o].count;
         o++;
     }
-    if (o >= W.nops) return;
+    if (o >= W.nops) return false;
     const GhostOp &op = W.ops[o];
-    int p[3], s[3];
     if (op.kind == 0) {      // plane: fixed index along op.dim, ranges on the other two
-        int a = op.dim == 0 ? 1 : 0, b = op.dim == 2 ? 1 : 2;
-        int na = op.hi[0] - op.lo[0] + 1;
-        int ia = op.lo[0] + (int)(t % na), ib = op.lo[1] + (int)(t / na);
-        p[op.dim] = op.dst[0];
-        s[op.dim] = op.src[0];
-        p[a] = s[a] = ia;
-        p[b] = s[b] = ib;
+        const int na = op.hi[0] - op.lo[0] + 1;
+        const int q = (int)((unsigned)t / (unsigned)na);
+        const int ia = op.lo[0] + (int)t - q * na, ib = op.lo[1] + q;
+        p[0] = s[0] = ia;
+        p[1] = s[1] = op.dim == 0 ? ia : ib;
+        p[2] = s[2] = ib;
+        if (op.dim == 0) { p[0] = op.dst[0]; s[0] = op.src[0]; }
+        if (op.dim == 1) { p[1] = op.dst[0]; s[1] = op.src[0]; }
+        if (op.dim == 2) { p[2] = op.dst[0]; s[2] = op.src[0]; }
     } else {                 // z-line at fixed (x, y)
-        int kk = op.lo[0] + (int)t;
-        p[0] = op.dst[0]; p[1] = op.dst[1]; p[2] = kk;
-        s[0] = op.src[0]; s[1] = op.src[1]; s[2] = kk;
+        p[2] = s[2] = op.lo[0] + (int)t;
+        p[0] = op.dst[0]; p[1] = op.dst[1];
+        s[0] = op.src[0]; s[1] = op.src[1];
     }
-    double v = op.a == 0.0 ? 0.0 : op.a * F[fidx(f, s[0], s[1], s[2])];
+    return true;
+}
+
+__global__ void __launch_bounds__(256) k_ghost_ops(FShape f, double *__restrict__ F, GhostWave W) {
+    int o, p[3], s[3];
+    if (!ghost_place(W, (long)blockIdx.x * blockDim.x + threadIdx.x, o, p, s)) return;
+    const GhostOp &op = W.ops[o];
+    const double v = op.a == 0.0 ? 0.0 : op.a * F[fidx(f, s[0], s[1], s[2])];
     F[fidx(f, p[0], p[1], p[2])] = v + op.b;
+}
+
+// Two waves in one launch: copies onto x and y pads (S) and then z walls (W).  A wall entry over a pad
+// takes its value from where S would have copied the pad from, and S leaves out the planes that W
+// writes, so that neither reads what the other writes.
+__global__ void __launch_bounds__(256) k_ghost_pair(FShape f, double *__restrict__ F, GhostWave S, GhostWave W, long ns) {
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    int o, p[3], s[3];
+    if (t < ns) {
+        ghost_place(S, t, o, p, s);
+        for (int q = 0; q < W.nops; q++)
+            if (p[2] == W.ops[q].dst[0]) return;
+        F[fidx(f, p[0], p[1], p[2])] = F[fidx(f, s[0], s[1], s[2])];
+        return;
+    }
+    if (!ghost_place(W, t - ns, o, p, s)) return;
+    const double a = W.ops[o].a, b = W.ops[o].b;
+    double v = 0.0;
+    if (a != 0.0) {
+        for (int q = 0; q < S.nops; q++) {
+            const GhostOp &c = S.ops[q];
+            if (c.kind == 1) {
+                if (s[0] == c.dst[0] && s[1] == c.dst[1] && s[2] >= c.lo[0] && s[2] <= c.hi[0]) {
+                    s[0] = c.src[0];
+                    s[1] = c.src[1];
+                    break;
+                }
+            } else {
+                const int e = c.dim == 0 ? s[1] : s[0];
+                if ((c.dim == 0 ? s[0] : s[1]) == c.dst[0] && e >= c.lo[0] && e <= c.hi[0] && s[2] >= c.lo[1] && s[2] <= c.hi[1]) {
+                    if (c.dim == 0) s[0] = c.src[0];
+                    else s[1] = c.src[0];
+                    break;
+                }
+            }
+        }
+        v = a * F[fidx(f, s[0], s[1], s[2])];
+    }
+    F[fidx(f, p[0], p[1], p[2])] = v + b;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -692,10 +740,41 @@ void ts_jacobi_vres(const FShape &f, const Metrics &M, const Bulk &B, const doub
                        with_quotients(J), sync, out, host);
 }
 
-void ts_ghost_wave(const FShape &f, double *F, const GhostWave &W, hipStream_t s) {
+static long wave_count(const GhostWave &W) {
     long n = 0;
     for (int o = 0; o < W.nops; o++) n += W.ops[o].count;
+    return n;
+}
+
+void ts_ghost_wave(const FShape &f, double *F, const GhostWave &W, hipStream_t s) {
+    const long n = wave_count(W);
     if (n > 0) hipLaunchKernelGGL(k_ghost_ops, dim3(nb(n)), dim3(256), 0, s, f, F, W);
+}
+
+// S copies within planes of z and W writes whole planes of z from planes that neither writes
+static bool ghost_pair_ok(const FShape &f, const GhostWave &S, const GhostWave &W) {
+    for (int o = 0; o < S.nops; o++)
+        if (S.ops[o].a != 1.0 || S.ops[o].b != 0.0 || (S.ops[o].kind == 0 && S.ops[o].dim == 2)) return false;
+    for (int o = 0; o < W.nops; o++) {
+        if (W.ops[o].kind != 0 || W.ops[o].dim != 2 || W.ops[o].lo[0] != -1 || W.ops[o].lo[1] != -1 ||
+            W.ops[o].hi[0] != f.n[0] || W.ops[o].hi[1] != f.n[1])
+            return false;
+        for (int q = 0; q < W.nops; q++)
+            if (W.ops[o].a != 0.0 && W.ops[o].src[0] == W.ops[q].dst[0]) return false;
+    }
+    return S.nops > 0 && W.nops > 0;
+}
+
+void ts_ghost_waves(const FShape &f, double *F, const GhostWave *W, int n, hipStream_t s) {
+    for (int w = 0; w < n; w++) {
+        if (w + 1 < n && ghost_pair_ok(f, W[w], W[w + 1])) {
+            const long ns = wave_count(W[w]), nw = wave_count(W[w + 1]);
+            if (ns + nw > 0) hipLaunchKernelGGL(k_ghost_pair, dim3(nb(ns + nw)), dim3(256), 0, s, f, F, W[w], W[w + 1], ns);
+            w++;
+        } else {
+            ts_ghost_wave(f, F, W[w], s);
+        }
+    }
 }
 
 JacobiCoef jacobi_coef(const double h[3], double dt, double Re) {
@@ -741,12 +820,12 @@ int ts_jacobi_loop(const FShape &f, const Metrics &M, const Bulk &B, double *&F,
     int n = 0;
     ts_jacobi(f, M, B, F, R, G, J, io.s);
     std::swap(F, G);
-    for (int w = 0; w < nbc; w++) ts_ghost_wave(f, F, bc[w], io.s);
+    ts_ghost_waves(f, F, bc, nbc, io.s);
     int status = 0;
     while (true) {
         ts_jacobi_vres(f, M, B, F, R, G, J, io.sync, io.dmax, io.hmax, io.s);
         JCHK(hipEventRecord(io.ev, io.s));
-        for (int w = 0; w < nbc; w++) ts_ghost_wave(f, G, bc[w], io.s);
+        ts_ghost_waves(f, G, bc, nbc, io.s);
         JCHK(hipGetLastError());
         JCHK(hipEventSynchronize(io.ev));
         double maxError;

@@ -12,10 +12,11 @@ pytestmark = pytest.mark.gpu
 RTOL = 1e-12
 
 GRIDS = {
-    # 2 and 3 planes per chunk, 4 and 5, 1, 1 and 2
+    # several planes per chunk, unevenly, and one; z periodic, with walls and walls all round
     "65x129x129": dict(ind=(6, 7, 7), L=(1.0, 2.0, 2.0), domain="PPN", mesh="UUD", beta=(1.0, 1.0, 1.2)),
     "129x129x129": dict(ind=(7, 7, 7), L=(1.0, 1.0, 1.0), domain="NNN", mesh="DDD", beta=(1.1, 0.7, 1.3)),
     "33x5x17": dict(ind=(5, 2, 4), L=(1.0, 2.0, 1.5), domain="NPP", mesh="DUU", beta=(1.1, 1.0, 1.0)),
+    "65x33x65": dict(ind=(6, 5, 6), L=(2.0, 1.0, 2.0), domain="PPP", mesh="UUU"),
     "257x17x129": dict(ind=(8, 4, 7), L=(1.0, 1.0, 1.0), domain="PNP", mesh="UDU", beta=(1.0, 0.7, 1.0)),
 }
 
@@ -130,4 +131,31 @@ def test_outputs_that_share_memory():
         fg.sync()
         _close(buf.download(), expect(step), "shared outputs")
     fg.close()
+    o.close()
+
+
+@pytest.mark.parametrize("grid", list(GRIDS))
+def test_jacobi_solves(grid):
+    """Same sweeps and fields as the oracle where a chunk of a sweep holds several planes, with the pads and
+    the z walls filled in one launch (no x and y walls) and in several."""
+    from saras_amd import ts
+    kw = dict(GRIDS[grid], dt=1e-3, Re=200.0)
+    o, g = po.OracleTS(po.ts_params(**kw)), ts.Hydro(ts.ts_desc(**kw))
+    rng = np.random.default_rng(4)
+    for c in range(3):
+        a = o.array(c)
+        a[...] = 0.1 * rng.standard_normal(a.shape)
+        g.upload(c, a)
+        o.impose_vbc(c)
+        g.imposeVBC(c)
+        assert np.array_equal(g.download(c), a), c
+    P = o.array(po.PRES)
+    P[...] = 0.0
+    g.upload(ts.P, P)
+    o.build_rhs()
+    g.buildRHS()
+    for c in range(3):
+        assert o.solve_v(c) == g.solveV(c), c
+        _close(g.download(c), o.array(c), f"V{c}")
+    g.close()
     o.close()
