@@ -553,7 +553,7 @@ static int fgrid_create_impl(const sr_fgrid_desc *desc, sr_fgrid *g) {
     HIPCHK(hipEventCreateWithFlags(&g->jev, hipEventDisableTiming));
     HIPCHK(hipMalloc((void **)&g->dmax, sizeof(unsigned long long)));
     HIPCHK(hipMalloc((void **)&g->jsync, sizeof(JacobiSync)));
-    HIPCHK(hipMemset(g->jsync, 0, sizeof(JacobiSync)));
+    HIPCHK(hipMemsetAsync(g->jsync, 0, sizeof(JacobiSync), g->s));
     HIPCHK(hipHostMalloc((void **)&g->hmax, sizeof(unsigned long long), hipHostMallocDefault));
     return SR_OK;
 }

@@ -261,7 +261,7 @@ static int create_impl(const sr_ts_desc *desc, sr_ts *t) {
     HIPCHK(hipHostMalloc((void **)&t->hred, sizeof(double) * 4, hipHostMallocDefault));
     HIPCHK(hipMalloc((void **)&t->dmax, sizeof(unsigned long long)));
     HIPCHK(hipMalloc((void **)&t->jsync, sizeof(JacobiSync)));
-    HIPCHK(hipMemset(t->jsync, 0, sizeof(JacobiSync)));
+    HIPCHK(hipMemsetAsync(t->jsync, 0, sizeof(JacobiSync), t->s));
     HIPCHK(hipHostMalloc((void **)&t->hmax, sizeof(unsigned long long), hipHostMallocDefault));
     for (int c = 0; c < 3; c++) {
         t->vbc[c] = vbc_waves(d, t->fv[c], c);
