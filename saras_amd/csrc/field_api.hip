@@ -441,18 +441,19 @@ ColMet col_met(const sr_fgrid *g) {
     return ColMet{{1.0 / g->h[0], 1.0 / g->h[1], 1.0 / g->h[2]}, g->half};
 }
 VelGeo vel_geo(const sr_fgrid *g) { return VelGeo{{g->N[0], g->N[1], g->N[2]}}; }
-// Whether the components' outputs H can be written by one launch that reads the inputs U: no output shares
-// memory with another one or with another component's input.  A caller may let them (the components are
-// then done in order, as if one by one).
-bool one_launch(const sr_fgrid *g, double *const H[3], const double *const *U) {
-    auto apart = [&](const double *a, int la, const double *b, int lb) {
-        return a + fsz(g->shape[la]) <= b || b + fsz(g->shape[lb]) <= a;
+// Whether the components' outputs H can be written by one launch that reads the inputs U (one for each
+// component) and V (all of them for every component): no output shares memory with another one, with
+// another component's U or with a V.  A caller may let them (the components are then done in order, as
+// if one by one, each reading what the ones before it left).
+bool one_launch(const sr_fgrid *g, double *const H[3], const double *const *U, const double *const *V = nullptr) {
+    auto apart = [&](const double *a, int c, const double *b, int e) {
+        return a + fsz(g->shape[SR_LOC_VX + c]) <= b || b + fsz(g->shape[SR_LOC_VX + e]) <= a;
     };
     for (int c = 0; c < 3; c++)
-        for (int e = 0; e < 3; e++)
-            if (e != c && (!apart(H[c], SR_LOC_VX + c, H[e], SR_LOC_VX + e) ||
-                           (U && !apart(H[c], SR_LOC_VX + c, U[e], SR_LOC_VX + e))))
-                return false;
+        for (int e = 0; e < 3; e++) {
+            if (V && !apart(H[c], c, V[e], e)) return false;
+            if (e != c && (!apart(H[c], c, H[e], e) || (U && !apart(H[c], c, U[e], e)))) return false;
+        }
     return true;
 }
 ColGeo node_geo(const sr_fgrid *g, int planes) { return col_geo(vel_geo(g).sx(), planes); }
@@ -679,7 +680,7 @@ extern "C" int sr_vf_nlin(sr_fgrid *g, const double *Ux, const double *Uy, const
         if (!U[c] || !V[c] || !H[c]) return set_err(SR_ERR_ARG, "null array");
     const ColGeo G = node_geo(g, g->N[0]);
     const bool self = Ux == Vx && Uy == Vy && Uz == Vz;
-    for (int part = 0, one = one_launch(g, H, nullptr); part < (one ? 1 : 3); part++)
+    for (int part = 0, one = one_launch(g, H, U, V); part < (one ? 1 : 3); part++)
         hipLaunchKernelGGL((self ? k_fd_nlin<true> : k_fd_nlin<false>), dim3(col_blocks(G)), dim3(kColThreads), 0, g->s, G,
                            vel_geo(g), g->M, Ux, Uy, Uz, Vx, Vy, Vz, Hx, Hy, Hz, col_met(g), one ? 7 : 1 << part);
     HIPCHK(hipGetLastError());

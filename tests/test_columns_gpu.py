@@ -134,6 +134,50 @@ def test_outputs_that_share_memory():
     o.close()
 
 
+# an output (component) that lies over part of an input: (output, input list, its component, planes between
+# the start of the first of the two and of the second).  Over another component's U anywhere; over Vx only
+# its plane before the first core one, which component x does not read.
+OVERLAPS = [("x", "U", "y", 3), ("z", "U", "x", 2), ("y", "U", "z", -4), ("x", "V", "x", None)]
+
+
+@pytest.mark.parametrize("case", OVERLAPS, ids=str)
+def test_nlin_output_over_part_of_an_input(case):
+    """The components are done in order, each reading what the ones before it left in memory."""
+    from saras_amd import _lib
+    out, which, comp, planes = "xyz".index(case[0]), case[1], "xyz".index(case[2]), case[3]
+    o, fg = _pair("33x5x17")
+    rng = np.random.default_rng(5)
+    shape = [o.loc_shape(c) for c in (1, 2, 3)]
+    A = {n: [rng.standard_normal(s) for s in shape] for n in "UVH"}
+    D = {n: [fg.array(c + 1, A[n][c]) for c in range(3)] for n in "UVH"}
+    if planes is None:
+        planes = shape[out][0] - 2   # the output's last core plane on the input's first plane
+    step = abs(planes) * int(np.prod(shape[out][1:]))
+    first = [("H", out), (which, comp)] if planes > 0 else [(which, comp), ("H", out)]
+    sizes = [int(np.prod(shape[c])) for _, c in first]
+    flat = rng.standard_normal(max(sizes[0], step + sizes[1]))
+    buf = _lib.DeviceArray(flat.shape)
+    buf.upload(flat)
+
+    class Part:
+        pass
+
+    for (name, c), at, n in zip(first, (0, step), sizes):
+        A[name][c] = flat[at:at + n].reshape(shape[c])
+        D[name][c] = Part()
+        D[name][c].ptr = buf.ptr + 8 * at
+    fg.vfComputeNLin(D["U"], D["V"], D["H"])
+    fg.sync()
+    for c in range(3):
+        o.fd_nlin(c + 1, A["U"][c], A["V"], A["H"][c])
+    _close(buf.download(), flat, case)
+    for c in range(3):
+        if c != out:
+            _close(D["H"][c].download(), A["H"][c], (case, c))
+    fg.close()
+    o.close()
+
+
 @pytest.mark.parametrize("grid", list(GRIDS))
 def test_jacobi_solves(grid):
     """Same sweeps and fields as the oracle where a chunk of a sweep holds several planes, with the pads and
