@@ -34,8 +34,9 @@ static void read_back(sr_mg *m) {
     if (e != hipSuccess && m->body_err == hipSuccess) m->body_err = e;
 }
 
-// before every cycle: the host mirror holds NaN until the cycle's read-back lands, so a read-back
-// that did not happen shows as a solve that never meets its stop rule, not as a stale norm
+// before every cycle and every norm of a guess: the host mirror holds NaN until the read-back, or the
+// kernel's own write, lands, so that one that did not happen shows as a solve that never meets its stop
+// rule, not as a stale norm
 static void poison_hres(sr_mg *m) {
     for (int i = 0; i < 4; i++) m->hres[i] = std::nan("");
 }
@@ -244,6 +245,7 @@ static int solve_mixed(sr_mg *m, int &cycles, double &res, bool &conv, double &s
     RETCHK(ensure_fp32(m));
     Level &V = m->lv[0];
     long sz = lay_size(V.L);
+    poison_hres(m);
     if (march0(m)) {
         march_step(m, V.u, nullptr, nullptr, nullptr, nullptr, V.f32);
         HIPCHK(hipGetLastError());
@@ -351,6 +353,7 @@ static int solve_gcr(sr_mg *m, int &cycles, double &res, bool &conv, double &swe
         HIPCHK(hipMemcpyAsync(V.t, V.u, sizeof(double) * sz, hipMemcpyDeviceToDevice, s));
     // no previous direction: the first step is the minimal-residual step along the cycle's result
     launch_fill<float>(m->zdir[0], sz, 0.0f, s);
+    poison_hres(m);
     if (march) {
         march_step(m, V.u, nullptr, nullptr, nullptr, nullptr, V.f32);
         HIPCHK(hipGetLastError());

@@ -1,0 +1,68 @@
+"""The library's host code over a HIP runtime whose kernels do nothing (fake_hip.cc).  CPU only."""
+import concurrent.futures as cf
+import ctypes as C
+import os
+import re
+import subprocess
+
+import numpy as np
+import pytest
+
+from saras_amd import _lib, build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host"))
+    obj = [os.path.join(out, s + ".o") for s in build.HIP_SOURCES]
+
+    def compile_one(s, o):
+        subprocess.run([build.HIPCC, f"--offload-arch={build.ARCH}", "--offload-host-only", "-O1", "-std=c++17", "-fPIC",
+                        "-w", "-c", os.path.join(build.CSRC, s), "-o", o], check=True, capture_output=True)
+
+    with cf.ThreadPoolExecutor(max_workers=8) as ex:
+        list(ex.map(compile_one, build.HIP_SOURCES, obj))
+    # the device code, which there is none of
+    names = subprocess.run(["nm", "-u", *obj], check=True, capture_output=True, text=True).stdout
+    none = [f"-Wl,--defsym={s}=0" for s in sorted(set(re.findall(r"__hip_fatbin\w*", names)))]
+    so = os.path.join(out, "libhost.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wl,-Bsymbolic", "-o", so, *obj,
+                    *[os.path.join(build.CSRC, s) for s in build.CPP_SOURCES], os.path.join(HERE, "fake_hip.cc"), *none],
+                   check=True, capture_output=True)
+    return so
+
+
+@pytest.fixture
+def fake(library, monkeypatch):
+    """The package on that library, and the fake runtime's own calls."""
+    monkeypatch.setattr(_lib, "LIB_PATH", library)
+    monkeypatch.setattr(_lib, "_lib", None)
+    L = _lib.load()
+    L.fake_launched.restype = C.c_char_p
+    L.fake_clear()
+    L.fake_refuse_lds(0)
+    yield L
+    L.fake_refuse_lds(0)
+
+
+def _launched(L):
+    return L.fake_launched().decode().split("\n")[:-1]
+
+
+def _problem(**kw):
+    from helpers import Problem
+    return Problem(**{**dict(ind=(4, 4, 4), domain="PPN", mesh="UUD", vc_count=3), **kw})
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["fp64", "refinement", "gcr"])
+def test_a_solve_whose_residuals_never_arrive_does_not_converge(fake, precision):
+    """The host's mirror of the residual holds zeros here, which would pass any stop rule."""
+    pb = _problem()
+    g = pb.gpu(precision=precision)
+    st = g.mgSolve(np.zeros(pb.shape), pb.random_rhs(0))
+    assert not st.converged and st.cycles == pb.vc_count and not st.residual == st.residual
+    if precision:
+        assert not st.residual0 == st.residual0
+    g.close()
