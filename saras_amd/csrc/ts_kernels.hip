@@ -823,13 +823,16 @@ int ts_jacobi_loop(const FShape &f, const Metrics &M, const Bulk &B, double *&F,
     ts_ghost_waves(f, F, bc, nbc, io.s);
     int status = 0;
     while (true) {
+        // not a maximum of absolute values: what is left here if the kernel's write does not land
+        *io.hmax = ~0ull;
         ts_jacobi_vres(f, M, B, F, R, G, J, io.sync, io.dmax, io.hmax, io.s);
         JCHK(hipEventRecord(io.ev, io.s));
         ts_ghost_waves(f, G, bc, nbc, io.s);
         JCHK(hipGetLastError());
         JCHK(hipEventSynchronize(io.ev));
         double maxError;
-        unsigned long long bits = *io.hmax;
+        const unsigned long long bits = *(volatile unsigned long long *)io.hmax;
+        if (bits == ~0ull) JCHK(hipErrorUnknown);
         std::memcpy(&maxError, &bits, sizeof(double));
         n += 1;
         if (maxError < tol) break;

@@ -66,3 +66,15 @@ def test_a_solve_whose_residuals_never_arrive_does_not_converge(fake, precision)
     if precision:
         assert not st.residual0 == st.residual0
     g.close()
+
+
+def test_a_viscous_solve_whose_residuals_never_arrive_fails(fake):
+    from saras_amd import field
+    fg = field.FieldGrid(field.fgrid_desc(ind=(3, 3, 3), domain="PPN"))
+    F, G, R = (fg.array(1) for _ in range(3))
+    P, D = field.PERIODIC, field.DIRICHLET
+    with pytest.raises(_lib.SarasError):
+        fg.jacobi(1, 0, 1e-3, field.bc([P, P, P, P, D, D]), R, F, G, Re=100.0)
+    for a in (F, G, R):
+        a.free()
+    fg.close()
