@@ -308,7 +308,9 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
         for (int q = 0; q < 2; q++) launch_fill<float>(m->zdir[q], sz, 0.0f, m->stream);
     }
     if (d->coarseDirect) RETCHK(build_coarse_direct(m));
-    if (rb_pass_attr() || march_outer_attr()) return set_err(SR_ERR_HIP, "LDS size of the sweep kernels refused");
+    // without the LDS that the marching kernels ask for, every level keeps the per-node ones
+    m->march_off = rb_pass_attr() || march_outer_attr();
+    if (m->march_off) (void)hipGetLastError();
     // coarse end of the cycle in LDS
     {
         int dev = 0, lds_max = 65536;
@@ -321,13 +323,19 @@ static int create_impl(const sr_mg_desc *d, sr_mg *m) {
             if (m->coarse_first64 <= depth) {
                 finish_coarse(m, m->cdesc64, false);
                 RETCHK(upload_coarse_coef<double>(m, m->cdesc64, m->ccoef64));
-                if (coarse_cycle_attr<double>(m->clds64)) m->coarse_first64 = 1 << 20;
+                if (coarse_cycle_attr<double>(m->clds64)) {
+                    m->coarse_first64 = 1 << 20;
+                    (void)hipGetLastError();
+                }
             }
             plan_coarse<float>(m, m->coarse_first32, m->cdesc32, m->clds32, limit);
             if (m->coarse_first32 <= depth) {
                 finish_coarse(m, m->cdesc32, true);
                 RETCHK(upload_coarse_coef<float>(m, m->cdesc32, m->ccoef32));
-                if (coarse_cycle_attr<float>(m->clds32)) m->coarse_first32 = 1 << 20;
+                if (coarse_cycle_attr<float>(m->clds32)) {
+                    m->coarse_first32 = 1 << 20;
+                    (void)hipGetLastError();
+                }
             }
         }
         (void)hipGetLastError();
@@ -496,8 +504,8 @@ void sr::mark(sr_mg *m, hipEvent_t e) {
 // Whether a smoothing of `count` red-black sweeps runs as one-launch sweeps (launch_rb_pass) that need
 // no ghosts beforehand.  They hand colour 1 back and forth between u and a second buffer and have to
 // end in u: any count from zero, even counts otherwise.
-static bool passes_ok(const Lay &L, const Bc &bc, int count, bool zero_start) {
-    return count > 0 && (zero_start || count % 2 == 0) && rb_pass_ok(L, bc);
+static bool passes_ok(const sr_mg *m, const Lay &L, const Bc &bc, int count, bool zero_start) {
+    return !m->march_off && count > 0 && (zero_start || count % 2 == 0) && rb_pass_ok(L, bc);
 }
 
 template <typename T>
@@ -517,7 +525,7 @@ void sr::smooth_level(sr_mg *m, int l, int count, int zeroBC, bool zero_start, b
     Level &V = m->lv[l];
     Bc bc = pressure_bc(m, l, zeroBC);
     hipStream_t s = m->stream;
-    if (m->d.gsSmooth && !exact && !first_done && passes_ok(V.L, bc, count, zero_start)) {
+    if (m->d.gsSmooth && !exact && !first_done && passes_ok(m, V.L, bc, count, zero_start)) {
         // colour 1 of tmp is free: the residual after pre-smoothing is formed on colour 0
         if (ea) mark(m, ea);
         smooth_passes<double>(V.L, V.u, V.t, V.f, V.c64, bc, count, zero_start, s);
@@ -597,7 +605,7 @@ void sr::vcycle_fp64(sr_mg *m) {
         // u: the restriction that makes its right-hand side does it (ZeroStart)
         Level &Nx = m->lv[l + 1];
         const bool fuse = d.gsSmooth && d.preSmooth > 0 && l + 1 != Lc && l + 1 != D &&
-                          !passes_ok(Nx.L, pressure_bc(m, l + 1, 1), d.preSmooth, true);
+                          !passes_ok(m, Nx.L, pressure_bc(m, l + 1, 1), d.preSmooth, true);
         const ZeroStart<double> zs{Nx.u, Nx.c64[0], Nx.c64[1], Nx.c64[2], pressure_bc(m, l + 1, 1)};
         launch_restrict<double>(m->lv[l].L, Nx.L, m->lv[l].t, Nx.f, m->stream, red0, fuse ? &zs : nullptr);
         if (l + 1 == Lc) {
@@ -621,7 +629,7 @@ void sr::vcycle_fp64(sr_mg *m) {
     // the separate fill (measured faster there)
     for (int l = bottom - 1; l >= 0; l--) {
         const Bc bc = pressure_bc(m, l, 1);
-        const bool img = l > 0 && d.gsSmooth && !passes_ok(m->lv[l].L, bc, d.postSmooth, false);
+        const bool img = l > 0 && d.gsSmooth && !passes_ok(m, m->lv[l].L, bc, d.postSmooth, false);
         launch_prolong<double, double>(m->lv[l].L, m->lv[l + 1].L, m->lv[l + 1].u, m->lv[l].u, 1, m->stream, pcol,
                                        img ? &bc : nullptr);
         smooth_level(m, l, d.postSmooth, l == 0 ? 0 : 1, false, false, nullptr, nullptr, img);
@@ -645,7 +653,7 @@ static void smooth32(sr_mg *m, int l, int count, int zeroBC, bool zero_start, hi
     bool wall = bc.rule[0] == G_WALL || bc.rule[1] == G_WALL || bc.rule[2] == G_WALL;
     bool zs = zero_start && !wall;
     hipStream_t s = m->stream;
-    if (!first_done && passes_ok(V.L, bc, count, zs)) {
+    if (!first_done && passes_ok(m, V.L, bc, count, zs)) {
         if (ea) mark(m, ea);
         smooth_passes<float>(V.L, V.u32, V.t32, V.f32, V.c32, bc, count, zs, s);
         if (eb) mark(m, eb);
@@ -689,7 +697,7 @@ void sr::vcycle_fp32(sr_mg *m) {
         const Bc nb = error_bc(m, l + 1, 1);
         const bool nwall = nb.rule[0] == G_WALL || nb.rule[1] == G_WALL || nb.rule[2] == G_WALL;
         const bool fuse = m->pre32 > 0 && !nwall && l + 1 != Lc && l + 1 != D &&
-                          !passes_ok(Nx.L, nb, m->pre32, true);
+                          !passes_ok(m, Nx.L, nb, m->pre32, true);
         const ZeroStart<float> zs{Nx.u32, Nx.c32[0], Nx.c32[1], Nx.c32[2], nb};
         launch_restrict<float>(V.L, Nx.L, V.t32, Nx.f32, s, red0, fuse ? &zs : nullptr);
         if (l + 1 == Lc) {
@@ -715,7 +723,7 @@ void sr::vcycle_fp32(sr_mg *m) {
     // post-smoothing starts without a ghost fill (as in the FP64 cycle)
     for (int l = bottom - 1; l >= 0; l--) {
         const Bc bc = error_bc(m, l, 1);
-        const bool img = l > 0 && !passes_ok(m->lv[l].L, bc, m->post32, false);
+        const bool img = l > 0 && !passes_ok(m, m->lv[l].L, bc, m->post32, false);
         launch_prolong<float, float>(m->lv[l].L, m->lv[l + 1].L, m->lv[l + 1].u32, m->lv[l].u32, 1, s, pcol,
                                      img ? &bc : nullptr);
         smooth32(m, l, m->post32, l == 0 ? 0 : 1, false, nullptr, nullptr, img);

@@ -95,7 +95,7 @@ static int norm_order(const sr_mg *m) {
 
 // Whether level 0 takes the marching kernels (mg_outer.hip), which leave the reduced quantities in the
 // host mirror themselves.
-static bool march0(const sr_mg *m) { return march_outer_ok(m->lv[0].L, pressure_bc(m, 0, 0)); }
+static bool march0(const sr_mg *m) { return !m->march_off && march_outer_ok(m->lv[0].L, pressure_bc(m, 0, 0)); }
 
 // One outer step as a march: from x_in, with e (refinement) or e and z (GCR) into x_out; without r32 the
 // norms of f - L x_in alone.

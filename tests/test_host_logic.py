@@ -78,3 +78,18 @@ def test_a_viscous_solve_whose_residuals_never_arrive_fails(fake):
     for a in (F, G, R):
         a.free()
     fg.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2], ids=["fp64", "refinement", "gcr"])
+def test_without_large_lds_a_solver_runs_the_per_node_kernels(fake, precision):
+    big = ("k_rb_pass", "k_march", "k_coarse_cycle")
+    pb = _problem()
+    for refused in (0, 1):
+        fake.fake_refuse_lds(refused)
+        g = pb.gpu(precision=precision)
+        fake.fake_clear()
+        g.vCycle()
+        g.mgSolve(np.zeros(pb.shape), pb.random_rhs(0))
+        ran = {b for b in big for name in _launched(fake) if b in name}
+        assert ran == (set() if refused else set(big)), (refused, ran)
+        g.close()
