@@ -407,15 +407,12 @@ extern "C" int sr_mg_residual(sr_mg *m, const double *p, const double *rhs, doub
     if (!m || !p || !rhs) return set_err(SR_ERR_ARG, "null argument");
     Level &V = m->lv[0];
     load_level0(m, rhs, p);
-    const bool march = march0(m);
-    if (r || !march) launch_fill_ghosts<double>(V.L, V.u, pressure_bc(m, 0, 0), m->stream);
-    if (march) {
-        poison_hres(m);
-        march_step(m, V.u, nullptr, nullptr, nullptr, nullptr, nullptr);
-    } else {
-        norm_level0(m);
-        HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, m->stream));
-    }
+    // Per-node norm: the arrays were just loaded and the last-level cache holds all but the largest, where
+    // the march of the solves is slower (us per call, per-node against march: 33 x 65 x 257 nodes 55 / 63,
+    // 65 x 257 x 513 167 / 189, 257 x 257 x 129 148 / 156; 257^3 313 / 297); and the guess keeps its ghosts.
+    launch_fill_ghosts<double>(V.L, V.u, pressure_bc(m, 0, 0), m->stream);
+    norm_level0(m);
+    HIPCHK(hipMemcpyAsync(m->hres, m->dres, sizeof(double) * 4, hipMemcpyDeviceToHost, m->stream));
     if (r) {
         residual_level(m, 0);
         launch_unpack<double, double>(V.L, V.t, r, m->stream);

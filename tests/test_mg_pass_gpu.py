@@ -151,3 +151,24 @@ def test_residual_norms_match_oracle(case, precision):
         assert hist[0] <= g.history()[0] * (1 + 1e-5)
         assert np.all(hist[1:] <= hist[:-1] * (1 + 1e-5)), hist
         g.close()
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[3], CASES[5]], ids=str)
+def test_residual_leaves_the_guess_with_its_ghosts(case):
+    """sr_mg_residual without the residual field leaves level 0 as with it: the operators go on from there."""
+    from saras_amd import _lib
+    pb = _problem(*case)
+    g = pb.gpu()
+    p, f, r = (_lib.DeviceArray(pb.shape) for _ in range(3))
+    p.upload(pb.random_rhs(6))
+    f.upload(pb.random_rhs(5))
+    state = []
+    for out in (r.ptr, None):
+        g.residual_device(p.ptr, f.ptr, out)
+        guess = g.download(po.P, 0)
+        g.computeResidual()
+        state.append((guess, g.download(po.T, 0)))
+    for a, b in zip(*state):
+        assert np.array_equal(a, b)
+    assert np.array_equal(state[0][1][1:-1, 1:-1, 1:-1], r.download()[1:-1, 1:-1, 1:-1])
+    g.close()
