@@ -18,37 +18,57 @@
 namespace sr {
 
 constexpr int kColThreads = 256;
-// workgroups of a number of columns per plane, chunks of planes, planes per chunk (quotient, remainder)
+// Workgroups per plane, chunks of planes, planes per chunk (quotient, remainder), and whether the
+// workgroups of a chunk follow each other (by_chunk) or the chunks of a plane's part.
 struct ColGeo {
-    int nb, nch, cq, cr;
+    int nb, nch, cq, cr, by_chunk;
 };
 constexpr int kColPlanes = 64;   // most planes of a chunk
 // Planes whose loads are issued together; 257^3 operators with 2 and 4: 1562 and 1580 us.
 constexpr int kColAhead = 2;
 
-// Eight workgroups per CU where the planes suffice, and at most kColPlanes planes each.  The 257^3
-// operators with 1024 / 2048 / 4096 / 8192 / 16384 workgroups: 1611 / 1586 / 1571 / 1590 / 1683 us.
-inline ColGeo col_geo(long plane, int planes, int threads = kColThreads) {
+// Padded planes of `rows` rows of `row` entries.  Eight workgroups per CU where the planes suffice, and at
+// most kColPlanes planes each: the 257^3 operators with 1024 / 2048 / 4096 / 8192 / 16384 workgroups take
+// 1611 / 1586 / 1571 / 1590 / 1683 us.  Short chunks hold an even number of planes where two are loaded
+// together (ahead), as the last of an odd one leaves half of the loads unused (129^3: second derivatives
+// 9.1 -> 8.7 us, one thread per entry 9.8; not with 1024 threads, of which two workgroups fill a CU: a
+// Jacobi sweep 14.2 -> 16.6), and one plane only while that makes at most four workgroups per CU
+// (257 x 5 x 257: advection of a node field 8.1 us with one plane, 6.5 with two; one thread per entry 6.0).
+//
+// Each XCD takes a contiguous eighth of the workgroups.  With the chunks of a plane's part after each
+// other that is an eighth of the rows, whose neighbour rows belong to others: on 513 x 9 x 513 nodes one
+// row and its two neighbours, and a node field's advection took 31.9 us, 23.8 with one thread per entry.
+// There the workgroups of a chunk follow each other, an eighth of the planes per XCD: 21.6 us; 513 x 65 x
+// 257 88.4 against 93.5.  From 16 rows per XCD on the first order is as good or better (129^3 20.0 / 20.4,
+// 257^3 operators 1537 / 1562).
+inline ColGeo col_geo(int rows, int row, int planes, int threads = kColThreads, int ahead = kColAhead) {
+    const int scale = threads / kColThreads;
     ColGeo G;
-    G.nb = (int)((plane + threads - 1) / threads);
-    int nch = 2048 * 256 / threads / G.nb;
-    if (nch < (planes + kColPlanes - 1) / kColPlanes) nch = (planes + kColPlanes - 1) / kColPlanes;
-    if (nch > planes) nch = planes;
-    G.nch = nch;
-    G.cq = planes / nch;
-    G.cr = planes % nch;
+    G.nb = (int)(((long)rows * row + threads - 1) / threads);
+    G.nch = max(1, min(2048 / scale / G.nb, planes));
+    const int len = (planes + G.nch - 1) / G.nch;
+    if (planes < 2 * G.nch) {
+        if ((long)G.nb * planes > 1024 / scale) G.nch = (planes + 1) / 2;
+    } else if (scale == 1 && len < 8 && len % ahead) {
+        const int even = (planes + len - 2) / (len - 1);
+        if ((long)G.nb * even <= 2304) G.nch = even;
+    }
+    G.nch = max(G.nch, (planes + kColPlanes - 1) / kColPlanes);
+    G.cq = planes / G.nch;
+    G.cr = planes % G.nch;
+    G.by_chunk = rows < 130 && planes > rows;
     return G;
 }
 inline unsigned col_blocks(const ColGeo &G) { return (unsigned)(G.nb * G.nch); }
 
-// the thread's entry of the padded plane and the planes of its chunk, counted from 0; the chunks of a
-// plane's part follow each other (part after part of one chunk instead: 1562 against 1537 us)
+// the thread's entry of the padded plane and the planes of its chunk, counted from 0
 struct Col {
     unsigned t;
     int i0, i1;
 };
 __device__ inline Col column(const ColGeo &G) {
-    const unsigned b = xcd_block(), tile = b / (unsigned)G.nch, chunk = b - tile * (unsigned)G.nch;
+    const unsigned b = xcd_block(), inner = (unsigned)(G.by_chunk ? G.nb : G.nch), q = b / inner, r = b - q * inner;
+    const unsigned tile = G.by_chunk ? r : q, chunk = G.by_chunk ? q : r;
     Col C;
     C.t = tile * blockDim.x + threadIdx.x;
     C.i0 = (int)chunk * G.cq + min((int)chunk, G.cr);

@@ -676,7 +676,7 @@ static ColMet col_met(const double *h) { return ColMet{{1.0 / h[0], 1.0 / h[1], 
 void ts_build_rhs(const FShape &fp, const Metrics &M, const double *const *V, const double *P, double *const *H,
                   const double *h, double visc, double dt, const double *T, double Fb, hipStream_t s) {
     const VelGeo S{{fp.n[0], fp.n[1], fp.n[2]}};
-    const ColGeo G = col_geo(S.sx(), fp.n[0]);
+    const ColGeo G = col_geo(fp.n[1] + 2, fp.n[2] + 2, fp.n[0]);
     hipLaunchKernelGGL((T ? k_build_rhs<true> : k_build_rhs<false>), dim3(col_blocks(G)), dim3(kColThreads), 0, s, G, S, M, V[0],
                        V[1], V[2], P, H[0], H[1], H[2], col_met(h), visc, dt, T, Fb);
 }
@@ -684,7 +684,7 @@ void ts_build_rhs(const FShape &fp, const Metrics &M, const double *const *V, co
 void ts_build_trhs(const FShape &fp, const Metrics &M, const double *const *V, const double *T, double *R,
                    const double *h, double kappa, double dt, hipStream_t s) {
     const VelGeo S{{fp.n[0], fp.n[1], fp.n[2]}};
-    const ColGeo G = col_geo(S.sx(), fp.n[0] + 2);
+    const ColGeo G = col_geo(fp.n[1] + 2, fp.n[2] + 2, fp.n[0] + 2);
     hipLaunchKernelGGL(k_build_trhs, dim3(col_blocks(G)), dim3(kColThreads), 0, s, G, S, M, V[0], V[1], V[2], T, R, col_met(h),
                        kappa, dt);
 }
@@ -715,7 +715,7 @@ static JacobiCoef with_quotients(JacobiCoef J) {
 
 void ts_jacobi(const FShape &f, const Metrics &M, const Bulk &B, const double *V, const double *R, double *G,
                const JacobiCoef &J, hipStream_t s) {
-    const ColGeo C = col_geo((long)(f.n[1] + 2) * (f.n[2] + 2), f.n[0] + 2, kJacobiThreads);
+    const ColGeo C = col_geo(f.n[1] + 2, f.n[2] + 2, f.n[0] + 2, kJacobiThreads);
     hipLaunchKernelGGL(k_jacobi_march<false>, dim3(col_blocks(C)), dim3(kJacobiThreads), 0, s, C, f, M, B, V, R, G,
                        with_quotients(J), nullptr, nullptr, nullptr);
 }
@@ -735,7 +735,7 @@ void ts_jacobi_res(const FShape &f, const Metrics &M, const Bulk &B, const doubl
 void ts_jacobi_vres(const FShape &f, const Metrics &M, const Bulk &B, const double *V, const double *R, double *G,
                     const JacobiCoef &J, JacobiSync *sync, unsigned long long *out, unsigned long long *host,
                     hipStream_t s) {
-    const ColGeo C = col_geo((long)(f.n[1] + 2) * (f.n[2] + 2), f.n[0] + 2, kJacobiThreads);
+    const ColGeo C = col_geo(f.n[1] + 2, f.n[2] + 2, f.n[0] + 2, kJacobiThreads);
     hipLaunchKernelGGL(k_jacobi_march<true>, dim3(col_blocks(C)), dim3(kJacobiThreads), 0, s, C, f, M, B, V, R, G,
                        with_quotients(J), sync, out, host);
 }

@@ -59,9 +59,12 @@ API Err __hipPopCallConfiguration(Dim *grid, Dim *block, size_t *lds, void **str
     *stream = cfg_stream;
     return kOk;
 }
-API Err hipLaunchKernel(const void *f, Dim grid, Dim block, void **, size_t, void *) {
-    launched() += names()[f] + " " + std::to_string((unsigned long)grid.x * grid.y * grid.z) + " " +
-                  std::to_string(block.x * block.y * block.z) + "\n";
+API Err hipLaunchKernel(const void *f, Dim grid, Dim block, void **args, size_t, void *) {
+    const std::string &name = names()[f];
+    launched() += name + " " + std::to_string(grid.x) + " " + std::to_string(block.x * block.y * block.z);
+    if (name.find("ColGeo") != std::string::npos)   // a march of columns.h: its first argument
+        for (int q = 0; q < 5; q++) launched() += " " + std::to_string(((const int *)args[0])[q]);
+    launched() += "\n";
     return kOk;
 }
 API Err hipFuncSetAttribute(const void *, int, int) { return refuse_lds ? kNoLds : kOk; }

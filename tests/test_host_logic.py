@@ -93,3 +93,35 @@ def test_without_large_lds_a_solver_runs_the_per_node_kernels(fake, precision):
         ran = {b for b in big for name in _launched(fake) if b in name}
         assert ran == (set() if refused else set(big)), (refused, ran)
         g.close()
+
+
+@pytest.mark.parametrize("ind", [(2, 2, 2), (2, 8, 8), (8, 2, 8), (8, 8, 2), (6, 6, 6), (7, 7, 7), (8, 8, 8), (9, 3, 9),
+                                 (9, 6, 8), (10, 5, 7), (12, 2, 2), (2, 2, 12), (3, 9, 9)], ids=str)
+def test_split_of_the_column_marches(fake, ind):
+    """Every plane in one chunk, no chunk longer than the metrics' LDS rows; chunks of one plane (half of a
+    pair of loads) only on a grid that they hardly fill the device with; a contiguous eighth of the
+    workgroups, an XCD's, holds at least 16 rows of every plane or an eighth of many planes."""
+    from saras_amd import field
+    fg = field.FieldGrid(field.fgrid_desc(ind=ind))
+    V, H, F, out = [fg.array(c) for c in (1, 2, 3)], [fg.array(c) for c in (1, 2, 3)], fg.array(0), fg.array(0)
+    fake.fake_clear()
+    fg.vfComputeDiff(V, H)
+    fg.vfComputeNLin(V, V, H)
+    fg.sfComputeNLin(V, F, out)
+    fg.divergence(V, out)
+    fg.calcDerivative2(0, 1, F, out)
+    rows, row = (1 << ind[1]) + 3, (1 << ind[2]) + 3
+    lines = _launched(fake)
+    assert len(lines) == 5
+    for line in lines:
+        grid, threads, nb, nch, cq, cr, by_chunk = (int(x) for x in line.split()[1:])
+        planes = nch * cq + cr
+        assert planes == (1 << ind[0]) + (3 if "diverg" in line or "deriv" in line else 1)
+        assert grid == nb * nch and nb * threads >= rows * row > (nb - 1) * threads
+        assert cr < nch and 1 <= cq + (cr > 0) <= 64
+        assert cq > 1 or cr >= nch - 1 or grid <= 1024, line
+        assert grid <= max(2304, nb * -(-planes // 64)), line
+        assert by_chunk == (rows < 16 * 8 + 2 and planes > rows), line
+    for a in V + H + [F, out]:
+        a.free()
+    fg.close()
