@@ -56,9 +56,8 @@ struct MarchGeo {
 
 struct MarchPlan {
     MarchGeo g;
-    int R;   // thread rows
     int blocks() const { return g.ntile * g.nch; }
-    int threads() const { return R * g.tpr; }
+    int threads() const { return g.R * g.tpr; }
 };
 
 // Tiles of up to 13 rows (15 thread rows with the halo rows: 15 % of colour 0 updated twice) and as
@@ -78,8 +77,8 @@ inline MarchPlan march_plan(const Lay &L, int planes = 1) {
     P.g.ntile = (L.ny + R - 3) / (R - 2);
     P.g.tq = L.ny / P.g.ntile;
     P.g.tr = L.ny % P.g.ntile;
-    P.g.R = P.R = P.g.tq + (P.g.tr > 0) + 2;
-    P.g.nch = (P.R * P.g.tpr > 512 ? 256 : 512) / P.g.ntile;
+    P.g.R = P.g.tq + (P.g.tr > 0) + 2;
+    P.g.nch = (P.threads() > 512 ? 256 : 512) / P.g.ntile;
     if (P.g.nch > L.nx / planes) P.g.nch = L.nx / planes;
     if (P.g.nch < 1) P.g.nch = 1;
     P.g.cq = L.nx / P.g.nch;

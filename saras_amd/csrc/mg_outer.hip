@@ -406,7 +406,7 @@ void launch_march_residual(const Lay &L, const double *x_in, const float *e, con
                            const double *cy, const double *cz, const Bc &bc, bool color0, const MarchSums &S, hipStream_t s) {
     const MarchPlan P = outer_plan(L);
     const int nc = color0 ? 1 : 2;
-    const size_t lds = 2 * (size_t)P.R * nc * L.khs * sizeof(double) + 4 * (size_t)P.g.tpr * sizeof(Co<double>);
+    const size_t lds = 2 * (size_t)P.g.R * nc * L.khs * sizeof(double) + 4 * (size_t)P.g.tpr * sizeof(Co<double>);
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(P.blocks()), dim3(threads64(P)), lds, s, L, P.g, x_in, e, z, coef, f, x_out, z_next,
                            r32, cx, cy, cz, bc, S.part, S.counter, S.fterms, S.out, S.host);
@@ -422,7 +422,7 @@ void launch_march_dots(const Lay &L, const float *e, const float *z, const float
                        const float *cz, const Bc &bc, bool q1r, double *part, unsigned *counter, double *coef,
                        hipStream_t s) {
     const MarchPlan P = outer_plan(L);
-    const size_t lds = 2 * (size_t)P.R * (q1r ? 3 : 4) * L.khs * sizeof(float) + 4 * (size_t)P.g.tpr * sizeof(Co<float>);
+    const size_t lds = 2 * (size_t)P.g.R * (q1r ? 3 : 4) * L.khs * sizeof(float) + 4 * (size_t)P.g.tpr * sizeof(Co<float>);
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(P.blocks()), dim3(threads64(P)), lds, s, L, P.g, e, z, r32, cx, cy, cz, bc, part,
                            counter, coef);

@@ -137,7 +137,6 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, MarchGeo G, const T *__
         Pair<T> &A2 = A[0], &A1 = A[1], &An = A[2];
         Co<T> &X1 = Xs[0], &X = Xs[1], &Xn = Xs[2];
         Pair<T> &f0 = F0[0], &f0n = F0[1], &f1 = F1[0], &f1n = F1[1];
-        constexpr int par = 0;
         const int bsz = R * khs;
         T *const lbc = lb + flip * bsz, *const lbn = lb + bsz - flip * bsz;
         T *const lac = la + flip * bsz, *const lap = la + bsz - flip * bsz;
@@ -152,8 +151,8 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, MarchGeo G, const T *__
                 Bc_ = ld2(ub + s * ps, here(vo1));
                 Bp = ld2(ub + sp * ps, here(vo1));
                 if (halo) {
-                    Ym[par] = ld2(ub + s * ps, here(vom));
-                    Yp[par] = ld2(ub + s * ps, here(vop));
+                    Ym[0] = ld2(ub + s * ps, here(vom));
+                    Yp[0] = ld2(ub + s * ps, here(vop));
                 }
                 if (antix && sm != s - 1) Bm = Pair<T>{-Bm.a, -Bm.b};
                 if (antix && sp != s + 1) Bp = Pair<T>{-Bp.a, -Bp.b};
@@ -179,8 +178,8 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, MarchGeo G, const T *__
             if (!ZERO) {
                 Bn = ld2(ub + src(0, min(p + 2, nx + 1), nx) * ps, here(vo1));
                 if (halo) {
-                    Ym[par ^ 1] = ld2(ub + s1 * ps, here(vom));
-                    Yp[par ^ 1] = ld2(ub + s1 * ps, here(vop));
+                    Ym[1] = ld2(ub + s1 * ps, here(vom));
+                    Yp[1] = ld2(ub + s1 * ps, here(vop));
                 }
             }
             f1n = ld2(f + s * ps, here(vo1));
@@ -193,8 +192,8 @@ __global__ void __launch_bounds__(1024) k_rb_pass(Lay L, MarchGeo G, const T *__
         } else {
             Pair<T> m_ = ld2(lbc, lom), p_ = ld2(lbc, lop);
             if (halo) {
-                m_ = Pair<T>{ysm * Ym[par].a, ysm * Ym[par].b};
-                p_ = Pair<T>{ysp * Yp[par].a, ysp * Yp[par].b};
+                m_ = Pair<T>{ysm * Ym[0].a, ysm * Ym[0].b};
+                p_ = Pair<T>{ysp * Yp[0].a, ysp * Yp[0].b};
             }
             An = update(X, Bc_, Bm, Bp, m_, p_, lbc, ys, f0, kb, Z0, Z1);
         }
@@ -246,7 +245,7 @@ void launch_rb_pass(const Lay &L, const T *ub, T *u, T *bo, const T *f, const T 
                     const Bc &bc, bool zero, bool last, hipStream_t s) {
     const MarchPlan P = march_plan(L);
     const dim3 grid(P.blocks()), blk(P.threads());
-    const size_t lds = 4 * (size_t)P.R * L.khs * sizeof(T) + 4 * (size_t)P.g.tpr * sizeof(Co<T>);
+    const size_t lds = 4 * (size_t)P.g.R * L.khs * sizeof(T) + 4 * (size_t)P.g.tpr * sizeof(Co<T>);
     auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, blk, lds, s, L, P.g, ub, u, bo, f, cx, cy, cz, bc); };
     const bool zper = bc.rule[2] == G_PERIODIC;
     if (zero && last) zper ? go(k_rb_pass<T, true, true, true>) : go(k_rb_pass<T, true, true, false>);
