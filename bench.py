@@ -34,6 +34,11 @@ sys.path.insert(0, ROOT)
 
 METRIC = "ms/Poisson solve to 1e-10 rel. residual, 257³ (learned+mixed vs FP64 MG)"
 HBM_PEAK_GBS = 8000.0
+# HBM bytes of what the roofline entries price, from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE (KiB per
+# dispatch) scaled by what the same counters read for a device copy of known size (FETCH_SIZE x 2.005,
+# WRITE_SIZE x 1.0); the summaries and commands are in profiles/
+TRAFFIC_BYTES = {"k_rb_pass<float> 257x257x257": 76.8e6, "k_rb_pass<double> 257x257x257": 175.3e6,
+                 "k_build_rhs 129x129x129": 149.6e6, "sr_vf_nlin (V advects V)": 1710.7e6}
 
 
 def half_sweep_bytes(solver, kernel):
@@ -217,7 +222,7 @@ def tgv_bench(args):
     # the step kernels one by one (HIP events on the handle's stream) against their algorithmic
     # bytes; timed after the stepped state was read, since they overwrite what they write
     kernels = {}
-    for kid, name in ((0, "k_build_rhs"), (1, "k_jacobi_march (Vx: sweep)"), (2, "k_jacobi_res (Vx)"),
+    for kid, name in ((0, "k_build_rhs"), (1, "k_jacobi_march (Vx: sweep)"),
                       (6, "k_jacobi_march (Vx: sweep + residual of its input)"), (3, "k_divergence"),
                       (4, "k_project x3"), (5, "k_energy")):
         kms = h.time_kernel(kid, reps=20)
@@ -271,7 +276,7 @@ def tgv_bench(args):
                    "step_kernels": kernels},
         "roofline": {"bound": "hbm", "kernel": "k_build_rhs (the largest non-multigrid kernel of the step)",
                      "achieved": kernels["k_build_rhs"]["GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": kernels["k_build_rhs"]["frac"], "traffic": None,
+                     "frac": kernels["k_build_rhs"]["frac"], "traffic": TRAFFIC_BYTES["k_build_rhs 129x129x129"],
                      "bytes_per_launch": kernels["k_build_rhs"]["bytes"],
                      "avg_launch_ms": kernels["k_build_rhs"]["ms"]},
         "cpu_baseline": cpu,
@@ -429,7 +434,7 @@ def rbc_bench(args):
         "roofline": {"bound": "hbm", "kernel": "k_rb_pass<float> finest level, per half sweep (FP32 V-cycle)",
                      "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
-                     "traffic": None,
+                     "traffic": TRAFFIC_BYTES.get(f"k_rb_pass<float> {n[0]}x{n[1]}x{n[2]}"),
                      "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5)},
         "cpu_baseline": cpu,
     }
@@ -516,7 +521,8 @@ def seq_bench(args):
                    "legs": res},
         "roofline": {"bound": "hbm", "kernel": "k_rb_pass<float> finest level, per half sweep (FP32 V-cycle)",
                      "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None, "traffic": None,
+                     "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
+                     "traffic": TRAFFIC_BYTES["k_rb_pass<float> 257x257x257"],
                      "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5)},
         "cpu_baseline": cpu,
     }
@@ -645,12 +651,12 @@ def fields_bench(args):
          "F read, out written over the padded array"),
         ("sr_vf_diff", lambda: fg.vfComputeDiff(V, H), sum(3 * w * core(c + 1) for c in range(3)),
          "per component: V_c and H_c read, H_c written"),
-        ("sr_vf_nlin (V advects V)", lambda: fg.vfComputeNLin(V, V, H), sum(5 * w * core(c + 1) for c in range(3)),
-         "per component: Vx, Vy, Vz and H_c read, H_c written"),
+        ("sr_vf_nlin (V advects V)", lambda: fg.vfComputeNLin(V, V, H), sum(3 * w * core(c + 1) for c in range(3)),
+         "V and H read, H written"),
         ("sr_divergence", lambda: fg.divergence(V, out), 4 * w * fsz(0),
          "three face arrays read, the node array written"),
-        ("sr_gradient", lambda: fg.gradient(P, G), sum(2 * w * core(c + 1) for c in range(3)),
-         "per component: P read, G_c written"),
+        ("sr_gradient", lambda: fg.gradient(P, G), w * core(0) + sum(w * core(c + 1) for c in range(3)),
+         "P read, G written"),
     ]
     timer = HipTimer(fg.stream())
     reps = max(args.steps, 5)
@@ -725,7 +731,7 @@ def fields_bench(args):
                    "jacobi_visc_Vx": {"call_ms": round(jac_ms, 3), "sweeps": int(sweeps),
                                       "note": "synchronous: the residual is read on the host after every sweep"}},
         "roofline": {"bound": "hbm", "kernel": dom_name, "achieved": dom["GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": dom["frac"], "traffic": None},
+                     "frac": dom["frac"], "traffic": TRAFFIC_BYTES.get(dom_name)},
         "cpu_baseline": cpu,
     }
     print(json.dumps(res))
@@ -876,7 +882,7 @@ def main():
         "roofline": {"bound": "hbm", "kernel": "k_rb_pass<double> finest level, per half sweep",
                      "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None,
-                     "traffic": None,
+                     "traffic": TRAFFIC_BYTES["k_rb_pass<double> 257x257x257"],
                      "bytes_per_launch": bytes_sweep, "avg_launch_ms_in_solve": round(sweep_ms, 5)},
         "cpu_baseline": cpu,
     }

@@ -32,7 +32,8 @@ extern "C" {
 /* which level array (lib/poisson/poisson.h:70-73) */
 #define SR_PRESSURE 0            /* pressureData */
 #define SR_RESIDUAL 1            /* residualData: the right-hand side of each level */
-#define SR_TMP      2            /* tmpDataArray: residual f - L u computed by computeResidual */
+#define SR_TMP      2            /* tmpDataArray: residual f - L u computed by computeResidual;
+                                    scratch of every other call (cycles and solves use it)        */
 
 #define SR_SEM_REFERENCE 0       /* padded-array mean removal, stop on |r_prev - r| < mgTolerance */
 #define SR_SEM_PROJECTED 1       /* RHS projected onto range(L), stop on relative residual       */
@@ -139,7 +140,10 @@ int sr_mg_op_vcycle(sr_mg *mg);                            /* poisson.cc:219-280
  * one kernel at one level: kernel 0 = red-black half sweep, 1 = residual, 2 = restriction,
  * 3 = prolongation-correction, 4 = ghost fill, 5 = level-0 residual norm, 6 = the FP32 half
  * sweep of the mixed-precision hierarchy, 7 / 8 = the single-workgroup coarse end of the FP64 /
- * FP32 cycle (level argument ignored).  Device state is modified (scratch use only).           */
+ * FP32 cycle (level argument ignored).  Device state is modified (scratch use only).
+ * 0, 5 and 6 are the per-node kernels, which cycles and solves run on levels with Dirichlet walls or
+ * with more than 513 nodes along z; elsewhere whole sweeps, norms and outer steps are one launch
+ * each and have no kernel id (sr_mg_stats.sweep0_ms times the sweeps within a solve).            */
 int sr_mg_time_kernel(sr_mg *mg, int kernel, int level, int reps, double *avg_ms);
 /* Algorithmic bytes one launch of that kernel moves (the roofline numerator).                   */
 int sr_mg_kernel_bytes(const sr_mg *mg, int kernel, int level, double *bytes);

@@ -129,9 +129,9 @@ int sr_ts_pressure_solver(sr_ts *ts, sr_mg **mg);
 /* Measurement (no reference counterpart): the algorithmic HBM bytes of one launch of a step kernel
    and its average duration over `reps` launches on the handle's fields (HIP events on the handle's
    stream; the kernels overwrite what they write, so a handle timed this way is for measurement).
-   kernel 0: the three nseRHS kernels (40 B per face node: V_c, the two other components, P read,
-   H_c written); 1: one Jacobi sweep of Vx (24 B per padded entry); 2: its residual maximum (16 B per
-   bulk node); 3: divergence (32 B per node); 4: the three projection updates (24 B per face node);
+   kernel 0: nseRHS of the three components in one launch (V and P read, H written); 1: one Jacobi
+   sweep of Vx (24 B per padded entry); 2: the residual maximum of an iterate by itself (16 B per
+   bulk node; no step runs it); 3: divergence (32 B per node); 4: the three projection updates (24 B per face node);
    5: the energy reduction (24 B per node); 6: one Jacobi sweep of Vx together with the residual
    maximum of its input, the form the step runs (24 B per padded entry). */
 int sr_ts_kernel_bytes(const sr_ts *ts, int kernel, double *bytes);

@@ -6,10 +6,10 @@
 // offsets, y and z metrics), the x neighbours of a value stay in registers, and every load is a plane's
 // address plus a 32-bit offset.  One thread per entry instead spent some 300 instructions per wavefront
 // on indices and metrics and was bound by them: 163 us for the second derivatives of a 257^3 field, which
-// move 0.41 GB.  Here it is 116 us, and every kernel takes about 20 us per 257^3 array of values that
-// miss the L1 cache, those of neighbouring rows among them, whichever workgroup size (256 or 1024), chunk
-// length or order: it is the way from the L2 cache that binds, not HBM (derivative along z, whose
-// neighbours are in the L1 cache: 56 us, 4.9 TB/s).
+// move 0.41 GB.  Here it is 116 us.  At 257^3 the L1 caches read 0.8 GB from the L2 caches for it and 2.6
+// GB for the advection of a velocity (351 us), 7 TB/s, neighbouring rows among them, about 20 us per
+// array; HBM carries 1.02 to 1.4 times what a kernel has to move, at 3.9-5.2 TB/s, where a large copy gets
+// 4.75.  Workgroup size (256 or 1024), chunk length and order change these by a few per cent.
 #pragma once
 
 #include "ts_kernels.h"

@@ -10,12 +10,14 @@
 // residual that a restriction reads is formed once per fine node, the dense coarsest operator is
 // applied by all threads, and all levels' coefficients come in one block.
 //
-// Per cycle at 257^3 (levels 17^3 to 3^3): 42 us in FP32 and 43 us in FP64, against 66 and 76 us with
+// Per cycle at 257^3 (levels 17^3 to 3^3): 47 us in FP32 and 50 us in FP64, against 66 and 76 us with
 // ghost layers whose images every update wrote, index arithmetic in every half sweep and a residual
-// evaluated once per tap; V(4,4) with the iterated coarsest level (Taylor-Green) 83 against 186 us, of
+// evaluated once per tap; V(4,4) with the iterated coarsest level (Taylor-Green) 79 against 186 us, of
 // which the 65 coarsest iterations take 19 (about 100 before).  The four half sweeps at 17^3 take 7 us,
-// 10 us as three nodes of each colour per thread with all indices kept, 8 us at the start of FP32 but 16
-// in FP64 with everything in registers (spills).
+// 10 us as three nodes of each colour per thread with all indices kept, 8 us in FP32 but 16 in FP64 with
+// everything in registers (spills).  A level of more than 1024 columns of three (33 x 17 x 9, the first of
+// the 129 x 65 x 33 grid in FP32: 1122) takes a second round in every half sweep, which sets its columns
+// up again: 58 us a cycle there.
 #include "mg_kernels.h"
 
 #include <type_traits>

@@ -9,9 +9,11 @@
 //
 // Per-node kernels of these steps (seven vector loads of neighbour values per quantity, ghosts filled, a
 // second launch for the sums and a copy for the host) took at 257^3: GCR step and residual 82 + 147 + 5,
-// products 87 + 8, norm of colour 0 58 + 5 us; these take 148, 74 and 68.  A GCR step has to move 0.81 GB
-// (x, f, e, z read, x, z, r written; 5.5 TB/s), so that it is bound by HBM; the products (0.2 GB of
-// which the halos make 0.24) and the norms by their instructions and the turn from plane to plane.
+// products 87 + 8, norm of colour 0 58 + 5 us; these take 137, 71 and 65.  A GCR step has to move 0.75 GB
+// (x, f, e, z read, x, z, r written) and is bound by HBM: 0.72 GB of it pass there, 5.3 TB/s.  The
+// products (0.20 GB, 0.22 with the halos, 3.1 TB/s) and the norm (0.20, 0.23, 3.5) reach neither that nor
+// the rate of their instructions, which take 32 and 18 % of the time to issue: one workgroup per CU waits
+// for its loads and at a barrier in every plane.
 //
 // Ghosts are neither read nor written: the neighbour beyond a periodic or mirror boundary is resolved
 // to the node it copies.  (Dirichlet walls keep the kernels of mg_kernels.hip.)

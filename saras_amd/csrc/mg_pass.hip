@@ -2,9 +2,10 @@
 //
 // Two half sweeps (k_rb_sweep) read the neighbour values of every node through seven vector loads and
 // are held by the address unit, not by HBM: 121 us (FP64) and 63 us (FP32) a sweep at 257^3, where a
-// sweep has to move 323 and 161 MB with its halos.  This kernel takes 55 and 40 us, 71 and 47 us as the
-// last sweep of a smoothing, which stores colour 0 too: 5.4-5.9 TB/s in FP64, about the rate of a large
-// copy; in FP32 it is bound by its instructions (190 vector instructions per four nodes).
+// sweep has to move 272 and 136 MB.  This kernel takes 55 and 40 us, 71 and 47 us as the last sweep of a
+// smoothing, which stores colour 0 too.  FP64: 312 and 389 MB pass HBM, 5.4-5.7 TB/s, above the rate of a
+// large copy.  FP32: 162 and 197 MB, 4.1 TB/s; its vector instructions (190 per four nodes) take 52-57 %
+// of the time to issue, the rest goes with one workgroup per CU that waits at every plane's barrier.
 //
 // A workgroup marches over the planes of a chunk of x with a tile of y rows and the whole of z.  Each
 // thread owns the two half-row entries 2t, 2t+1 of one row: its x neighbours stay in registers from
